@@ -1376,8 +1376,8 @@ int vx_mlp_param_count(void) { return kMlpParams; }
 int vx_mlp_forward(void* stream, const float* params, const float* x, uint32_t n, float* y) {
     if (!params || (n && (!x || !y))) return VX_E_INVALID_ARG;
     if (n == 0) return VX_OK;
-    unsigned grid = (unsigned)std::min<uint64_t>((n + kMlpWaves - 1) / kMlpWaves, 1024);
-    k_mlp_fwd<<<grid, 64 * kMlpWaves, 0, (hipStream_t)stream>>>(params, x, n, y, nullptr, nullptr);
+    unsigned grid = (unsigned)std::min<uint64_t>(((uint64_t)n + kMlpTile - 1) / kMlpTile, 1024);
+    k_mlp<false><<<grid, 256, 0, (hipStream_t)stream>>>(params, x, n, y, nullptr, nullptr, nullptr, nullptr);
     return hipGetLastError() == hipSuccess ? VX_OK : VX_E_HIP;
 }
 
@@ -1386,9 +1386,11 @@ int vx_mlp_gradient(void* stream, const float* params, const float* x, const flo
     if (!params || !grad || (n && (!x || !target || !y || !workspace))) return VX_E_INVALID_ARG;
     if (n == 0) return VX_E_INVALID_ARG;
     hipStream_t st = (hipStream_t)stream;
-    unsigned grid = (unsigned)std::min<uint64_t>((n + kMlpWaves - 1) / kMlpWaves, 1024);
-    k_mlp_fwd<<<grid, 64 * kMlpWaves, 0, st>>>(params, x, n, y, target, workspace);
-    k_mlp_grad<<<(kMlpParams + 255) / 256, 256, 0, st>>>(x, target, y, n, workspace, grad, loss);
+    // one block per 64 samples, 256 at most (one per CU): their partial gradients fit the
+    // n * 257 floats of the workspace (two blocks and more: n >= 65)
+    unsigned grid = (unsigned)std::min<uint64_t>(((uint64_t)n + kMlpTile - 1) / kMlpTile, 256);
+    k_mlp<true><<<grid, 256, 0, st>>>(params, x, n, y, target, workspace, grad, loss);
+    if (grid > 1) k_mlp_reduce<<<kMlpPart / 64, 256, 0, st>>>(workspace, grid, n, grad, loss);
     return hipGetLastError() == hipSuccess ? VX_OK : VX_E_HIP;
 }
 

@@ -5,12 +5,11 @@
 //   W1 [64][16] | b1 [64] | W2 [64][64] | b2 [64] | W3 [64] | b3
 // Loss: mean squared error over the batch, L = (1/n) sum_s (y_s - t_s)^2.
 //
-// One wavefront per sample: lane j owns hidden unit j of both layers.  Weights are
-// staged in LDS once per block, W1 and W2 transposed for the forward products (lane
-// j reads column j: consecutive lanes, consecutive banks) and W2 as stored for the
-// backward product dh1 = W2^T dh2 (lane k reads column k of W2).  Per-parameter
-// gradients are reduced over the batch by one lane per parameter in sample order, so
-// results do not depend on scheduling.
+// Forward, backward and the gradients are matrix products over the batch (K = 16, 64 or
+// the samples), so they run on the f32 matrix unit (v_mfma_f32_16x16x4_f32: f32 inputs and
+// accumulation) in one pass over the samples: nothing per sample goes to memory but y.
+// Partial gradients per block are added in block order, so results do not depend on
+// scheduling.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -21,122 +20,202 @@ constexpr int kIn = 16, kHid = 64;
 constexpr int kOffW1 = 0, kOffB1 = kOffW1 + kHid * kIn, kOffW2 = kOffB1 + kHid,
               kOffB2 = kOffW2 + kHid * kHid, kOffW3 = kOffB2 + kHid, kOffB3 = kOffW3 + kHid;
 constexpr int kMlpParams = kOffB3 + 1;  // 5313
-constexpr int kMlpWaves = 4;            // samples in flight per block
+constexpr int kMlpTile = 64;            // samples of one tile: 16 per wavefront
+constexpr int kMlpPart = 5376;          // floats of one block's partial gradients (loss at kMlpParams)
 
-__device__ inline float wave_sum_f(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
+typedef float MlpAcc __attribute__((ext_vector_type(4)));
 
-struct MlpLds {
-    float w1t[kIn][kHid];   // w1t[i][j] = W1[j][i]
-    float w2t[kHid][kHid];  // w2t[k][j] = W2[j][k]
-    float w2[kHid][kHid];   // as stored (backward)
-    float h1[kMlpWaves][kHid];
-    float dh2[kMlpWaves][kHid];
+// A 16 x 16 product over 4 k: lane l gives A[l % 16][l / 16] and B[l / 16][l % 16] and holds
+// rows 4 * (l / 16) + r, column l % 16 of the result.
+__device__ inline MlpAcc mlp_mma(float a, float b, MlpAcc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+struct MlpLds {  // odd row lengths: a column walk meets every bank
+    float x[kMlpTile][kIn + 1];
+    float w1[kHid][kIn + 1];
+    float w2[kHid][kHid + 1];
+    float h1[kMlpTile][kHid + 1];
+    float d1[kMlpTile][kHid + 1];
+    float d2[kMlpTile][kHid + 1];
+    float sum[4][4][kHid];  // per wavefront: b1, b2, W3; [3]: b3 and the loss
 };
 
-__device__ inline void mlp_stage(const float* P, MlpLds& S, bool backward) {
-    for (int e = threadIdx.x; e < kHid * kIn; e += blockDim.x) {
-        int j = e / kIn, i = e % kIn;
-        S.w1t[i][j] = P[kOffW1 + e];
-    }
-    for (int e = threadIdx.x; e < kHid * kHid; e += blockDim.x) {
-        int j = e / kHid, k = e % kHid;
-        float w = P[kOffW2 + e];
-        S.w2t[k][j] = w;
-        if (backward) S.w2[j][k] = w;
-    }
-    __syncthreads();
-}
-
-// Forward (and, with target, the per-sample backward terms) of one sample per wave.
-// ws (backward only): per sample h1[64], h2[64], dh1[64], dh2[64], then dy[n].
-__global__ __launch_bounds__(64 * kMlpWaves) void k_mlp_fwd(const float* P, const float* x, uint32_t n,
-                                                            float* y, const float* target, float* ws) {
+// Blocks take tiles of 64 samples: a1 = x W1^T + b1, a2 = relu(a1) W2^T + b2,
+// y = relu(a2) . W3 + b3.  BACK: also dL/da2, dL/da1 and the block's share of every
+// parameter's gradient, accumulated in registers over its tiles and written to
+// part[block][kMlpPart] (or, by a single block, to grad and loss).
+//
+// The tile is 64 samples because one tile's 14 k MFMA cycles per SIMD are about what its
+// loads and barriers take, and a batch of 8192 then gives 128 blocks.  The form it replaces
+// wrote 1 KB per sample to memory and reduced it with one lane per parameter, a chain of n
+// dependent loads: a training step of 8192 rows (gradient and Adam) took 2067 us and takes
+// 24 us now, which is the host's time to call it.
+template <bool BACK>
+__global__ __launch_bounds__(256) void k_mlp(const float* P, const float* x, uint32_t n, float* y,
+                                             const float* target, float* part, float* grad, float* loss) {
     __shared__ MlpLds S;
-    const bool backward = target != nullptr;
-    mlp_stage(P, S, backward);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const float b1 = P[kOffB1 + lane], b2 = P[kOffB2 + lane], w3 = P[kOffW3 + lane], b3 = P[kOffB3];
-    const uint32_t stride = gridDim.x * kMlpWaves;
-    for (uint32_t s0 = blockIdx.x * kMlpWaves; s0 < n; s0 += stride) {
-        // the block's waves take samples s0 .. s0+3; a wave past n idles (block-uniform loop)
-        uint32_t s = s0 + w;
-        bool ok = s < n;
-        float a1 = b1;
-        if (ok) {
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, q = lane >> 4;
+    for (int e = tid; e < kHid * kIn; e += 256) S.w1[e / kIn][e % kIn] = P[kOffW1 + e];
+    for (int e = tid; e < kHid * kHid; e += 256) S.w2[e / kHid][e % kHid] = P[kOffW2 + e];
+    float b1[4], b2[4], w3[4];
 #pragma unroll
-            for (int i = 0; i < kIn; i++) a1 = fmaf(S.w1t[i][lane], x[(size_t)s * kIn + i], a1);
+    for (int t = 0; t < 4; t++) {
+        b1[t] = P[kOffB1 + 16 * t + c];
+        b2[t] = P[kOffB2 + 16 * t + c];
+        w3[t] = P[kOffW3 + 16 * t + c];
+    }
+    const float b3 = P[kOffB3];
+    MlpAcc g1 = {0.f, 0.f, 0.f, 0.f}, g2[4];
+    float gb1[4], gb2[4], g3[4], gb3 = 0.f, gl = 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        g2[t] = MlpAcc{0.f, 0.f, 0.f, 0.f};
+        gb1[t] = gb2[t] = g3[t] = 0.f;
+    }
+    for (uint64_t s0 = (uint64_t)blockIdx.x * kMlpTile; s0 < n; s0 += (uint64_t)gridDim.x * kMlpTile) {
+        __syncthreads();  // the previous tile's rows were read
+        for (int e = tid; e < kMlpTile * kIn; e += 256) {
+            const uint64_t s = s0 + e / kIn;
+            S.x[e / kIn][e % kIn] = s < n ? x[s * kIn + e % kIn] : 0.f;
         }
-        float h1 = a1 > 0.f ? a1 : 0.f;
-        S.h1[w][lane] = h1;
         __syncthreads();
-        float a2 = b2;
-#pragma unroll 8
-        for (int k = 0; k < kHid; k++) a2 = fmaf(S.w2t[k][lane], S.h1[w][k], a2);
-        float h2 = a2 > 0.f ? a2 : 0.f;
-        float out = wave_sum_f(w3 * h2) + b3;
-        if (ok && lane == 0 && y) y[s] = out;
-        if (backward) {
-            float dy = ok ? 2.f * (out - target[s]) / (float)n : 0.f;
-            float dh2 = a2 > 0.f ? dy * w3 : 0.f;
-            S.dh2[w][lane] = dh2;
-            __syncthreads();
-            float g = 0.f;
-#pragma unroll 8
-            for (int j = 0; j < kHid; j++) g = fmaf(S.w2[j][lane], S.dh2[w][j], g);
-            float dh1 = a1 > 0.f ? g : 0.f;
-            if (ok) {
-                float* r = ws + (size_t)s * 4 * kHid;
-                r[lane] = h1;
-                r[kHid + lane] = h2;
-                r[2 * kHid + lane] = dh1;
-                r[3 * kHid + lane] = dh2;
-                if (lane == 0) ws[(size_t)n * 4 * kHid + s] = dy;
+        const int r0 = 16 * w;  // this wavefront's samples of the tile
+        bool ok[4];             // row 4q + r of them
+#pragma unroll
+        for (int r = 0; r < 4; r++) ok[r] = s0 + r0 + 4 * q + r < n;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            MlpAcc a = {b1[t], b1[t], b1[t], b1[t]};
+#pragma unroll
+            for (int k = 0; k < kIn; k += 4) a = mlp_mma(S.x[r0 + c][k + q], S.w1[16 * t + c][k + q], a);
+#pragma unroll
+            for (int r = 0; r < 4; r++) S.h1[r0 + 4 * q + r][16 * t + c] = ok[r] && a[r] > 0.f ? a[r] : 0.f;
+        }
+        __syncthreads();
+        MlpAcc a2[4];
+        MlpAcc out = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            a2[t] = MlpAcc{b2[t], b2[t], b2[t], b2[t]};
+#pragma unroll
+            for (int k = 0; k < kHid; k += 4) a2[t] = mlp_mma(S.h1[r0 + c][k + q], S.w2[16 * t + c][k + q], a2[t]);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                a2[t][r] = a2[t][r] > 0.f ? a2[t][r] : 0.f;
+                out[r] = fmaf(w3[t], a2[t][r], out[r]);
             }
         }
-        __syncthreads();  // S.h1 / S.dh2 are rewritten by the next sample
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) out[r] += __shfl_xor(out[r], o);
+            out[r] += b3;
+            if (ok[r] && c == 0 && y) y[s0 + r0 + 4 * q + r] = out[r];
+        }
+        if constexpr (BACK) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float e = ok[r] ? out[r] - target[s0 + r0 + 4 * q + r] : 0.f;
+                const float dy = 2.f * e / (float)n;
+                if (c == 0) {
+                    gb3 += dy;
+                    gl = fmaf(e, e, gl);
+                }
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    const float d = ok[r] && a2[t][r] > 0.f ? dy * w3[t] : 0.f;
+                    S.d2[r0 + 4 * q + r][16 * t + c] = d;
+                    gb2[t] += d;
+                    if (ok[r]) g3[t] = fmaf(dy, a2[t][r], g3[t]);
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                MlpAcc a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int k = 0; k < kHid; k += 4) a = mlp_mma(S.d2[r0 + c][k + q], S.w2[k + q][16 * t + c], a);
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float d = S.h1[r0 + 4 * q + r][16 * t + c] > 0.f ? a[r] : 0.f;
+                    S.d1[r0 + 4 * q + r][16 * t + c] = d;
+                    gb1[t] += d;
+                }
+            }
+            __syncthreads();
+            // the tile's products over its samples: rows j = 16 w + ..
+#pragma unroll
+            for (int k = 0; k < kMlpTile; k += 4) {
+                const float dj = S.d2[k + q][r0 + c];
+#pragma unroll
+                for (int t = 0; t < 4; t++) g2[t] = mlp_mma(dj, S.h1[k + q][16 * t + c], g2[t]);
+                g1 = mlp_mma(S.d1[k + q][r0 + c], S.x[k + q][c], g1);
+            }
+        }
+    }
+    if constexpr (BACK) {
+        const bool one = gridDim.x == 1;
+        float* G = one ? grad : part + (size_t)blockIdx.x * kMlpPart;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+#pragma unroll
+            for (int o = 16; o < 64; o <<= 1) {
+                gb1[t] += __shfl_xor(gb1[t], o);
+                gb2[t] += __shfl_xor(gb2[t], o);
+                g3[t] += __shfl_xor(g3[t], o);
+            }
+            if (q == 0) {
+                S.sum[w][0][16 * t + c] = gb1[t];
+                S.sum[w][1][16 * t + c] = gb2[t];
+                S.sum[w][2][16 * t + c] = g3[t];
+            }
+        }
+#pragma unroll
+        for (int o = 16; o < 64; o <<= 1) {
+            gb3 += __shfl_xor(gb3, o);
+            gl += __shfl_xor(gl, o);
+        }
+        if (lane == 0) {
+            S.sum[w][3][0] = gb3;
+            S.sum[w][3][1] = gl;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int j = 16 * w + 4 * q + r;
+#pragma unroll
+            for (int t = 0; t < 4; t++) G[kOffW2 + j * kHid + 16 * t + c] = g2[t][r];
+            G[kOffW1 + j * kIn + c] = g1[r];
+        }
+        __syncthreads();
+        if (tid < 3 * kHid) {
+            const int v = tid / kHid, j = tid % kHid;
+            const float t = (S.sum[0][v][j] + S.sum[1][v][j]) + (S.sum[2][v][j] + S.sum[3][v][j]);
+            G[(v == 0 ? kOffB1 : v == 1 ? kOffB2 : kOffW3) + j] = t;
+        } else if (tid < 3 * kHid + 2) {
+            const int v = tid - 3 * kHid;
+            const float t = (S.sum[0][3][v] + S.sum[1][3][v]) + (S.sum[2][3][v] + S.sum[3][3][v]);
+            if (v == 0) G[kOffB3] = t;
+            else if (!one) G[kMlpParams] = t;
+            else if (loss) *loss = t / (float)n;
+        }
     }
 }
 
-// dL/dparam for every parameter, reduced over the batch in sample order; the lane
-// of b3 also writes the loss.
-__global__ void k_mlp_grad(const float* x, const float* target, const float* y, uint32_t n, const float* ws,
-                           float* grad, float* loss) {
-    uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= (uint32_t)kMlpParams) return;
-    const float* dy = ws + (size_t)n * 4 * kHid;
-    float g = 0.f;
-    if (p < (uint32_t)kOffB1) {
-        int j = p / kIn, i = p % kIn;
-        for (uint32_t s = 0; s < n; s++) g = fmaf(ws[(size_t)s * 4 * kHid + 2 * kHid + j], x[(size_t)s * kIn + i], g);
-    } else if (p < (uint32_t)kOffW2) {
-        int j = p - kOffB1;
-        for (uint32_t s = 0; s < n; s++) g += ws[(size_t)s * 4 * kHid + 2 * kHid + j];
-    } else if (p < (uint32_t)kOffB2) {
-        int e = p - kOffW2, j = e / kHid, k = e % kHid;
-        for (uint32_t s = 0; s < n; s++) {
-            const float* r = ws + (size_t)s * 4 * kHid;
-            g = fmaf(r[3 * kHid + j], r[k], g);
-        }
-    } else if (p < (uint32_t)kOffW3) {
-        int j = p - kOffB2;
-        for (uint32_t s = 0; s < n; s++) g += ws[(size_t)s * 4 * kHid + 3 * kHid + j];
-    } else if (p < (uint32_t)kOffB3) {
-        int j = p - kOffW3;
-        for (uint32_t s = 0; s < n; s++) g = fmaf(dy[s], ws[(size_t)s * 4 * kHid + kHid + j], g);
-    } else {
-        float l = 0.f;
-        for (uint32_t s = 0; s < n; s++) {
-            g += dy[s];
-            float e = y[s] - target[s];
-            l = fmaf(e, e, l);
-        }
-        if (loss) *loss = l / (float)n;
+// The blocks' partial gradients added in a fixed order: 64 parameters per block, four
+// lanes each (block b of the first pass goes to lane b % 4).
+__global__ __launch_bounds__(256) void k_mlp_reduce(const float* part, uint32_t blocks, uint32_t n, float* grad,
+                                                    float* loss) {
+    __shared__ float s[4][64];
+    const uint32_t i = threadIdx.x & 63u, g = threadIdx.x >> 6, p = blockIdx.x * 64 + i;
+    float v = 0.f;
+#pragma unroll 8
+    for (uint32_t b = g; b < blocks; b += 4) v += part[(size_t)b * kMlpPart + p];
+    s[g][i] = v;
+    __syncthreads();
+    if (g == 0 && p <= (uint32_t)kMlpParams) {
+        v = (s[0][i] + s[1][i]) + (s[2][i] + s[3][i]);
+        if (p < (uint32_t)kMlpParams) grad[p] = v;
+        else if (loss) *loss = v / (float)n;
     }
-    grad[p] = g;
 }
 
 // Adam (Kingma & Ba, 2015) with bias correction; step counts from 1.
