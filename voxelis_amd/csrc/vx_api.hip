@@ -872,9 +872,19 @@ template <typename T>
 int to_vec_impl(vx_interner* h, size_t n, const uint64_t* roots, const uint8_t* depths, uint32_t lod,
                 uint64_t stride, void* out) {
     Pool<T> P = pool_of<T>(h);
-    uint64_t total = (uint64_t)n * stride;
-    VX_LAUNCH(h, KID_TO_VEC, k_to_vec<T>, grid_for(total), kBlock, P, (uint64_t)n, roots, depths, lod, stride,
-              (T*)out);
+    // a lane per voxel for trees of at most 4^3 voxels, and for extractions that give every
+    // CU's lanes at most a few voxels each: their time is one walk's, and the cells' kernel
+    // has two more loads in a row (one tree of 32^3: 1.5 us longer)
+    if (stride <= 64 || (uint64_t)n * stride <= (1u << 19)) {
+        VX_LAUNCH(h, KID_TO_VEC, k_to_vec_small<T>, grid_for((uint64_t)n * stride), kBlock, P, (uint64_t)n, roots, depths,
+                  lod, stride, (T*)out);
+    } else {
+        // cells of 8^3 voxels; no tree has more than 16^3 of them, whatever the stride
+        const uint64_t cells = std::min<uint64_t>((stride + 511) / 512, 4096);
+        const uint64_t blocks = ((uint64_t)n * cells + kDenseCells - 1) / kDenseCells;
+        VX_LAUNCH(h, KID_TO_VEC, k_to_vec<T>, (unsigned)std::min<uint64_t>(blocks, 1u << 20), 256, P, (uint64_t)n, roots,
+                  depths, lod, stride, cells, (T*)out);
+    }
     return hipGetLastError() == hipSuccess ? VX_OK : VX_E_HIP;
 }
 

@@ -2973,49 +2973,188 @@ __device__ inline uint64_t canon_combine(uint64_t h, uint64_t child, uint32_t i)
     return mix64(h ^ (child + 0x9E3779B97F4A7C15ull * (uint64_t)(i + 1)));
 }
 
-// Merkle hash of a tree, seeds S0/S1; one lane per tree, iterative DFS.
 // to_vec (utils/common.rs:158-246) at a reduced depth (MaxDepth::for_lod,
-// core/max_depth.rs:137-140): one lane per output voxel, output in y, z, x order.
-// A branch reached at the reduced depth gives its LOD value; an empty child gives
-// the default value; a leaf covers its whole cube.
+// core/max_depth.rs:137-140), output in y, z, x order.  A branch reached at the reduced
+// depth gives its LOD value; an empty child gives the default value; a leaf covers its
+// whole cube.
+//
+// One step of the walk: the child of `node` at digit ci (a leaf or empty node stays).
 template <typename T>
-__global__ void k_to_vec(Pool<T> P, uint64_t n, const uint64_t* roots, const uint8_t* depths, uint32_t lod,
-                         uint64_t stride, T* out) {
+__device__ inline uint64_t dense_step(const Pool<T>& P, uint64_t node, uint32_t ci) {
+    if (node == kEmpty || bid_is_leaf(node)) return node;
+    if (bid_index(node) >= P.capacity) {
+        atomicOr(&P.ctl->err, kErrPoison);
+        return kEmpty;
+    }
+    return P.children[8ull * bid_index(node) + ci];
+}
+
+template <typename T>
+__device__ inline T dense_value(const Pool<T>& P, uint64_t node) {
+    return node != kEmpty && bid_index(node) < P.capacity ? P.values[bid_index(node)] : (T)0;
+}
+
+// The reduced depth of tree t, or ~0 when it is skipped (VX_E_RANGE at the next sync).
+template <typename T>
+__device__ inline uint32_t dense_depth(const Pool<T>& P, uint32_t D, uint32_t lod, uint64_t stride) {
+    const uint32_t Dl = D > lod ? D - lod : 0u;
+    if (D > (uint32_t)kMaxDepth || (1ull << (3 * Dl)) > stride) {
+        atomicOr(&P.ctl->err, kErrRange);
+        return ~0u;
+    }
+    return Dl;
+}
+
+// Small extractions (to_vec_impl's rule): one lane per voxel.
+template <typename T>
+__global__ void k_to_vec_small(Pool<T> P, uint64_t n, const uint64_t* roots, const uint8_t* depths, uint32_t lod,
+                               uint64_t stride, T* out) {
     const uint64_t total = n * stride;
     VX_LOOP(i, total) {
         if (i < total) {
-            uint64_t t = i / stride, v = i - t * stride;
-            uint32_t D = depths[t];
-            if (D > (uint32_t)kMaxDepth) {
-                atomicOr(&P.ctl->err, kErrRange);
-                continue;
-            }
-            uint32_t Dl = D > lod ? D - lod : 0u;
-            uint64_t N = 1ull << Dl;
-            if (N * N * N > stride) {
-                if (v == 0) atomicOr(&P.ctl->err, kErrRange);
-                continue;
-            }
-            if (v >= N * N * N) continue;
-            uint32_t x = (uint32_t)(v % N), z = (uint32_t)((v / N) % N), y = (uint32_t)(v / (N * N));
+            const uint64_t t = i / stride;
+            const uint32_t v = (uint32_t)(i - t * stride);
+            const uint32_t Dl = dense_depth(P, depths[t], lod, stride);
+            if (Dl == ~0u || v >= 1u << (3 * Dl)) continue;
+            const uint32_t m = (1u << Dl) - 1, x = v & m, z = (v >> Dl) & m, y = v >> (2 * Dl);
             uint64_t node = roots[t];
-            for (uint32_t d = 0; d < Dl && node != kEmpty && !bid_is_leaf(node); d++) {
-                if (bid_index(node) >= P.capacity) {
-                    atomicOr(&P.ctl->err, kErrPoison);
-                    node = kEmpty;
-                    break;
-                }
-                uint32_t s = Dl - 1 - d;
-                uint32_t ci = ((x >> s) & 1u) | (((y >> s) & 1u) << 1) | (((z >> s) & 1u) << 2);
-                node = P.children[8ull * bid_index(node) + ci];
+            for (uint32_t d = 0; d < Dl; d++) {
+                const uint32_t s = Dl - 1 - d;
+                node = dense_step(P, node, ((x >> s) & 1u) | (((y >> s) & 1u) << 1) | (((z >> s) & 1u) << 2));
             }
-            T val = 0;
-            if (node != kEmpty && bid_index(node) < P.capacity) val = P.values[bid_index(node)];
-            out[i] = val;
+            out[i] = dense_value(P, node);
         }
     }
 }
 
+// Larger trees, by cells of 8^3 output voxels.  A block takes 8 consecutive cells of one
+// tree in x, z, y order (of several trees when they have fewer), two per wavefront: the
+// walk from the root to the cells' nodes is made once for all eight, then one lane per
+// brick takes the two levels below, the brick's 64-byte row of children and its eight
+// values, so a voxel costs an eighth of a walk's last loads and nothing of its first.  The
+// rows are loaded by four lanes each, one after the other in memory: a wavefront's load
+// costs an L1 look-up per line it meets, and these look-ups (eight values of every brick,
+// each at a place of its own) are what bounds the kernel.  The cells meet in LDS and leave
+// as 8-voxel rows, eight rows of one x line side by side.
+// 300 u16 trees of 64^3 (157 MB): 309 us with a lane per voxel walking from the root, 86 us
+// so (1.8 TB/s); 95 us when each lane loads its own brick's row, 104 us with one cell per
+// wavefront, 124 us with the next cells' walk overlapped (fewer wavefronts fit).
+constexpr uint32_t kDenseCells = 8;
+
+struct DenseCell {  // lane l's cell, l % 8
+    uint64_t t, node;
+    uint32_t x, z, y;
+    uint32_t Dl;  // the tree's reduced depth; ~0: no cell
+    uint32_t up;  // levels above the cell
+};
+
+template <typename T>
+__device__ inline DenseCell dense_cell(const Pool<T>& P, uint64_t u, uint64_t total, uint64_t cells,
+                                       const uint64_t* roots, const uint8_t* depths, uint32_t lod, uint64_t stride) {
+    DenseCell C;
+    const bool live = u < total;
+    if (!live) u = 0;
+    C.t = total >> 32 ? u / cells : (uint32_t)u / (uint32_t)cells;
+    const uint32_t c = (uint32_t)(u - C.t * cells);
+    const uint32_t D = depths[C.t];
+    C.node = roots[C.t];
+    C.Dl = live ? dense_depth(P, D, lod, stride) : ~0u;
+    C.up = C.Dl != ~0u && C.Dl > 3 ? C.Dl - 3 : 0u;
+    if (c >= 1u << (3 * C.up)) C.Dl = ~0u;  // a place past the tree's cells
+    const uint32_t m = (1u << C.up) - 1;
+    C.x = c & m;
+    C.z = (c >> C.up) & m;
+    C.y = (c >> (2 * C.up)) & m;
+    return C;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_to_vec(Pool<T> P, uint64_t n, const uint64_t* roots, const uint8_t* depths,
+                                                uint32_t lod, uint64_t stride, uint64_t cells, T* out) {
+    struct __align__(2 * sizeof(T)) Pair {
+        T a, b;
+    };
+    struct __align__(sizeof(T) * 8 < 16 ? sizeof(T) * 8 : 16) Row {
+        T v[8];
+    };
+    __shared__ Row s_v[kDenseCells][64];  // [cell][y * 8 + z]
+    const uint32_t lane = __lane_id(), w = threadIdx.x >> 6;
+    const uint64_t total = n * cells;
+    for (uint64_t u0 = (uint64_t)blockIdx.x * kDenseCells; u0 < total; u0 += (uint64_t)gridDim.x * kDenseCells) {
+        // every wavefront: lane l walks to cell l % 8
+        DenseCell C = dense_cell(P, u0 + (lane & 7u), total, cells, roots, depths, lod, stride);
+        for (uint32_t d = 0; d < C.up; d++) {
+            const uint32_t s = C.up - 1 - d;
+            C.node = dense_step(P, C.node, ((C.x >> s) & 1u) | (((C.y >> s) & 1u) << 1) | (((C.z >> s) & 1u) << 2));
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const uint32_t cell = w + 4u * k;
+            const uint32_t cD = __shfl(C.Dl, cell);
+            const uint64_t cn = shfl64(C.node, cell);
+            if (cD == ~0u) continue;  // uniform over the wavefront
+            if (cD < 3) {             // a tree of a few voxels: one lane each
+                const uint64_t ct = shfl64(C.t, cell);
+                if (lane < 1u << (3 * cD)) {
+                    const uint32_t m = (1u << cD) - 1, x = lane & m, z = (lane >> cD) & m, y = lane >> (2 * cD);
+                    uint64_t q = cn;
+                    for (uint32_t d = 0; d < cD; d++) {
+                        const uint32_t s = cD - 1 - d;
+                        q = dense_step(P, q, ((x >> s) & 1u) | (((y >> s) & 1u) << 1) | (((z >> s) & 1u) << 2));
+                    }
+                    out[ct * stride + lane] = dense_value(P, q);
+                }
+                continue;
+            }
+            // lane l: the node of the brick with digits l >> 3 and l & 7 (x | y << 1 | z << 2)
+            uint64_t nd = dense_step(P, dense_step(P, cn, lane >> 3), lane & 7u);
+            if (nd != kEmpty && bid_index(nd) >= P.capacity) nd = kEmpty;
+            // its eight values, two per lane of four: bricks 16 j + lane / 4 in round j
+            ulonglong2 ch[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint64_t q = shfl64(nd, 16 * j + (lane >> 2));
+                ch[j] = ulonglong2{q, q};
+                if (q != kEmpty && !bid_is_leaf(q)) ch[j] = ((const ulonglong2*)(P.children + 8ull * bid_index(q)))[lane & 3u];
+            }
+            T v[8];  // (index 0, the empty branch, holds the default value)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                v[2 * j] = P.values[bid_index(ch[j].x) < P.capacity ? bid_index(ch[j].x) : 0u];
+                v[2 * j + 1] = P.values[bid_index(ch[j].y) < P.capacity ? bid_index(ch[j].y) : 0u];
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t b = 16 * j + (lane >> 2), h = b >> 3, l = b & 7u;
+                const uint32_t x = ((h & 1u) << 2) | ((l & 1u) << 1), y = ((h & 2u) << 1) | (l & 2u) | (lane & 1u),
+                               z = (h & 4u) | ((l & 4u) >> 1) | ((lane >> 1) & 1u);
+                *(Pair*)&s_v[cell][y * 8 + z].v[x] = Pair{v[2 * j], v[2 * j + 1]};
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const uint32_t e = threadIdx.x + 256u * k;
+            // one x line's rows of the eight cells side by side, or each cell's rows
+            const uint32_t cell = cells >= kDenseCells ? e & 7u : e >> 6, r = cells >= kDenseCells ? e >> 3 : e & 63u;
+            const uint32_t rD = __shfl(C.Dl, cell);
+            const uint64_t rt = shfl64(C.t, cell);
+            const uint32_t rx = __shfl(C.x, cell), rz = __shfl(C.z, cell), ry = __shfl(C.y, cell);
+            if (rD == ~0u || rD < 3) continue;
+            T* dst = out + rt * stride + (((((uint64_t)ry * 8 + (r >> 3)) << rD) + rz * 8 + (r & 7u)) << rD) + rx * 8;
+            const Row q = s_v[cell][r];
+            if (((uintptr_t)dst & (alignof(Row) - 1)) == 0) {
+                *(Row*)dst = q;
+            } else {  // the caller's buffer or stride is not aligned to whole rows
+#pragma unroll
+                for (int i = 0; i < 8; i++) dst[i] = q.v[i];
+            }
+        }
+        __syncthreads();  // the rows are read before the next cells overwrite them
+    }
+}
+
+// Merkle hash of a tree, seeds S0/S1; one lane per tree, iterative DFS.
 template <typename T>
 __global__ void k_canon(Pool<T> P, uint32_t n, const uint64_t* roots, uint64_t* out) {
     const uint64_t S0 = 0x736F6D6570736575ull, S1 = 0x646F72616E646F6Dull;
