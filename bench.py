@@ -36,7 +36,7 @@ UNEVEN_WORKLOAD = ("uneven batched edits: 4096 u16 trees, MaxDepth uniform over 
                    "per tree, all trees in one launch sequence, values alternating v and v+1 per step")
 TERRAIN_WORKLOAD = ("perlin-dune terrain, 64x64 trees of 32^3 (MaxDepth 5), u8, one batch per tree, all "
                     "trees in one launch sequence, ids alternating 1/2 and 2/1 per step")
-HC_KERNELS = ("k_brick_build", "k_brick_retry", "k_probe[bricks]", "k_level_build", "k_probe[upper]", "k_commit")
+HC_KERNELS = ("k_brick_build", "k_probe[bricks]", "k_level_build", "k_probe[upper]", "k_commit")
 # rocprofv3 kernel symbol -> the library's kernel name
 TRACE_NAMES = {"k_probe_bricks": "k_probe[bricks]", "k_probe": "k_probe[upper]"}
 

@@ -39,7 +39,7 @@ constexpr uint64_t kMaxGrid = 8192;
 // block; at least `blocks` blocks stay so the launch still spreads over the chip.
 inline uint32_t probe_group(uint32_t ntiles, uint32_t blocks) {
     if (blocks == 0) return 1;
-    return std::max<uint32_t>(1u, std::min<uint32_t>(16u, ntiles / blocks));
+    return std::max<uint32_t>(1u, std::min<uint32_t>(kProbeTiles, ntiles / blocks));
 }
 
 inline unsigned grid_for(uint64_t work) {
@@ -92,14 +92,14 @@ struct LevelBufs {
 
 // Kernel ids of the per-kernel timer (vx_interner_profile_*).
 enum KernelId : uint32_t {
-    KID_BEGIN = 0, KID_PREPARE, KID_BRICK_SCAN, KID_LEAF_ALLOC, KID_BRICK_BUILD, KID_PROBE_BRICKS,
+    KID_BEGIN = 0, KID_PREPARE, KID_UNUSED0, KID_DRY_LEAVES, KID_BRICK_BUILD, KID_PROBE_BRICKS,
     KID_UNUSED, KID_LEVEL_BUILD, KID_PROBE_UPPER, KID_COMMIT, KID_FINALIZE,
     KID_END_ALLOC, KID_LEAF_CLEANUP, KID_GC, KID_GET, KID_CANON, KID_FILL, KID_ROLLBACK, KID_TO_VEC,
     KID_SET_DESCEND, KID_SET_LEVEL, KID_GET_GROUPED, KID_EDIT_KEYS, KID_SORT_HIST, KID_SORT_SCAN,
     KID_SORT_SCATTER, KID_EDIT_SCATTER, KID_COUNT
 };
 const char* const kKernelNames[KID_COUNT] = {
-    "k_begin", "k_prepare", "k_brick_retry", "k_leaf_alloc", "k_brick_build", "k_probe[bricks]",
+    "k_begin", "k_prepare", "", "k_dry_leaves", "k_brick_build", "k_probe[bricks]",
     "", "k_level_build", "k_probe[upper]", "k_commit", "k_finish",
     "k_end_alloc", "k_leaf_cleanup", "k_gc_round", "k_get", "k_canon", "k_fill", "k_rollback", "k_to_vec",
     "k_set_descend", "k_set_level", "k_get_grouped", "k_edit_keys", "k_sort_hist", "k_sort_scan",
@@ -144,8 +144,8 @@ struct vx_interner {
     uint32_t* free_stack = nullptr;
     uint64_t* tab = nullptr;
     uint64_t* single = nullptr;  // u8/u16: the one-leaf key index (8 slots x every value)
-    uint32_t* leaf_map = nullptr;
-    uint64_t* leaf_ids = nullptr;  // u16: the brick pass's leaf id of every value
+    uint64_t* leaf_ids = nullptr;    // u8/u16: the leaf id of every value
+    uint32_t* leaf_claim = nullptr;  // ... and the epoch of its last creation
     uint64_t* ltab = nullptr;      // four-byte voxels: the hashed leaf table
     uint64_t lslots = 0;
     uint32_t* need_list = nullptr;
@@ -156,7 +156,7 @@ struct vx_interner {
     bool own_stream = false;
     int poisoned = 0;
     // workspace
-    Grow chunks, slot_off, ptr_tables, gc_front[2], stage, scratch, deferred, drift, undo, owners;
+    Grow chunks, slot_off, ptr_tables, gc_front[2], stage, scratch, drift, undo, owners;
     Grow set_rec, set_meta;  // single-voxel set: the recorded path of every tree
     // edit-list path: zero-kept dense Batch buffers, sort buffers, tree records
     Grow edit_ws, edit_keys[2], edit_order[2], edit_tmp, edit_trees, edit_first, edit_status;
@@ -193,8 +193,8 @@ Pool<T> pool_of(vx_interner* h) {
     P.tab = h->tab;
     P.single = h->single;
     P.tmask = h->tslots - 1;
-    P.leaf_map = h->leaf_map;
     P.leaf_ids = h->leaf_ids;
+    P.leaf_claim = h->leaf_claim;
     P.ltab = h->ltab;
     P.lmask = h->lslots ? h->lslots - 1 : 0;
     P.need_list = h->need_list;
@@ -463,7 +463,7 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
         }
         uint64_t ns = ntiles[hh] * TILE;
         // slot and candidate indices travel as 32-bit values (pending results, the
-        // owner list, deferred bricks)
+        // owner list)
         if (ns > 0xFFFFFFFFull) return VX_E_INVALID_ARG;
         LevelBufs& B = h->lv[hh];
         if (!B.res.ensure(ns * 8) || !B.key.ensure(ns * 72) || !B.hash.ensure(ns * 8) ||
@@ -503,12 +503,10 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     HIPCHK(hipMemcpyAsync(g_tables.ptr, hptrs, tab_bytes, hipMemcpyHostToDevice, s));
     P.levels = (const Cands*)((void**)g_tables.ptr + 2 * (kLevels + 1));
     pinned_release(h);
-    uint32_t nvalues = sizeof(T) <= 2 ? 1u << (8 * sizeof(T)) : 0u;  // four-byte voxels: the request list
     uint64_t nb = std::max<uint64_t>(dmax >= 2 ? L[1].nslots : 1, 1);
-    if (!h->deferred.ensure(nb * 8) || !h->drift.ensure(nb * sizeof(Drift))) return VX_E_HIP;
-    uint64_t* ddef = (uint64_t*)h->deferred.ptr;
+    if (!h->drift.ensure(nb * sizeof(Drift))) return VX_E_HIP;
     Drift* ddrift = (Drift*)h->drift.ptr;
-    // undo log: one entry per deferred brick, collapsed upper node or fill leaf at most
+    // undo log: one entry per collapsed upper node or fill leaf at most
     uint64_t undo_cap = n;
     LevelTiles LT;
     std::memset(&LT, 0, sizeof(LT));
@@ -542,7 +540,6 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     const T* sv = (const T*)opt.set_values;
     VX_LAUNCH(h, KID_SET_DESCEND, k_set_descend<T>, grid_for(n), kBlock, P, dchunks, (uint32_t)n, roots, sx, sv,
               drec, dmeta);
-    VX_LAUNCH(h, KID_LEAF_ALLOC, k_leaf_alloc<T>, 1, 1024, P, dchunks, (uint32_t)n, nvalues);
     const unsigned wpb = TILE / 64;
     for (uint32_t hh = 1; hh <= dmax; hh++) {
         unsigned th = (unsigned)ntiles[hh];
@@ -555,7 +552,7 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     }
     (void)wpb;
     if (!opt.dry && dmax >= 1)
-        VX_LAUNCH(h, KID_COMMIT, k_commit<T VX_COMMA TILE>, h->tune.commit_grid, TILE, P);
+        VX_LAUNCH(h, KID_COMMIT, k_commit<T VX_COMMA TILE>, h->tune.commit_grid, TILE, P, dchunks, ddrift);
     return hipGetLastError() == hipSuccess ? VX_OK : VX_E_HIP;
     };
     auto launch_all = [&]() -> int {
@@ -570,23 +567,20 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     // chunk set-up, plus the old-tree descent over the level-3 slots in extra blocks
     unsigned np = grid_for(n);
     unsigned nd = L[3].nslots ? grid_for(L[3].nslots) : 0u;
-    unsigned nl = P.leaf_ids && dmax >= 2 ? 65536u / kBlock : 0u;
-    VX_LAUNCH(h, KID_PREPARE, k_prepare<T>, np + nd + nl, kBlock, P, dchunks, (uint32_t)n, roots, pre_status, np,
+    VX_LAUNCH(h, KID_PREPARE, k_prepare<T>, np + nd, kBlock, P, dchunks, (uint32_t)n, roots, pre_status, np,
               nd, L[3], doff, O);
     unsigned t1 = (unsigned)ntiles[1];
     if (dmax >= 2 && br == kBR)
         VX_LAUNCH(h, KID_BRICK_BUILD, k_brick_build<T VX_COMMA TILE VX_COMMA kBR>, t1 / kBR, TILE, P, dchunks, L[1],
-                  res_ptrs_h[1], K[1], tiles_h[1], ddef, ddrift, O.at[2]);
+                  res_ptrs_h[1], K[1], tiles_h[1], ddrift, O.at[2]);
     else if (dmax >= 2 && br == 2)
         VX_LAUNCH(h, KID_BRICK_BUILD, k_brick_build<T VX_COMMA TILE VX_COMMA 2>, t1 / 2, TILE, P, dchunks, L[1],
-                  res_ptrs_h[1], K[1], tiles_h[1], ddef, ddrift, O.at[2]);
+                  res_ptrs_h[1], K[1], tiles_h[1], ddrift, O.at[2]);
     else if (dmax >= 2)
         VX_LAUNCH(h, KID_BRICK_BUILD, k_brick_build<T VX_COMMA TILE VX_COMMA 1>, t1, TILE, P, dchunks, L[1],
-                  res_ptrs_h[1], K[1], tiles_h[1], ddef, ddrift, O.at[2]);
-    VX_LAUNCH(h, KID_LEAF_ALLOC, k_leaf_alloc<T>, 1, 1024, P, dchunks, (uint32_t)n, nvalues);
+                  res_ptrs_h[1], K[1], tiles_h[1], ddrift, O.at[2]);
+    if (opt.dry) VX_LAUNCH(h, KID_DRY_LEAVES, k_dry_leaves<T>, sizeof(T) == 1 ? 1 : 256, kBlock, P);
     if (dmax >= 2) {
-        VX_LAUNCH(h, KID_BRICK_SCAN, k_brick_retry<T VX_COMMA TILE>, 1024, kBlock, P, dchunks, L[1], res_ptrs_h[1], K[1],
-                  tiles_h[1], ddef, ddrift);
         uint32_t g1 = probe_group(t1, h->tune.probe_blocks_bricks);
         VX_LAUNCH(h, KID_PROBE_BRICKS, k_probe_bricks<T VX_COMMA TILE>, (t1 + g1 - 1) / g1, TILE, P, K[1], tiles_h[1],
                   res_ptrs_h[1], dchunks, L[1], t1, g1);
@@ -599,7 +593,7 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
                       res_ptrs_h[hh], dchunks, L[hh], th, gh);
         }
         // every level's new nodes, written once no probe runs any more
-        if (!opt.dry) VX_LAUNCH(h, KID_COMMIT, k_commit<T VX_COMMA TILE>, h->tune.commit_grid, TILE, P);
+        if (!opt.dry) VX_LAUNCH(h, KID_COMMIT, k_commit<T VX_COMMA TILE>, h->tune.commit_grid, TILE, P, dchunks, ddrift);
     }
     }
     uint32_t* gf0 = (uint32_t*)h->gc_front[0].ptr;
@@ -811,9 +805,8 @@ int fill_impl(vx_interner* h, size_t n, uint64_t* roots, const uint64_t* vals) {
     if (!h->gc_front[0].ensure(gcap * 4) || !h->gc_front[1].ensure(gcap * 4)) return VX_E_HIP;
     uint32_t* gf0 = (uint32_t*)h->gc_front[0].ptr;
     uint32_t* gf1 = (uint32_t*)h->gc_front[1].ptr;
-    uint32_t nvalues = sizeof(T) <= 2 ? 1u << (8 * sizeof(T)) : 0u;
     VX_LAUNCH(h, KID_BEGIN, k_begin, 1, 1, h->ctl);
-    VX_LAUNCH(h, KID_FILL, k_fill_prepare<T>, grid_for(n), kBlock, P, (uint32_t)n, roots, vals, gf0);
+    VX_LAUNCH(h, KID_FILL, k_fill_prepare<T>, grid_for(n), kBlock, P, (uint32_t)n, roots, gf0);
     for (uint32_t r = 0; r < (uint32_t)kLevels + 1; r++) {
         uint32_t* fr = (r & 1) ? gf1 : gf0;
         uint32_t* nx = (r & 1) ? gf0 : gf1;
@@ -822,7 +815,6 @@ int fill_impl(vx_interner* h, size_t n, uint64_t* roots, const uint64_t* vals) {
         VX_LAUNCH(h, KID_GC, k_gc_round<T>, grid, kBlock, P, r, fr, nx, r == 0, (uint64_t)gcap, false);
     }
     VX_LAUNCH(h, KID_BEGIN, k_begin, 1, 1, h->ctl);
-    VX_LAUNCH(h, KID_LEAF_ALLOC, k_leaf_alloc_only<T>, 1, 1024, P, nvalues);
     VX_LAUNCH(h, KID_FILL, k_fill_finish<T>, grid_for(n), kBlock, P, (uint32_t)n, roots, vals);
     VX_LAUNCH(h, KID_END_ALLOC, k_end_alloc<T>, 1, 256, P, false, (uint32_t*)nullptr);
     return hipGetLastError() == hipSuccess ? VX_OK : VX_E_HIP;
@@ -950,11 +942,11 @@ int vx_interner_create(uint32_t value_size, uint64_t budget_bytes, double load_f
     bool ok = dmalloc(&h->children, cap * 64) && dmalloc(&h->tmg, cap * 4) &&
               dmalloc(&h->values, cap * value_size) && dmalloc(&h->refs, cap * 4) &&
               dmalloc(&h->free_stack, cap * 4) &&
-              dmalloc(&h->tab, ts * 8) && dmalloc(&h->leaf_map, nv * 4) &&
+              dmalloc(&h->tab, ts * 8) &&
               dmalloc(&h->leaf_need, nv) && dmalloc(&h->new_leaves, nnew * 4) &&
               (direct || (dmalloc(&h->ltab, h->lslots * 8) && dmalloc(&h->need_list, h->lslots * 4))) &&
               (!direct || dmalloc(&h->single, 8 * nv * 8)) &&
-              (value_size != 2 || dmalloc(&h->leaf_ids, nv * 8)) &&
+              (!direct || (dmalloc(&h->leaf_ids, nv * 8) && dmalloc(&h->leaf_claim, nv * 4))) &&
               dmalloc(&h->ctl, sizeof(Ctl));
     if (!ok || hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) {
         vx_interner_destroy(h);
@@ -967,7 +959,9 @@ int vx_interner_create(uint32_t value_size, uint64_t budget_bytes, double load_f
              hipMemset(h->tmg, 0, cap * 4) == hipSuccess &&
              hipMemset(h->values, 0, cap * value_size) == hipSuccess &&
              hipMemset(h->refs, 0, cap * 4) == hipSuccess &&
-             hipMemset(h->tab, 0, ts * 8) == hipSuccess && hipMemset(h->leaf_map, 0, nv * 4) == hipSuccess &&
+             hipMemset(h->tab, 0, ts * 8) == hipSuccess &&
+             (!direct || (hipMemset(h->leaf_ids, 0, nv * 8) == hipSuccess &&
+                          hipMemset(h->leaf_claim, 0, nv * 4) == hipSuccess)) &&
              hipMemset(h->leaf_need, 0, nv) == hipSuccess &&
              (direct || hipMemset(h->ltab, 0, h->lslots * 8) == hipSuccess) &&
              (!direct || hipMemset(h->single, 0, 8 * nv * 8) == hipSuccess);
@@ -989,7 +983,7 @@ int vx_interner_destroy(vx_interner* h) {
     if (!h) return VX_OK;
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     void* ptrs[] = {h->children, h->tmg, h->values, h->refs, h->free_stack,
-                    h->tab, h->leaf_map, h->leaf_need, h->new_leaves, h->ctl, h->leaf_ids,
+                    h->tab, h->leaf_claim, h->leaf_need, h->new_leaves, h->ctl, h->leaf_ids,
                     h->ltab, h->need_list, h->single};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -1000,7 +994,6 @@ int vx_interner_destroy(vx_interner* h) {
     h->gc_front[1].release();
     h->stage.release();
     h->scratch.release();
-    h->deferred.release();
     h->drift.release();
     h->undo.release();
     h->owners.release();

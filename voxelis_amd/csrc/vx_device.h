@@ -111,10 +111,10 @@ struct Ctl {
     uint32_t next_index;  // bump cursor (interner/macros.rs:16-34)
     uint32_t free_top0;   // snapshot at the start of a launch sequence
     uint32_t next0;
-    uint32_t alloc_count;  // allocations in the current sequence
+    uint32_t alloc_count;  // branch nodes allocated in the current sequence (ranks after its new leaves)
     uint32_t err;
-    uint32_t n_new_leaves;
-    uint32_t n_deferred;  // bricks waiting for leaves created later in the sequence
+    uint32_t n_new_leaves;  // leaves created in the current sequence: allocation ranks [0, n_new_leaves)
+    uint32_t epoch;         // counts launch sequences: marks the leaf claims of the current one
     uint64_t live_leaves;
     uint64_t live_branches;
     uint32_t rebuild;   // this call rebuilds the pattern table (bit 0) and the i32 leaf table (bit 1)
@@ -125,18 +125,12 @@ struct Ctl {
     uint32_t abort_;          // this apply could not allocate: 1 capacity, 2 reservation
     uint32_t n_undo;          // entries of the undo log (reference-count deltas applied)
     uint32_t h1_fail;         // a tree of this apply failed in the brick pass (leaf-brick panic)
-    uint32_t n_need;          // i32: values requested by this apply (need_list entries)
-    uint32_t n_owners;        // new branch nodes of the last apply (its owner list), for the GC
-    uint32_t pad1;
+    uint32_t n_need;          // i32: values a dry run requested (need_list entries)
     uint32_t ncand[kLevels + 1];
     uint32_t gc_count[kLevels + 2];
-    uint32_t own_base;  // alloc_count when the apply's first probe starts
+    uint32_t pad1;
     // statistics, striped over 64 cache lines by block index (summed when read)
     uint64_t st[kStatStripes][32];
-    // u8 interners: the leaf id of every value at the start of the current apply
-    // (written by k_prepare, read by the brick pass; leaves created later in the
-    // apply are not in it)
-    uint64_t leaf_ids8[256];
 };
 
 // Per-tree record of one apply launch sequence (trees sorted by depth on the host).
@@ -207,14 +201,14 @@ struct Pool {
     uint64_t* tab;
     uint64_t tmask;
     uint64_t* single;  // u8/u16: the direct-mapped index of one-leaf keys (nullptr: none)
-    uint32_t* leaf_map;  // u8/u16: value -> node index (0 = none)
+    uint64_t* leaf_ids;    // u8/u16: the leaf id of every value (0: none)
+    uint32_t* leaf_claim;  // u8/u16: the epoch in which a value's leaf was last claimed for creation
     uint64_t* ltab;      // i32: open-addressing leaf table (value << 32 | index)
     uint64_t lmask;      // its slot count - 1
-    uint32_t* need_list; // i32: values requested by this apply (k_leaf_alloc creates them)
+    uint32_t* need_list; // i32: values requested by a dry run
     uint32_t need_cap;
-    uint64_t* leaf_ids;  // u16: the leaf id of every value at the start of the apply (k_prepare)
-    uint8_t* leaf_need;
-    uint32_t* new_leaves;
+    uint8_t* leaf_need;   // u8/u16: values requested by a dry run
+    uint32_t* new_leaves; // by allocation rank: the leaves this sequence created
     Ctl* ctl;
     uint32_t capacity;
     uint32_t dry;          // 1: count what an apply would create, change nothing
@@ -224,7 +218,7 @@ struct Pool {
     uint32_t* per_tree;    // optional: new branch nodes owned by each tree (caller's index)
     const Cands* levels;   // candidate arrays of every level (pending keys of earlier levels)
     Drift* undo;           // reference-count deltas applied outside commits (rolled back on abort)
-    uint64_t* owners;      // by allocation rank - Ctl::own_base: (height << 32) | candidate
+    uint64_t* owners;      // by allocation rank after the new leaves: (height << 32) | candidate
     uint32_t undo_cap;
 };
 

@@ -208,13 +208,12 @@ __device__ inline uint32_t calc_average(const uint32_t v[8]) {
 
 // ------------------------------------------------------------------ leaf table
 
-// value -> leaf node index (get_or_create_leaf's map, interner/mod.rs:627-710).  u8/u16:
-// direct-mapped arrays (leaf_map; leaf_need marks values to create).  i32: 2^32 values
-// cannot be mapped directly, so an open-addressing table (ltab) of 8-byte slots
-// value << 32 | index: 0 empty, kLeafTomb a removed entry (value 0 never has a leaf), and
-// index kLeafNeed a value requested by this apply and not created yet; the claim that
-// inserts a request lists the value once (need_list) for k_leaf_alloc.  A value is the
-// whole key, so a slot compare is the full-key compare.
+// value -> leaf (get_or_create_leaf's map, interner/mod.rs:627-710).  u8/u16: a
+// direct-mapped array of leaf ids.  i32: 2^32 values cannot be mapped directly, so an
+// open-addressing table (ltab) of 8-byte slots value << 32 | index: 0 empty, kLeafTomb a
+// removed entry (value 0 never has a leaf), and index kLeafNeed a value whose leaf is being
+// created (leaf_acquire) or that a dry run requested.  A value is the whole key, so a slot
+// compare is the full-key compare.
 constexpr uint64_t kLeafTomb = 1ull;
 constexpr uint32_t kLeafNeed = 0xFFFFFFFFu;
 
@@ -233,11 +232,11 @@ __device__ inline uint64_t ltab_find(const Pool<T>& P, uint32_t v) {
     return ~0ull;
 }
 
-// The live leaf index of value v (0: none, or requested and not created yet).
+// The live leaf index of value v (0: none).
 template <typename T>
 __device__ inline uint32_t leaf_index(const Pool<T>& P, uint32_t v) {
     if constexpr (sizeof(T) <= 2) {
-        return P.leaf_map[v];
+        return bid_index(P.leaf_ids[v]);
     } else {
         const uint64_t s = ltab_find(P, v);
         if (s == ~0ull) return 0;
@@ -246,60 +245,229 @@ __device__ inline uint32_t leaf_index(const Pool<T>& P, uint32_t v) {
     }
 }
 
-// Ask k_leaf_alloc to create the leaf of value v; returns the key of its dry-run
-// placeholder id (capacity + key): the value itself for u8/u16, the request's slot for
-// i32 (one per value, the same for every requester).
+// Loads and stores that see and show other compute dies' work of the same launch.
+template <typename V>
+__device__ inline V load_agent(const V* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename V>
+__device__ inline void store_agent(V* p, V v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// i32: the entry of value v, inserted as kLeafNeed when there is none (*won).  Returns its
+// slot, or ~0 when the table is full.
+template <typename T>
+__device__ inline uint64_t ltab_claim(const Pool<T>& P, uint32_t v, bool* won, uint64_t* entry) {
+    *won = false;
+    *entry = 0;
+    uint64_t s = leaf_hash(v) & P.lmask;
+    uint64_t first_tomb = ~0ull;
+    for (uint64_t g = 0; g <= 4 * (P.lmask + 1); g++) {
+        const uint64_t e = P.ltab[s];
+        if (e != 0 && e != kLeafTomb && (uint32_t)(e >> 32) == v) {
+            *entry = e;
+            return s;
+        }
+        if (e == kLeafTomb && first_tomb == ~0ull) first_tomb = s;
+        if (e == 0 || (first_tomb != ~0ull && g > P.lmask)) {
+            const uint64_t target = first_tomb != ~0ull ? first_tomb : s;
+            const uint64_t expected = first_tomb != ~0ull ? kLeafTomb : 0ull;
+            const uint64_t want = ((uint64_t)v << 32) | kLeafNeed;
+            // (a plain load of a value that is taken everywhere at once may be old: a fresh
+            // one first, so that not every wavefront's exchange meets at one slot)
+            uint64_t seen = load_agent(&P.ltab[target]);
+            if (seen == expected)
+                seen = atomicCAS((unsigned long long*)&P.ltab[target], (unsigned long long)expected,
+                                 (unsigned long long)want);
+            if (seen == expected) {
+                *won = true;
+                *entry = want;
+                return target;
+            }
+            if ((uint32_t)(seen >> 32) == v && seen != kLeafTomb) {
+                *entry = seen;
+                return target;
+            }
+            s = (target + 1) & P.lmask;  // another value took the slot: go on behind it
+            first_tomb = ~0ull;
+            continue;
+        }
+        s = (s + 1) & P.lmask;
+    }
+    atomicOr(&P.ctl->err, kErrTableFull | kErrPoison);
+    return ~0ull;
+}
+
+// i32: the slot and current entry of value v (0: none).
+template <typename T>
+__device__ inline uint64_t ltab_peek(const Pool<T>& P, uint32_t v, uint64_t* slot) {
+    uint64_t s = leaf_hash(v) & P.lmask;
+    for (uint64_t g = 0; g <= P.lmask; g++) {
+        const uint64_t e = load_agent(&P.ltab[s]);
+        *slot = s;
+        if (e == 0 || (e != kLeafTomb && (uint32_t)(e >> 32) == v)) return e;
+        s = (s + 1) & P.lmask;
+    }
+    return 0;
+}
+
+// A dry run's request for the leaf of value v; returns the key of its placeholder id
+// (capacity + key): the value itself for u8/u16, the request's slot for i32 (one per value,
+// the same for every requester).
 template <typename T>
 __device__ inline uint32_t leaf_request(const Pool<T>& P, uint32_t v) {
     if constexpr (sizeof(T) <= 2) {
         P.leaf_need[v] = 1;
         return v;
     } else {
-        uint64_t s = leaf_hash(v) & P.lmask;
-        uint64_t first_tomb = ~0ull;
-        for (uint64_t g = 0; g <= 4 * (P.lmask + 1); g++) {
-            const uint64_t e = P.ltab[s];
-            if (e != 0 && e != kLeafTomb && (uint32_t)(e >> 32) == v) return (uint32_t)s;
-            if (e == kLeafTomb && first_tomb == ~0ull) first_tomb = s;
-            if (e == 0 || (first_tomb != ~0ull && g > P.lmask)) {
-                const uint64_t target = first_tomb != ~0ull ? first_tomb : s;
-                const uint64_t expected = first_tomb != ~0ull ? kLeafTomb : 0ull;
-                const uint64_t want = ((uint64_t)v << 32) | kLeafNeed;
-                const uint64_t seen = atomicCAS((unsigned long long*)&P.ltab[target], (unsigned long long)expected,
-                                                (unsigned long long)want);
-                if (seen == expected) {
-                    const uint32_t pos = atomicAdd(&P.ctl->n_need, 1u);
-                    if (pos < P.need_cap) P.need_list[pos] = v;
-                    else atomicOr(&P.ctl->err, kErrTableFull | kErrPoison);
-                    return (uint32_t)target;
-                }
-                if ((uint32_t)(seen >> 32) == v && seen != kLeafTomb) return (uint32_t)target;
-                s = (target + 1) & P.lmask;  // another value took the slot: go on behind it
-                first_tomb = ~0ull;
-                continue;
-            }
-            s = (s + 1) & P.lmask;
+        bool won;
+        uint64_t e;
+        const uint64_t s = ltab_claim(P, v, &won, &e);
+        if (won) {
+            const uint32_t pos = atomicAdd(&P.ctl->n_need, 1u);
+            if (pos < P.need_cap) P.need_list[pos] = v;
+            else atomicOr(&P.ctl->err, kErrTableFull | kErrPoison);
         }
-        atomicOr(&P.ctl->err, kErrTableFull | kErrPoison);
-        return 0;
+        return (uint32_t)s;
     }
 }
 
-// Publish the leaf index of value v (k_leaf_alloc, snapshot import).
+template <typename T>
+__device__ inline uint32_t alloc_at(const Pool<T>& P, uint32_t k, bool* ok, uint32_t ft0, uint32_t next0);
+
+// The leaf id of value v as it is now, whoever created it (kEmpty: none).
+template <typename T>
+__device__ inline uint64_t leaf_now(const Pool<T>& P, uint32_t v) {
+    if constexpr (sizeof(T) <= 2) {
+        return load_agent(&P.leaf_ids[v]);
+    } else {
+        uint64_t slot;
+        const uint64_t e = ltab_peek(P, v, &slot);
+        return e && (uint32_t)e != kLeafNeed ? make_leaf((uint32_t)e, tmg_gen(P.tmg[(uint32_t)e])) : kEmpty;
+    }
+}
+
+// get_or_create_leaf (interner/mod.rs:669-708) for values that had no leaf when their
+// launch looked: when it returns, value(i) has a leaf (leaf_now finds it) for every bit i < n
+// of need, created by one lane of the launch and awaited by the others, or could not be
+// allocated (the apply then aborts).  Called by any lanes of a wavefront together.
+//
+// A new leaf used to be requested here and created by one block of a later launch, and its
+// bricks rebuilt by a third one: a new id written everywhere (64 x 64 terrain trees, u8)
+// took 1.24 ms of brick passes and takes 0.14 ms here; 0.85 M new 32-bit ids took 56 ms of
+// creation and as much again to take their requests back, and are 1.2 ms of the 1.6 ms pass.
+//
+// A lane that claims a value (its epoch word, or the i32 table's slot) publishes the id
+// without waiting for anyone, and every claim of a wavefront is published before one of its
+// lanes waits, so every wait ends; it also ends when an allocation fails, and it is bounded.
+// Ids are exchanged with agent-scope accesses; the new node's columns are read by later
+// launches only.  (The loops are kept rolled: this is the rare path of kernels whose
+// registers are full.)
+template <typename T, typename V>
+__device__ inline void leaf_ensure(const Pool<T>& P, uint32_t need, int n, V value) {
+    const uint32_t lane = __lane_id();
+    const uint64_t below = (1ull << lane) - 1ull;
+    uint32_t won = 0, wait = 0;
+    if (!__ballot(need != 0)) return;
+#pragma unroll 1
+    for (int i = 0; i < n; i++) {
+        bool on = (need >> i) & 1u, pending = on;
+        if (!__ballot(on)) continue;
+        const uint32_t v = value(i);
+        // one lane a value asks for the few values that many lanes miss
+#pragma unroll 1
+        for (int r = 0; r < kMatchRounds; r++) {
+            const uint64_t act = __ballot(pending);
+            if (!act) break;
+            const int leader = __ffsll((unsigned long long)act) - 1;
+            const bool same = pending && v == (uint32_t)__builtin_amdgcn_readlane(v, leader);
+            if (same && (int)lane != leader) {
+                on = false;
+                wait |= 1u << i;
+            }
+            if (same) pending = false;
+        }
+        if (on) {
+            bool w = false;
+            if constexpr (sizeof(T) <= 2) {
+                const uint32_t epoch = P.ctl->epoch, c = load_agent(&P.leaf_claim[v]);
+                if (load_agent(&P.leaf_ids[v]) == kEmpty) {
+                    w = c != epoch && atomicCAS(&P.leaf_claim[v], c, epoch) == c;
+                    wait |= (w ? 0u : 1u) << i;
+                }
+            } else {
+                uint64_t e;
+                if (ltab_claim(P, v, &w, &e) != ~0ull) wait |= (w ? 0u : 1u) << i;
+            }
+            won |= (w ? 1u : 0u) << i;
+        }
+    }
+    uint32_t total = 0;
+    for (int i = 0; i < n; i++) total += (uint32_t)__popcll(__ballot((won >> i) & 1u));
+    if (total) {  // uniform over the calling lanes
+        const int leader = __ffsll((unsigned long long)__ballot(true)) - 1;
+        uint32_t k = 0;
+        if ((int)lane == leader) k = atomicAdd(&P.ctl->n_new_leaves, total);
+        k = __shfl(k, leader);
+        const uint32_t ft0 = P.ctl->free_top0, next0 = P.ctl->next0;
+#pragma unroll 1
+        for (int i = 0; i < n; i++) {
+            const uint64_t b = __ballot((won >> i) & 1u);
+            if ((won >> i) & 1u) {
+                const uint32_t rank = k + (uint32_t)__popcll(b & below), v = value(i);
+                bool ok;
+                const uint32_t idx = alloc_at(P, rank, &ok, ft0, next0);
+                uint64_t slot = 0;
+                if constexpr (sizeof(T) == 4) ltab_peek(P, v, &slot);
+                if (ok) {
+                    const uint32_t gen = tmg_gen(P.tmg[idx]);
+                    // a recycled node keeps its old children (the free does not clear
+                    // them): a leaf has none.  Its count is 0 already.
+                    ulonglong2* ch = (ulonglong2*)(P.children + 8ull * idx);
+                    for (int j = 0; j < 4; j++) ch[j] = ulonglong2{kEmpty, kEmpty};
+                    P.values[idx] = (T)v;
+                    P.tmg[idx] = tmg_make(0u, gen);
+                    P.new_leaves[rank] = idx;
+                    if constexpr (sizeof(T) <= 2) store_agent(&P.leaf_ids[v], make_leaf(idx, gen));
+                    else store_agent(&P.ltab[slot], ((uint64_t)v << 32) | idx);
+                } else if constexpr (sizeof(T) == 4) {
+                    store_agent(&P.ltab[slot], kLeafTomb);
+                }
+            }
+            k += (uint32_t)__popcll(b);
+        }
+    }
+#pragma unroll 1
+    for (int i = 0; i < n; i++) {
+        if (!((wait >> i) & 1u)) continue;
+        for (uint32_t g = 0; leaf_now(P, value(i)) == kEmpty && !load_agent(&P.ctl->abort_); g++) {
+            if (g == 1u << 20) {
+                atomicOr(&P.ctl->err, kErrPoison);
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+    }
+}
+
+// The same for one value.
+template <typename T>
+__device__ inline uint64_t leaf_acquire(const Pool<T>& P, uint32_t v) {
+    leaf_ensure(P, 1u, 1, [&](int) { return v; });
+    return leaf_now(P, v);
+}
+
+// Publish the leaf index of value v (snapshot import, table rebuild).
 template <typename T>
 __device__ inline void leaf_publish(const Pool<T>& P, uint32_t v, uint32_t idx) {
     if constexpr (sizeof(T) <= 2) {
-        P.leaf_map[v] = idx;
+        P.leaf_ids[v] = make_leaf(idx, tmg_gen(P.tmg[idx]));
     } else {
         const uint64_t want = ((uint64_t)v << 32) | idx;
         uint64_t s = leaf_hash(v) & P.lmask;
         for (uint64_t g = 0; g <= P.lmask; g++) {
-            const uint64_t e = P.ltab[s];
-            if (e != 0 && e != kLeafTomb && (uint32_t)(e >> 32) == v) {  // its request
-                P.ltab[s] = want;
-                return;
-            }
-            if (e == 0 && atomicCAS((unsigned long long*)&P.ltab[s], 0ull, (unsigned long long)want) == 0ull) return;
+            if (atomicCAS((unsigned long long*)&P.ltab[s], 0ull, (unsigned long long)want) == 0ull) return;
             s = (s + 1) & P.lmask;
         }
         atomicOr(&P.ctl->err, kErrTableFull | kErrPoison);
@@ -310,7 +478,7 @@ __device__ inline void leaf_publish(const Pool<T>& P, uint32_t v, uint32_t idx) 
 template <typename T>
 __device__ inline void leaf_remove(const Pool<T>& P, uint32_t v) {
     if constexpr (sizeof(T) <= 2) {
-        P.leaf_map[v] = 0;
+        P.leaf_ids[v] = kEmpty;
     } else {
         const uint64_t s = ltab_find(P, v);
         if (s != ~0ull) {
@@ -318,20 +486,6 @@ __device__ inline void leaf_remove(const Pool<T>& P, uint32_t v) {
             atomicAdd((unsigned long long*)stat(P.ctl, ST_LTOMB), 1ull);
         }
     }
-}
-
-template <typename T>
-__device__ inline uint64_t leaf_id_of(const Pool<T>& P, uint32_t v) {
-    uint32_t idx = leaf_index(P, v);
-    return make_leaf(idx, tmg_gen(P.tmg[idx]));
-}
-
-template <typename T>
-__device__ inline uint32_t alloc_at(const Pool<T>& P, uint32_t k, bool* ok, uint32_t ft0, uint32_t next0);
-
-template <typename T>
-__device__ inline uint32_t alloc_node(const Pool<T>& P, bool* ok) {
-    return alloc_at(P, atomicAdd(&P.ctl->alloc_count, 1u), ok, P.ctl->free_top0, P.ctl->next0);
 }
 
 // The index of the launch sequence's k-th allocation: the free stack first, then
@@ -356,6 +510,13 @@ __device__ inline uint32_t alloc_at(const Pool<T>& P, uint32_t k, bool* ok, uint
     }
     *ok = true;
     return (uint32_t)b;
+}
+
+// How many of the first n allocation ranks got a node (the others failed in alloc_at).
+template <typename T>
+__device__ inline uint64_t alloc_done(const Pool<T>& P, uint64_t n) {
+    const uint64_t room = (uint64_t)P.ctl->free_top0 + (P.capacity > P.ctl->next0 ? P.capacity - P.ctl->next0 : 0u);
+    return min(n, min((uint64_t)P.alloc_limit, room));
 }
 
 // A reference-count delta applied outside a commit, logged so an aborted apply
@@ -450,14 +611,14 @@ __device__ inline void ctl_begin(Ctl* ctl) {
         ctl->next0 = ctl->next_index;
         ctl->alloc_count = 0;
         ctl->n_new_leaves = 0;
-        ctl->n_deferred = 0;
+        ctl->epoch++;
+        ctl->n_need = 0;
         ctl->n_drift = 0;
         ctl->dry_owners = 0;
         ctl->dry_new_leaves = 0;
         ctl->abort_ = 0;
         ctl->n_undo = 0;
         ctl->h1_fail = 0;
-        ctl->n_owners = 0;
         for (int i = 0; i <= kLevels; i++) ctl->ncand[i] = 0;
         for (int i = 0; i < kLevels + 2; i++) ctl->gc_count[i] = 0;
     }
@@ -467,59 +628,59 @@ __global__ void k_begin(Ctl* ctl) {
     if (blockIdx.x == 0 && threadIdx.x == 0) ctl_begin(ctl);
 }
 
-// i32: requests still open at the end of an apply (a dry run's, whose placeholders were
-// counted; a leaf whose creation failed) leave the table.  One block.
+// A dry run's leaf requests are counted and dropped once the brick pass has made them
+// (their placeholder ids are in the keys by then).
 template <typename T>
-__device__ inline void drop_requests(const Pool<T>& P) {
-    if constexpr (sizeof(T) == 4) {
-        const uint32_t nn = min(P.ctl->n_need, P.need_cap);
-        for (uint32_t i = threadIdx.x; i < nn; i += blockDim.x) {
-            const uint64_t sl = ltab_find(P, P.need_list[i]);
-            if (sl != ~0ull && (uint32_t)P.ltab[sl] == kLeafNeed) P.ltab[sl] = kLeafTomb;
+__global__ void k_dry_leaves(Pool<T> P) {
+    const uint32_t n = sizeof(T) == 4 ? min(P.ctl->n_need, P.need_cap) : 1u << (8 * sizeof(T));
+    VX_LOOP(i, n) {
+        bool created = false;
+        if (i < n) {
+            if constexpr (sizeof(T) == 4) {
+                const uint64_t sl = ltab_find(P, P.need_list[i]);
+                created = sl != ~0ull && (uint32_t)P.ltab[sl] == kLeafNeed;
+                if (created) P.ltab[sl] = kLeafTomb;
+            } else if (P.leaf_need[i]) {
+                P.leaf_need[i] = 0;
+                created = P.leaf_ids[i] == kEmpty;
+            }
         }
+        wave_append(&P.ctl->dry_new_leaves, created);
     }
 }
 
 // Close the allocation window of a launch sequence.  An aborted apply
 // (rollback = true) gives every allocation back instead: the allocator cursors
-// stay, reference counts of the taken indices go back to zero and new leaves
-// leave the value map.  counts (optional): new branches, new leaves.
+// stay and reference counts of the taken indices go back to zero (the rollback took the
+// new leaves off the value map).  counts (optional): new branches, new leaves.
 template <typename T>
 __global__ void k_end_alloc(Pool<T> P, bool rollback, uint32_t* counts) {
     Ctl* ctl = P.ctl;
+    const uint32_t n = ctl->n_new_leaves + ctl->alloc_count;
     const bool abort = rollback && !P.dry && ctl->abort_ != 0;
     if (abort) {
-        uint32_t n = ctl->alloc_count;
         uint32_t ft0 = ctl->free_top0;
-        uint64_t room = (uint64_t)ft0 + (P.capacity > ctl->next0 ? P.capacity - ctl->next0 : 0u);
-        uint64_t nok = n;
-        if (nok > P.alloc_limit) nok = P.alloc_limit;
-        if (nok > room) nok = room;
+        const uint64_t nok = alloc_done(P, n);
         for (uint64_t i = threadIdx.x; i < nok; i += blockDim.x) {
             uint32_t idx = i < ft0 ? P.free_stack[ft0 - 1 - i] : (uint32_t)(ctl->next0 + (i - ft0));
             P.refs[idx] = 0;
         }
-        uint32_t nl = ctl->n_new_leaves;
-        for (uint32_t i = threadIdx.x; i < nl; i += blockDim.x)
-            leaf_remove(P, (uint32_t)P.values[P.new_leaves[i]]);
-        drop_requests(P);
         __syncthreads();
         if (threadIdx.x == 0) {
-            ctl->live_leaves -= nl;
             ctl->n_new_leaves = 0;
             ctl->alloc_count = 0;
             if (counts) counts[0] = counts[1] = 0xFFFFFFFFu;
         }
         return;
     }
-    drop_requests(P);
     if (threadIdx.x == 0) {
-        uint32_t n = ctl->alloc_count;
-        ctl->n_owners = P.dry || n < ctl->own_base ? 0u : n - ctl->own_base;
         if (counts) {
-            counts[0] = P.dry ? ctl->dry_owners : n - ctl->n_new_leaves;
+            counts[0] = P.dry ? ctl->dry_owners : ctl->alloc_count;
             counts[1] = P.dry ? ctl->dry_new_leaves : ctl->n_new_leaves;
         }
+        const uint64_t made = alloc_done(P, ctl->n_new_leaves);
+        ctl->live_leaves += made;
+        *stat(ctl, ST_LEAF_MISS) += made;
         uint32_t used_free = n < ctl->free_top0 ? n : ctl->free_top0;
         ctl->free_top = ctl->free_top0 - used_free;
         uint64_t nx = (uint64_t)ctl->next0 + (n - used_free);
@@ -574,133 +735,43 @@ __device__ inline void descend_body(const Pool<T>& P, const ChunkDev* chunks, co
     for (int i = 0; i < 8; i++) dst[i] = below[i];
 }
 
-// Read roots, mark the fill leaf as needed (Phase 0, voxtree.rs:742-754).  Blocks
-// nprep..nprep+ndesc run the old-tree descent over the level-3 slots instead, and the
-// blocks after them (u16) record the leaf id of every value for the brick pass.
+// Read roots and take the fill leaf (Phase 0, voxtree.rs:742-754): a tree with a fill
+// starts from it, and the fill leaf of a batch that also has patches keeps its reference
+// (H3).  Blocks nprep..nprep+ndesc run the old-tree descent over the level-3 slots instead.
 template <typename T>
 __global__ void k_prepare(Pool<T> P, ChunkDev* chunks, uint32_t n, const uint64_t* roots,
                           const int32_t* pre_status, uint32_t nprep, uint32_t ndesc, LevelInfo L3,
                           const uint64_t* doff, OldNodes O) {
-    if (blockIdx.x >= nprep + ndesc) {
-        if (P.leaf_ids)
-            for (uint32_t v = (blockIdx.x - nprep - ndesc) * blockDim.x + threadIdx.x; v < 65536u;
-                 v += (gridDim.x - nprep - ndesc) * blockDim.x) {
-                const uint32_t li = P.leaf_map[v];
-                P.leaf_ids[v] = li ? make_leaf(li, tmg_gen(P.tmg[li])) : kEmpty;
-            }
-        return;
-    }
     if (blockIdx.x >= nprep) {
         uint64_t stride = (uint64_t)ndesc * blockDim.x;
         for (uint64_t s = (uint64_t)(blockIdx.x - nprep) * blockDim.x + threadIdx.x; s < L3.nslots; s += stride)
             descend_body(P, chunks, L3, doff, n, O, roots, s);
         return;
     }
-    // the sequence's control-block reset rides in block 0 (nothing else here reads it)
-    if (blockIdx.x == 0 && threadIdx.x == 0) ctl_begin(P.ctl);
-    if (sizeof(T) == 1 && blockIdx.x == 0)
-        for (uint32_t v = threadIdx.x; v < 256; v += blockDim.x) {
-            uint32_t li = P.leaf_map[v];
-            P.ctl->leaf_ids8[v] = li ? make_leaf(li, tmg_gen(P.tmg[li])) : kEmpty;
-        }
+    // a dry run's control-block reset rides in block 0 (nothing else here reads it); any
+    // other call's came with its table maintenance, since leaves are created here
+    if (P.dry && blockIdx.x == 0 && threadIdx.x == 0) ctl_begin(P.ctl);
     for (uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (uint64_t)nprep * blockDim.x) {
-        {
-            ChunkDev& C = chunks[c];
-            C.root_in = roots[C.orig];
-            C.init = C.root_in;
-            C.status = C.status0;
-            // a depth-2 tree's height-2 node is its root (deeper trees: the descent)
-            if (C.depth == 2 && C.has_patches && !C.has_fill) O.at[2][doff[(size_t)2 * n + c]] = C.root_in;
-            if (P.per_tree) P.per_tree[C.orig] = 0;
-            if (pre_status && pre_status[C.orig] < 0 && C.status >= 0) C.status = pre_status[C.orig];
-            if (C.status >= 0 && C.has_fill) {
-                uint32_t v = (uint32_t)C.fill;
-                if (leaf_index(P, v) == 0) leaf_request(P, v);
-            }
-        }
-    }
-}
-
-// ------------------------------------------------------------------ Phase 1
-
-// One block: create the leaves marked as needed (interner/mod.rs:669-708), then
-// fix each tree's Phase-1 start node.  The fill leaf of a batch that also has
-// patches keeps its reference (H3, voxtree.rs:742-754).
-// Create the leaves requested so far (one block; a dry run only counts them).  Returns
-// the number created (or counted).
-template <typename T>
-__device__ inline uint32_t create_requested_leaves(const Pool<T>& P, uint32_t nvalues) {
-    __shared__ uint32_t created;
-    if (threadIdx.x == 0) created = 0;
-    __syncthreads();
-    const uint32_t nreq = sizeof(T) == 4 ? min(P.ctl->n_need, P.need_cap) : nvalues;
-    for (uint32_t r = threadIdx.x; r < nreq; r += blockDim.x) {
-        uint32_t v = r;
-        uint64_t sl = 0;
-        if constexpr (sizeof(T) == 4) {
-            v = P.need_list[r];
-            sl = ltab_find(P, v);
-            if (sl == ~0ull || (uint32_t)P.ltab[sl] != kLeafNeed) continue;
-        } else {
-            if (!P.leaf_need[v]) continue;
-            P.leaf_need[v] = 0;
-            if (P.leaf_map[v] != 0) continue;
-        }
-        if (P.dry) {  // counted; an i32 request stays until the end of the apply (its placeholder)
-            atomicAdd(&created, 1u);
-            continue;
-        }
-        bool ok;
-        uint32_t idx = alloc_node(P, &ok);
-        if (ok) {
-            // a recycled node keeps its old children (the free does not clear them): a
-            // leaf has none
-            uint64_t* ch = P.children + 8ull * idx;
-#pragma unroll
-            for (int j = 0; j < 8; j++) ch[j] = kEmpty;
-            P.values[idx] = (T)v;
-            P.tmg[idx] &= 0xFFFF0000u;  // a leaf: no types/mask, the generation kept
-            P.refs[idx] = 0;
-            if constexpr (sizeof(T) == 4) P.ltab[sl] = ((uint64_t)v << 32) | idx;
-            else P.leaf_map[v] = idx;
-            uint32_t k = atomicAdd(&P.ctl->n_new_leaves, 1u);
-            P.new_leaves[k] = idx;
-            atomicAdd(&created, 1u);
-        } else if constexpr (sizeof(T) == 4) {
-            P.ltab[sl] = kLeafTomb;
-        }
-    }
-    __syncthreads();
-    return created;
-}
-
-// One block: create the leaves marked as needed (interner/mod.rs:669-708), then
-// fix each tree's Phase-1 start node.  The fill leaf of a batch that also has
-// patches keeps its reference (H3, voxtree.rs:742-754).
-template <typename T>
-__global__ void k_leaf_alloc(Pool<T> P, ChunkDev* chunks, uint32_t n, uint32_t nvalues) {
-    const uint32_t created = create_requested_leaves(P, nvalues);
-    if (threadIdx.x == 0) {
-        if (P.dry) {
-            P.ctl->dry_new_leaves += created;
-        } else {
-            atomicAdd((unsigned long long*)&P.ctl->live_leaves, (unsigned long long)created);
-            atomicAdd((unsigned long long*)stat(P.ctl, ST_LEAF_MISS), (unsigned long long)created);
-        }
-    }
-    for (uint32_t c = threadIdx.x; c < n; c += blockDim.x) {
         ChunkDev& C = chunks[c];
-        if (C.status < 0 || !C.has_fill) continue;
-        uint32_t idx = leaf_index(P, (uint32_t)C.fill);
-        if (idx == 0 && P.dry) {
-            C.init = make_leaf(P.capacity + leaf_request(P, (uint32_t)C.fill), 0);
-            continue;
-        }
-        if (idx == 0) continue;  // allocation failed (OOM flagged)
-        C.init = make_leaf(idx, tmg_gen(P.tmg[idx]));
-        if (C.has_patches && !P.dry) {
-            ref_delta_logged(P, c, idx, 1, ST_H3);
-            atomicAdd((unsigned long long*)stat(P.ctl, ST_H3), 1ull);
+        C.root_in = roots[C.orig];
+        C.init = C.root_in;
+        C.status = C.status0;
+        // a depth-2 tree's height-2 node is its root (deeper trees: the descent)
+        if (C.depth == 2 && C.has_patches && !C.has_fill) O.at[2][doff[(size_t)2 * n + c]] = C.root_in;
+        if (P.per_tree) P.per_tree[C.orig] = 0;
+        if (pre_status && pre_status[C.orig] < 0 && C.status >= 0) C.status = pre_status[C.orig];
+        if (C.status >= 0 && C.has_fill) {
+            const uint32_t v = (uint32_t)C.fill;
+            const uint32_t li = leaf_index(P, v);
+            const uint64_t id = li ? make_leaf(li, tmg_gen(P.tmg[li]))
+                                : P.dry ? make_leaf(P.capacity + leaf_request(P, v), 0) : leaf_acquire(P, v);
+            if (id != kEmpty) {
+                C.init = id;
+                if (C.has_patches && !P.dry) {
+                    ref_delta_logged(P, (uint32_t)c, bid_index(id), 1, ST_H3);
+                    atomicAdd((unsigned long long*)stat(P.ctl, ST_H3), 1ull);
+                }
+            }
         }
     }
 }
@@ -800,12 +871,11 @@ __device__ inline void tile_count(uint32_t* s, int id, bool pred) {
 // the all-same brick becomes a leaf; otherwise the brick's children are built from
 // the old node, a split leaf, or nothing, and the changed slots get leaves.
 // Returns: 0 = not pushed, 1 = leaf result in *out, 2 = branch key in ch/tm,
-// 3 = a needed leaf does not exist yet (marked; the brick is retried later).
+// 3 = a leaf could not be created (the apply aborts).
 // Reference-count corrections of the reference's split-leaf quirks are queued in
 // *drift_idx / *drift_delta (applied once the tree's status is final).
-// The leaf id of a value, or kEmpty when no leaf holds it.  leaf_ids (u8: LDS, u16: the
-// table k_prepare writes) caches it for every value; otherwise the direct-mapped table is
-// read.
+// The leaf id of a value, or kEmpty when no leaf holds it.  leaf_ids (u8: the block's copy
+// in LDS, u16: the direct-mapped table) has it for every value; i32 looks it up.
 template <typename T>
 __device__ inline uint64_t leaf_lookup(const Pool<T>& P, const uint64_t* leaf_ids, uint32_t v) {
     if (leaf_ids) return leaf_ids[v];
@@ -817,7 +887,7 @@ template <typename T>
 __device__ inline int brick_work(const Pool<T>& P, const ChunkDev& C, uint32_t m, const uint32_t v[8],
                                  uint64_t base, uint64_t* out, uint64_t ch[8], uint32_t* tm,
                                  uint32_t* drift_idx, int32_t* drift_delta, int* flags,
-                                 const uint64_t lids[8], bool request = true) {
+                                 const uint64_t lids[8]) {
     *drift_idx = kNoIdx;
     bool all_same = m == 0xFFu;
 #pragma unroll
@@ -825,9 +895,8 @@ __device__ inline int brick_work(const Pool<T>& P, const ChunkDev& C, uint32_t m
     if (all_same) {
         uint64_t lid = lids[0];
         if (lid == kEmpty) {
-            const uint32_t key = request ? leaf_request(P, v[0]) : 0u;
             if (!P.dry) return 3;
-            *out = make_leaf(P.capacity + key, 0);  // dry run: a placeholder for the new leaf
+            *out = make_leaf(P.capacity + leaf_request(P, v[0]), 0);  // dry run: a placeholder for the new leaf
         } else {
             *out = lid;
         }
@@ -840,9 +909,8 @@ __device__ inline int brick_work(const Pool<T>& P, const ChunkDev& C, uint32_t m
     if (fill_split) {
         uint32_t fi = leaf_index(P, (uint32_t)C.fill);
         if (fi == 0) {
-            const uint32_t key = request ? leaf_request(P, (uint32_t)C.fill) : 0u;
             if (P.dry) {
-                base = make_leaf(P.capacity + key, 0);
+                base = make_leaf(P.capacity + leaf_request(P, (uint32_t)C.fill), 0);
             } else {
                 missing = true;
                 base = make_leaf(0, 0);
@@ -883,12 +951,11 @@ __device__ inline int brick_work(const Pool<T>& P, const ChunkDev& C, uint32_t m
             if (same) continue;
         }
         if (lid == kEmpty) {
-            const uint32_t key = request ? leaf_request(P, v[i]) : 0u;
             if (!P.dry) {
                 missing = true;
                 continue;
             }
-            ch[i] = make_leaf(P.capacity + key, 0);
+            ch[i] = make_leaf(P.capacity + leaf_request(P, v[i]), 0);
         } else {
             ch[i] = lid;
         }
@@ -929,29 +996,27 @@ constexpr int brick_rounds() { return TILE >= 512 ? 2 : 4; }
 // block start + j*TILE + lane in round j).  Phase 1 issues every round's loads at
 // once (edit mask, the 8 values and the old height-2 node above the brick) and
 // settles the bricks that need no old tree: untouched ones and all-same ones whose
-// leaf exists.  The rest (mixed bricks; all-same ones whose leaf is still missing)
-// are queued in LDS with their loaded data and take phase 2, one per lane, in
-// rounds of TILE: the old-tree descent and brick_work.  Round r of phase 2 emits
-// into candidate tile blk*R + r; a deferred brick keeps that tile (its round has a
-// free place for it) for the retry.  The pass is bound by memory latency, so it runs
-// as many waves per SIMD as fit without spilling: 5 for one slot per lane with u8 and
-// u16 values (their eight leaf ids are loaded together), 6 with 4-byte values; the
-// four-slot form's phase-1 loads and phase-2 keys take more registers and its queue more
-// LDS (5 waves for u8 and u16, 3 for 4-byte values).
+// leaf exists.  The rest (mixed bricks; all-same ones whose leaf is missing) are queued in
+// LDS with their loaded data and take phase 2, one per lane, in rounds of TILE: the
+// old-tree descent, the leaves that do not exist yet (leaf_ensure), and brick_work.  Round r of phase 2
+// emits into candidate tile blk*R + r.  The pass is bound by memory latency, so it runs
+// as many waves per SIMD as fit with next to no spilling: 5, but 3 for the four-slot form
+// with 4-byte values (its queue takes more LDS).
 template <typename T, int TILE, int R>
-__global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R == 1 ? (sizeof(T) == 4 ? 6 : 5) : (sizeof(T) == 4 ? 3 : 5), 8))) void k_brick_build(Pool<T> P, ChunkDev* chunks, LevelInfo L,
+__global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && sizeof(T) == 4 ? 3 : 5, 8))) void k_brick_build(Pool<T> P, ChunkDev* chunks, LevelInfo L,
                                                        uint64_t* res1, Cands K, uint32_t* tile_cnt,
-                                                       uint64_t* deferred, Drift* drift,
-                                                       const uint64_t* old2) {
+                                                       Drift* drift, const uint64_t* old2) {
     // a brick's 8 values
     typedef typename std::conditional<sizeof(T) == 1, uint2, typename std::conditional<sizeof(T) == 2, uint4,
                                                                                           Vox8x4>::type>::type Vox8;
     static_assert(sizeof(Vox8) == 8 * sizeof(T), "8 voxels");
-    static_assert(R * TILE <= 32768, "queued brick index is 15 bits (bit 15: all eight values equal)");
-    __shared__ uint32_t s_nq;
+    static_assert(R * TILE <= 0x4000, "queued brick index is 14 bits");
+    constexpr uint32_t kSame = 0x8000u, kMiss = 0x4000u;  // all eight values equal; a leaf is missing
+    __shared__ uint32_t s_nq, s_miss;
     __shared__ uint32_t s_cnt[R];
     __shared__ uint32_t s_st[8];
-    // u8: the leaf id of every value, from LDS (the value map does not change here)
+    // u8: the leaf id of every value, from LDS (loaded past the caches, so that a leaf
+    // created by an earlier block of the launch is seen)
     __shared__ uint64_t s_leaf[sizeof(T) == 1 ? 256 : 1];
     __shared__ uint64_t s_up[R * TILE];
     __shared__ Vox8 s_v[R * TILE];
@@ -968,7 +1033,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R == 1 ? (
     for (uint32_t i = threadIdx.x; i < kSetB; i += TILE) s_kh[i] = 0;
     uint64_t lm[sizeof(T) == 1 ? (256 + TILE - 1) / TILE : 1];
     if (sizeof(T) == 1)
-        for (uint32_t i = 0, v = threadIdx.x; v < 256; i++, v += TILE) lm[i] = P.ctl->leaf_ids8[v];
+        for (uint32_t i = 0, v = threadIdx.x; v < 256; i++, v += TILE) lm[i] = load_agent(&P.leaf_ids[v]);
     const uint64_t b0 = (uint64_t)blockIdx.x * (R * TILE);
     const BlockGroup BG = block_group(L, min(b0, L.nslots - 1), min(b0 + R * TILE, L.nslots) - 1);
     // phase 1 loads, without branches (lanes past the end load the last slot), in two
@@ -1044,7 +1109,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R == 1 ? (
     const uint64_t* leaf_ids = sizeof(T) == 1 ? s_leaf : P.leaf_ids;
     if (threadIdx.x < 8) s_st[threadIdx.x] = 0;
     if (threadIdx.x < R) s_cnt[threadIdx.x] = 0;
-    if (threadIdx.x == 0) s_nq = 0;
+    if (threadIdx.x == 0) s_nq = s_miss = 0;
     __syncthreads();
     uint32_t ncollapse = 0;
     // the leaf of every all-same brick's value, for all R slots before any is used (u8
@@ -1066,6 +1131,16 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R == 1 ? (
             lidj[j] = all_same ? leaf_lookup(P, leaf_ids, v[0]) : kEmpty;
         }
     }
+    // (a leaf may have been created in this launch since this die's cache or, u8, this block
+    // took the table: one more look, past the caches, before such bricks go to phase 2)
+    bool none = false;
+#pragma unroll
+    for (int j = 0; j < R; j++) none = none || (asj[j] && lidj[j] == kEmpty);
+    if (__ballot(none)) {
+#pragma unroll
+        for (int j = 0; j < R; j++)
+            if (asj[j] && lidj[j] == kEmpty) lidj[j] = leaf_now(P, (uint32_t)*(const T*)&vw[j]);
+    }
 #pragma unroll
     for (int j = 0; j < R; j++) {
         const uint64_t slot = b0 + (uint64_t)j * TILE + threadIdx.x;
@@ -1073,7 +1148,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R == 1 ? (
         const bool queue = m[j] != 0 && lid == kEmpty;
         const uint32_t q = wave_append(&s_nq, queue);
         if (queue) {
-            s_idx[q] = (uint16_t)((j * TILE + threadIdx.x) | (asj[j] ? 0x8000u : 0u));
+            s_idx[q] = (uint16_t)((j * TILE + threadIdx.x) | (asj[j] ? kSame : 0u));
             s_m[q] = (uint8_t)m[j];
             s_v[q] = vw[j];
             s_up[q] = up[j];
@@ -1088,18 +1163,22 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R == 1 ? (
     }
     __syncthreads();
     const uint32_t nq = s_nq;
+    // the queue's rounds; bricks that miss a leaf are left out, and once their leaves were
+    // created (by this block or another) they alone are taken by a second pass
+    for (int pass = 0; pass < 2; pass++) {
     for (int r = 0; r < R; r++) {
         if ((uint32_t)r * TILE >= nq) break;  // uniform
         const uint32_t q = (uint32_t)r * TILE + threadIdx.x;
         uint64_t out = kInvalid, slot = 0;
-        bool cand = false, defer = false;
+        bool cand = false, live = q < nq && (pass == 0 || (s_idx[q] & kMiss)), all_same = false;
+        const bool mine = live;
         int flags = 0;
-        uint64_t ch[8];
-        uint32_t tm = 0, c = 0;
-        if (q < nq) {
+        uint64_t ch[8], lids[8], base = kEmpty;
+        uint32_t tm = 0, c = 0, mm = 0, need = 0;
+        if (live) {
             const uint32_t qi = s_idx[q];
-            slot = b0 + (qi & 0x7FFFu);
-            const uint32_t mm = s_m[q];
+            slot = b0 + (qi & (kMiss - 1));
+            mm = s_m[q];
             const Vox8 w = s_v[q];
             const uint64_t upq = s_up[q];
             uint32_t v[8];
@@ -1118,13 +1197,15 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R == 1 ? (
             const uint64_t c_root = C.root_in;
             // (u8 and u16: a table load for every voxel, edited or not, so that the eight
             // are issued together; brick_work reads the leaf ids of edited voxels only)
-            uint64_t lids[8];
             if constexpr (sizeof(T) <= 2) {
 #pragma unroll
                 for (int i = 0; i < 8; i++) lids[i] = leaf_ids[v[i]];
             } else {
 #pragma unroll
-                for (int i = 0; i < 8; i++) lids[i] = (mm >> i) & 1u ? leaf_lookup(P, leaf_ids, v[i]) : kEmpty;
+                for (int i = 0; i < 8; i++) {
+                    lids[i] = kEmpty;
+                    if ((mm >> i) & 1u) lids[i] = pass == 0 ? leaf_lookup(P, leaf_ids, v[i]) : leaf_now(P, v[i]);
+                }
             }
             const bool up_branch = D >= 2 && upq != kEmpty && !bid_is_leaf(upq);
             const bool up_ok = up_branch && bid_index(upq) < P.capacity;
@@ -1133,8 +1214,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R == 1 ? (
             // ids: the compiler would otherwise load each in the branch that needs it,
             // one round trip after the other)
             asm volatile("" ::"v"(below), "v"(c_root), "v"((uint32_t)c_fill));
-            const bool all_same = (qi >> 15) != 0;  // taken in phase 1
-            uint64_t base = kEmpty;
+            all_same = (qi & kSame) != 0;  // taken in phase 1
             bool h1 = false;
             if (!all_same) {
                 if (c_fill) {
@@ -1161,37 +1241,63 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R == 1 ? (
             if (h1) {
                 chunks[c].status = -5;
                 P.ctl->h1_fail = 1u;
+                live = false;
             } else {
-                uint32_t didx = kNoIdx;
-                int32_t dd = 0;
-                int rc;
-                bool lids_all = true;
 #pragma unroll
-                for (int i = 0; i < 8; i++) lids_all = lids_all && lids[i] != kEmpty;
-                if (mm == 0xFFu && !all_same && base != kFillMark && !bid_is_leaf(base) && lids_all) {
-                    // brick_work's result for a completely written brick of distinct values
-                    // over a branch or nothing, whose leaves all exist (the dense case): the
-                    // key is the eight leaves, types = mask = 0xFF.  (Never 8 equal leaves,
-                    // brick_work's H2 case: a live leaf is the one leaf of its value, and
-                    // the values are not all the same.)
+                for (int i = 0; i < 8; i++) need |= (lids[i] == kEmpty ? 1u : 0u) << i;
+                need &= all_same ? 1u : mm;
+            }
+        }
+        // (a leaf created in this launch is seen past the caches)
+        if (__ballot(need != 0)) {
+            if constexpr (sizeof(T) <= 2) {
+                asm volatile("" ::: "memory");  // (the values again from LDS, below too: no registers hold them)
 #pragma unroll
-                    for (int i = 0; i < 8; i++) ch[i] = lids[i];
-                    tm = 0xFFFFu;
-                    rc = 2;
-                } else {
-                    rc = brick_work(P, C, mm, v, base, &out, ch, &tm, &didx, &dd, &flags, lids);
+                for (int i = 0; i < 8; i++)
+                    if ((need >> i) & 1u) {
+                        lids[i] = leaf_now(P, (uint32_t)((const T*)&s_v[q])[i]);
+                        if (lids[i] != kEmpty) need &= ~(1u << i);
+                    }
+            }
+            if (need && !P.dry) {
+                live = false;
+                if (pass == 0) {
+                    s_idx[q] |= kMiss;
+                    s_miss = 1;
                 }
-                if (didx != kNoIdx && !P.dry) {
-                    uint32_t pos = atomicAdd(&P.ctl->n_drift, 1u);
-                    drift[pos] = Drift{c, didx, dd, (uint32_t)(flags & 8 ? ST_H3 : ST_H4)};
-                }
-                if (rc == 2) {
-                    cand = true;
-                    out = res_pending(0xFFFFFFFFu);  // replaced by the probe
-                } else if (rc == 3) {
-                    defer = true;
-                    out = base;  // kept for the retry
-                }
+            }
+        }
+        if (live) {
+            uint32_t didx = kNoIdx;
+            int32_t dd = 0;
+            int rc;
+            bool lids_all = true;
+#pragma unroll
+            for (int i = 0; i < 8; i++) lids_all = lids_all && lids[i] != kEmpty;
+            if (mm == 0xFFu && !all_same && base != kFillMark && !bid_is_leaf(base) && lids_all) {
+                // brick_work's result for a completely written brick of distinct values
+                // over a branch or nothing, whose leaves all exist (the dense case): the
+                // key is the eight leaves, types = mask = 0xFF.  (Never 8 equal leaves,
+                // brick_work's H2 case: a live leaf is the one leaf of its value, and
+                // the values are not all the same.)
+#pragma unroll
+                for (int i = 0; i < 8; i++) ch[i] = lids[i];
+                tm = 0xFFFFu;
+                rc = 2;
+            } else {
+                asm volatile("" ::: "memory");
+                uint32_t v[8];
+                const Vox8 w = s_v[q];
+                load8<T>((const T*)&w, v);
+                rc = brick_work(P, chunks[c], mm, v, base, &out, ch, &tm, &didx, &dd, &flags, lids);
+            }
+            if (didx != kNoIdx && !P.dry) {
+                uint32_t pos = atomicAdd(&P.ctl->n_drift, 1u);
+                drift[pos] = Drift{c, didx, dd, (uint32_t)(flags & 8 ? ST_H3 : ST_H4)};
+            }
+            if (rc == 2) {
+                cand = true;
+                out = res_pending(0xFFFFFFFFu);  // replaced by the probe
             }
         }
         // Equal keys of the block (all rounds, any tree) share one candidate: the leader
@@ -1229,13 +1335,26 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R == 1 ? (
                 write_candidate(K, (uint64_t)tile * TILE + p2, ch, tm, hk, slot);
             }
         }
-        if (q < nq) res1[slot] = out;
-        const uint32_t dpos = wave_append(&P.ctl->n_deferred, defer);
-        if (defer) deferred[dpos] = ((uint64_t)tile << 32) | (uint32_t)slot;
+        if (mine) res1[slot] = out;
         tile_count(s_st, 0, cand);
         tile_count(s_st, 1, (flags & 1) != 0);
         tile_count(s_st, 2, (flags & 4) != 0);
         tile_count(s_st, 3, follow);
+    }
+    __syncthreads();
+    if (!s_miss) break;  // uniform
+    if (pass == 0) {
+        for (uint32_t q0 = 0; q0 < nq; q0 += TILE) {
+            const uint32_t q = q0 + threadIdx.x;
+            uint32_t need = 0;
+            if (q < nq && (s_idx[q] & kMiss)) {
+                const uint32_t mm = s_idx[q] & kSame ? 1u : s_m[q];
+                for (int i = 0; i < 8; i++)
+                    if (((mm >> i) & 1u) && leaf_index(P, (uint32_t)((const T*)&s_v[q])[i]) == 0) need |= 1u << i;
+            }
+            leaf_ensure(P, need, 8, [&](int i) { return (uint32_t)((const T*)&s_v[q])[i]; });
+        }
+    }
     }
     __syncthreads();
     if (threadIdx.x < R) tile_cnt[blockIdx.x * R + threadIdx.x] = s_cnt[threadIdx.x];
@@ -1243,77 +1362,6 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R == 1 ? (
     const int src[6] = {0, 1, 2, 3, 0, 3};
     if (threadIdx.x < 6 && s_st[src[threadIdx.x]])
         atomicAdd((unsigned long long*)stat(P.ctl, ids[threadIdx.x]), (unsigned long long)s_st[src[threadIdx.x]]);
-}
-
-// Bricks that waited for new leaves, and the queued reference-count corrections
-// of trees that did not fail (their status is final now).  A deferred entry is
-// (candidate tile << 32) | slot: the tile of the brick pass's round that queued it.
-template <typename T, int TILE>
-__global__ void k_brick_retry(Pool<T> P, const ChunkDev* chunks, LevelInfo L, uint64_t* res1, Cands K,
-                              uint32_t* tile_cnt, const uint64_t* deferred, const Drift* drift) {
-    mark_owner_base(P);
-    uint32_t nd = P.ctl->n_deferred;
-    VX_LOOP(i, nd) {
-        if (i < nd) {
-            const uint64_t e = deferred[i];
-            const uint64_t slot = (uint32_t)e;
-            const uint64_t tile = e >> 32;
-            const GroupPos G = group_pos(L, slot);
-            uint64_t local = slot - G.base;
-            uint32_t D = G.depth;
-            uint32_t sh = 3 * (D - 1);
-            uint32_t c = G.chunk_base + (uint32_t)(local >> sh);
-            uint32_t p = (uint32_t)(local & ((1ull << sh) - 1));
-            const ChunkDev& C = chunks[c];
-            uint64_t out = kInvalid;
-            if (C.status >= 0) {
-                uint32_t m = C.masks[2ull * p];
-                uint32_t v[8];
-                load8<T>((const T*)C.values + 8ull * p, v);
-                uint64_t ch[8];
-                uint32_t tm = 0, didx;
-                int32_t dd;
-                int flags = 0;
-                // no new requests here: k_leaf_alloc has run, a leaf still missing could
-                // not be allocated and the apply aborts
-                uint64_t lids[8];
-#pragma unroll
-                for (int i = 0; i < 8; i++)
-                    lids[i] = (m >> i) & 1u ? leaf_lookup(P, (const uint64_t*)nullptr, v[i]) : kEmpty;
-                int r = brick_work(P, C, m, v, res1[slot], &out, ch, &tm, &didx, &dd, &flags, lids, false);
-                if (didx != kNoIdx) {
-                    ref_delta_logged(P, c, didx, dd, flags & 8 ? ST_H3 : ST_H4);
-                    atomicAdd((unsigned long long*)stat(P.ctl, flags & 8 ? ST_H3 : ST_H4), 1ull);
-                }
-                if (flags & 1) atomicAdd((unsigned long long*)stat(P.ctl, ST_COLLAPSE), 1ull);
-                if (r == 2) {
-                    uint32_t pos = atomicAdd(&tile_cnt[tile], 1u);
-                    uint64_t k = tile * TILE + pos;
-                    for (int j = 0; j < 8; j++) key_word(K, k, j) = ch[j];
-                    key_word(K, k, 8) = tm;
-                    K.hash[k] = branch_hash(ch, tm);
-                    K.slot[k] = slot;
-                    atomicAdd((unsigned long long*)stat(P.ctl, ST_CAND), 1ull);
-                    atomicAdd((unsigned long long*)stat(P.ctl, ST_CAND1), 1ull);
-                    out = res_pending(0xFFFFFFFFu);
-                } else if (r == 3) {
-                    atomicOr(&P.ctl->abort_, 1u);  // the leaf could not be created
-                    out = kInvalid;
-                }
-            }
-            res1[slot] = out;
-        }
-    }
-    uint32_t ndr = P.ctl->n_drift;
-    VX_LOOP(j, ndr) {
-        if (j < ndr) {
-            Drift d = drift[j];
-            if (chunks[d.chunk].status >= 0) {
-                atomicAdd(&P.refs[d.idx], (uint32_t)d.delta);
-                atomicAdd((unsigned long long*)stat(P.ctl, (int)d.stat), 1ull);
-            }
-        }
-    }
 }
 
 // ------------------------------------------------------------------ interning
@@ -1461,6 +1509,7 @@ __device__ inline int probe_single(const Pool<T>& P, uint32_t level, uint64_t k,
 // The probe's statistics: each wavefront adds its sums to the block's LDS counters as
 // it ends; the last one to end adds them to the global counters.
 constexpr uint32_t kProbeStats = 7;
+constexpr uint32_t kProbeTiles = 16;  // the most tiles of one probe block
 
 template <typename T>
 __device__ inline void probe_stats_flush(const Pool<T>& P, uint32_t h, uint32_t* s_stat, uint32_t* s_done,
@@ -1493,7 +1542,29 @@ __device__ inline void probe_stats_flush(const Pool<T>& P, uint32_t h, uint32_t*
     }
 }
 
-// Probe of the candidates of tiles [t0, t0+tn) of one level (tn <= 64), packed
+// Whether the tree of a brick slot failed in the brick pass (the leaf-brick panic).
+__device__ inline bool brick_tree_failed(const LevelInfo& L, const ChunkDev* chunks, uint64_t slot) {
+    const GroupPos G = group_pos(L, slot);
+    return chunks[G.chunk_base + (uint32_t)((slot - G.base) >> (3 * (G.depth - 1)))].status < 0;
+}
+
+// The candidates of tiles [t0, t0+tn) of the brick level that a brick of a tree which did
+// not fail follows, as a bitmap in LDS (zeroed by the caller).  A follower lies in its
+// leader's block of the brick pass, which took up to four tiles of slots.
+template <int TILE>
+__device__ inline void mark_followed(const LevelInfo& L, const ChunkDev* chunks, const uint64_t* res, uint32_t t0,
+                                     uint32_t tn, uint32_t* s_want) {
+    const uint64_t k0 = (uint64_t)t0 * TILE, k1 = k0 + (uint64_t)tn * TILE;
+    const uint64_t s1 = min((uint64_t)((t0 + tn + 3) / 4 * 4) * TILE, L.nslots);
+    for (uint64_t s = (uint64_t)(t0 / 4 * 4) * TILE + threadIdx.x; s < s1; s += TILE) {
+        const uint64_t r = res[s];
+        const uint64_t k = (uint32_t)r;
+        if (res_is_pending(r) && k >= k0 && k < k1 && !brick_tree_failed(L, chunks, s))
+            atomicOr(&s_want[(k - k0) >> 5], 1u << ((k - k0) & 31u));
+    }
+}
+
+// Probe of the candidates of tiles [t0, t0+tn) of one level (tn <= kProbeTiles), packed
 // densely over the block's lanes: sparse tiles fill whole wavefronts, and equal keys
 // meet in the same pass more often.  Per pass over TILE of them: merge equal keys of
 // the pass through an LDS hash set (dedup_rounds 0 turns the merge off), look the
@@ -1512,6 +1583,7 @@ __device__ inline void probe_tiles(const Pool<T>& P, const Cands& K, const uint3
     constexpr uint32_t kSlots = 2 * TILE;  // the block's key set of one pass (load <= 1/2)
     __shared__ uint32_t s_pre[65];         // s_pre[t]: candidates of the group's tiles before tile t
     __shared__ uint32_t s_own, s_base;
+    __shared__ uint32_t s_want[kProbeTiles * TILE / 32];  // brick level, after a failed tree: mark_followed
     __shared__ uint32_t s_set[kSlots];     // hash slot -> lane + 1 of the key's leader (0: free)
     __shared__ uint64_t s_hash[TILE];      // by lane: the pass's key hash
     __shared__ uint32_t s_cand[TILE];      // ... its candidate index
@@ -1534,7 +1606,9 @@ __device__ inline void probe_tiles(const Pool<T>& P, const Cands& K, const uint3
     Q.levels = s_lv;
     uint32_t n_probes = 0, n_claims = 0, n_lost = 0, n_tomb = 0, n_hit = 0, n_dup = 0, n_miss = 0;
     // the allocation window of the sequence (constant during this launch)
-    const uint32_t ft0 = P.ctl->free_top0, next0 = P.ctl->next0, own_base = P.ctl->own_base;
+    // (branch nodes take the allocation ranks behind the sequence's new leaves)
+    const uint32_t ft0 = P.ctl->free_top0, next0 = P.ctl->next0, nleaves = P.ctl->n_new_leaves;
+    const bool h1 = L.h == 1 && P.ctl->h1_fail != 0;
     if (threadIdx.x < 64) {
         uint32_t x = threadIdx.x < tn ? tile_cnt[t0 + threadIdx.x] : 0u;
 #pragma unroll
@@ -1549,6 +1623,12 @@ __device__ inline void probe_tiles(const Pool<T>& P, const Cands& K, const uint3
         }
     }
     __syncthreads();
+    if (h1) {  // uniform
+        for (uint32_t i = threadIdx.x; i < kProbeTiles * TILE / 32; i += TILE) s_want[i] = 0;
+        __syncthreads();
+        mark_followed<TILE>(L, chunks, res, t0, tn, s_want);
+        __syncthreads();
+    }
     const uint32_t N = s_pre[tn];
     const uint32_t wbase = threadIdx.x & ~63u;
     const int lane = (int)__lane_id();
@@ -1580,9 +1660,15 @@ __device__ inline void probe_tiles(const Pool<T>& P, const Cands& K, const uint3
             for (int i = 0; i < 9; i++) key[i] = key_word(K, k, i);
             h = K.hash[k];
             slot = K.slot[k];
-            // (a key of a tree that hit the leaf-brick panic is interned all the same:
-            // keys merge across trees, so other trees may point at its candidate; the
-            // GC releases the nodes nothing references afterwards)
+            // a key of a tree that hit the leaf-brick panic is interned only for the other
+            // trees whose bricks share its candidate
+            const uint32_t kb = (uint32_t)(k - (uint64_t)t0 * TILE);
+            if (h1 && valid && brick_tree_failed(L, chunks, slot) && !((s_want[kb >> 5] >> (kb & 31u)) & 1u)) {
+                valid = false;
+                K.id[k] = kInvalid;
+                K.tslot[k] = ~0ull;
+                res[slot] = kInvalid;
+            }
             if (P.per_tree) {
                 const GroupPos G = group_pos(L, slot);
                 uint32_t c = G.chunk_base + (uint32_t)((slot - G.base) >> (3 * (G.depth - L.h)));
@@ -1655,10 +1741,10 @@ __device__ inline void probe_tiles(const Pool<T>& P, const Cands& K, const uint3
                 result = make_branch(P.capacity + 65536u + ka, 0, (uint32_t)key[8]);
             } else {
                 bool ok;
-                uint32_t idx = alloc_at(P, ka, &ok, ft0, next0);
+                uint32_t idx = alloc_at(P, nleaves + ka, &ok, ft0, next0);
                 result = ok ? make_branch(idx, tmg_gen(P.tmg[idx]), (uint32_t)key[8]) : kInvalid;
                 if (ok) P.values[idx] = (T)lod;
-                P.owners[ka - own_base] = ((uint64_t)L.h << 32) | k;  // the commit's list
+                P.owners[ka] = ((uint64_t)L.h << 32) | k;  // the commit's list
             }
             if (P.per_tree && tree != kNoIdx) atomicAdd(&P.per_tree[tree], 1u);
         }
@@ -1706,12 +1792,12 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(5, 8))) vo
 
 // Owners write their node (children, types/mask; the probe wrote its LOD value),
 // publish the table slot, and take one reference on each non-empty child.  The owners of an apply are
-// its allocation ranks [own_base, alloc_count) after the last probe (leaves are
-// allocated before own_base), listed by rank as (height << 32) | candidate.  No
+// its allocation ranks after the new leaves, listed as (height << 32) | candidate.  No
 // probe runs during the commit: until it, every new key is a pending table entry,
-// matched against its candidate.  Grid-stride over the owners.
+// matched against its candidate.  Grid-stride over the owners, then over the brick pass's
+// queued reference-count corrections of trees that did not fail (every status is final).
 template <typename T, int TILE>
-__global__ __launch_bounds__(TILE) void k_commit(Pool<T> P) {
+__global__ __launch_bounds__(TILE) void k_commit(Pool<T> P, const ChunkDev* chunks, const Drift* drift) {
     __shared__ uint32_t akey[kAggSlots], acnt[kAggSlots];
     __shared__ uint32_t s_owned;
     // the levels' candidate arrays, from LDS (read once per owner, ahead of its loads)
@@ -1721,7 +1807,7 @@ __global__ __launch_bounds__(TILE) void k_commit(Pool<T> P) {
     if (threadIdx.x < kLevels + 1) s_lv[threadIdx.x] = P.levels[threadIdx.x];
     __syncthreads();
     uint32_t owned = 0;
-    const uint32_t n = P.ctl->alloc_count - P.ctl->own_base;
+    const uint32_t n = P.ctl->alloc_count, ndrift = P.ctl->n_drift;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const uint64_t e = P.owners[i];
         const Cands& K = s_lv[e >> 32];
@@ -1750,6 +1836,13 @@ __global__ __launch_bounds__(TILE) void k_commit(Pool<T> P) {
             if (!agg_add(akey, acnt, ci, 1u)) atomicAdd(&P.refs[ci], 1u);
         }
     }
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < ndrift; i += gridDim.x * blockDim.x) {
+        const Drift d = drift[i];
+        if (chunks[d.chunk].status >= 0) {
+            atomicAdd(&P.refs[d.idx], (uint32_t)d.delta);
+            atomicAdd((unsigned long long*)stat(P.ctl, (int)d.stat), 1ull);
+        }
+    }
     // the block's owners go to the live count with one update (a counter every block
     // of the launch updates is a serial point)
     const uint32_t wo = wave_sum(owned);
@@ -1759,13 +1852,6 @@ __global__ __launch_bounds__(TILE) void k_commit(Pool<T> P) {
         if (akey[i] != kNoIdx && acnt[i]) atomicAdd(&P.refs[akey[i]], acnt[i]);
     if (threadIdx.x == 0 && s_owned)
         atomicAdd((unsigned long long*)&P.ctl->live_branches, (unsigned long long)s_owned);
-}
-
-// The first allocation rank of the apply's probes (the owners' list base), set by a
-// pass that runs after the leaf allocation and before the first probe.
-template <typename T>
-__device__ inline void mark_owner_base(const Pool<T>& P) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) P.ctl->own_base = P.ctl->alloc_count;
 }
 
 // A pending result names a candidate of the level; that candidate's id is final, or
@@ -2020,10 +2106,14 @@ __device__ inline void rollback_body(const Pool<T>& P, const ChunkDev* chunks, c
         }
     }
     if (!abort) return;
+    // new leaves leave the value map
+    const uint32_t nl = (uint32_t)alloc_done(P, P.ctl->n_new_leaves);
+    for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < nl; j += gridDim.x * blockDim.x)
+        leaf_remove(P, (uint32_t)P.values[P.new_leaves[j]]);
     uint32_t nu = P.ctl->n_undo < P.undo_cap ? P.ctl->n_undo : P.undo_cap;
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < nu; j += gridDim.x * blockDim.x)
         atomicSub(&P.refs[P.undo[j].idx], (uint32_t)P.undo[j].delta);
-    // queued corrections applied by k_brick_retry (trees whose status was final)
+    // queued corrections applied by the commit (trees that did not fail)
     uint32_t ndr = P.ctl->n_drift;
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < ndr; j += gridDim.x * blockDim.x) {
         Drift d = drift[j];
@@ -2265,7 +2355,7 @@ __global__ __launch_bounds__(256) void k_gc_round(Pool<T> P, uint32_t round, con
         hi = min(n, lo + share);
     }
     // a block past the frontier has nothing to do (the rounds near the leaves hold few
-    // nodes); the first round also releases new leaves and orphans with every block
+    // nodes); the first round also releases new leaves with every block
     if (!leaf_cleanup && (local ? lo >= hi : (uint64_t)blockIdx.x * blockDim.x >= n)) return;
     agg_init(akey, acnt);
     if (threadIdx.x == 0) {
@@ -2277,28 +2367,6 @@ __global__ __launch_bounds__(256) void k_gc_round(Pool<T> P, uint32_t round, con
     // round; no node that this GC visits references them
     if (leaf_cleanup) leaf_cleanup_body(P);
     uint32_t* next_count = &P.ctl->gc_count[round + 1];
-    // New branch nodes that nothing references go to the next round: keys of a tree that
-    // failed in the brick pass (the leaf-brick panic) are interned like every key, and
-    // the ones no other tree shares end up without a reference.  Every other new node
-    // holds one from its parent or its tree (the commit and the root swap ran).
-    if (leaf_cleanup && P.ctl->h1_fail) {
-        const uint32_t no = P.ctl->n_owners;
-        VX_LOOP(i, no) {
-            uint32_t idx = kNoIdx;
-            if (i < no) {
-                const uint64_t e = P.owners[i];
-                const Cands& K = P.levels[e >> 32];
-                const uint64_t id = K.id[(uint32_t)e];
-                if (K.tslot[(uint32_t)e] != ~0ull && id != kInvalid && P.refs[bid_index(id)] == 0u)
-                    idx = bid_index(id);
-            }
-            const uint32_t pos = wave_append(next_count, idx != kNoIdx);
-            if (idx != kNoIdx) {
-                if (pos < front_cap) next[pos] = idx;
-                else atomicOr(&P.ctl->err, kErrPoison);
-            }
-        }
-    }
     const int lane = (int)__lane_id();
     const uint64_t below = (1ull << lane) - 1ull;
     if (local) {
@@ -2479,8 +2547,11 @@ __global__ void k_tab_clear(uint64_t* tab, uint64_t nslots, Ctl* ctl, uint64_t l
         t4[i] = make_uint4(0u, 0u, 0u, 0u);
 }
 
+// The control block's reset for the call that follows rides in block 0 (the other blocks
+// read nothing that it writes).
 template <typename T>
 __global__ void k_tab_reinsert(Pool<T> P) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctl_begin(P.ctl);
     if (!(P.ctl->rebuild & 1u)) return;
     // the cleared table holds no tombstone (no other block reads the counter here)
     if (blockIdx.x == 0 && threadIdx.x < kStatStripes) P.ctl->st[threadIdx.x][ST_TOMB] = 0;
@@ -2548,8 +2619,6 @@ constexpr uint32_t kSetRec = 2 * kLevels;
 template <typename T>
 __global__ void k_set_descend(Pool<T> P, ChunkDev* chunks, uint32_t n, const uint64_t* roots, const int32_t* xyz,
                               const T* vals, uint64_t* rec, uint32_t* meta) {
-    // the sequence's control-block reset rides in block 0 (nothing else here reads it)
-    if (blockIdx.x == 0 && threadIdx.x == 0) ctl_begin(P.ctl);
     VX_LOOP(c, n) {
         if (c < n) {
             ChunkDev& C = chunks[c];
@@ -2596,7 +2665,8 @@ __global__ void k_set_descend(Pool<T> P, ChunkDev* chunks, uint32_t n, const uin
                     cur = kEmpty;
                 }
                 if (!unchanged && bid_is_leaf(cur) && (uint32_t)P.values[bid_index(cur)] == v) unchanged = true;
-                if (!unchanged && leaf_index(P, v) == 0) leaf_request(P, v);
+                // (a leaf that cannot be allocated aborts the call)
+                if (!unchanged && leaf_index(P, v) == 0) leaf_acquire(P, v);
             } else if (!unchanged) {
                 // voxtree.rs:581-660: present children are followed down to a leaf (split
                 // from there, or the voxel itself at depth D); a missing child changes nothing
@@ -2635,7 +2705,6 @@ __global__ __launch_bounds__(TILE) void k_set_level(
     Pool<T> P, const ChunkDev* chunks, LevelInfo L, const uint64_t* doff, uint32_t n, const int32_t* xyz,
     const T* vals, const uint64_t* rec, const uint32_t* meta, const uint64_t* res_prev,
     const uint64_t* cand_id_prev, uint64_t* res, Cands K, uint32_t* tile_cnt) {
-    if (L.h == 1) mark_owner_base(P);
     __shared__ uint32_t s_cnt;
     __shared__ uint32_t s_st[8];
     if (threadIdx.x < 8) s_st[threadIdx.x] = 0;
@@ -2748,17 +2817,13 @@ __global__ __launch_bounds__(TILE) void k_set_level(
 // VoxOpsBulkWrite::fill/clear (voxtree.rs:263-292): queue the old root for
 // dec_ref_recursive first, then (after GC and leaf creation) install leaf(v).
 template <typename T>
-__global__ void k_fill_prepare(Pool<T> P, uint32_t n, const uint64_t* roots, const uint64_t* vals,
-                               uint32_t* gc_front) {
-    const uint32_t vmask = sizeof(T) == 1 ? 0xFFu : sizeof(T) == 2 ? 0xFFFFu : 0xFFFFFFFFu;
+__global__ void k_fill_prepare(Pool<T> P, uint32_t n, const uint64_t* roots, uint32_t* gc_front) {
     VX_LOOP(c, n) {
         bool push = false;
         uint64_t r = kEmpty;
         if (c < n) {
             r = roots[c];
             push = r != kEmpty;
-            uint32_t v = (uint32_t)vals[c] & vmask;
-            if (v != 0 && leaf_index(P, v) == 0) leaf_request(P, v);
         }
         uint32_t k = wave_append(&P.ctl->gc_count[0], push);
         if (push) gc_front[k] = bid_index(r);
@@ -2774,24 +2839,17 @@ __global__ void k_fill_finish(Pool<T> P, uint32_t n, uint64_t* roots, const uint
             if (v == 0) {
                 roots[c] = kEmpty;
             } else {
-                uint32_t idx = leaf_index(P, v);
-                if (idx != 0) {
-                    atomicAdd(&P.refs[idx], 1u);
-                    roots[c] = make_leaf(idx, tmg_gen(P.tmg[idx]));
+                const uint32_t idx = leaf_index(P, v);
+                const uint64_t id = idx ? make_leaf(idx, tmg_gen(P.tmg[idx])) : leaf_acquire(P, v);
+                if (id != kEmpty) {
+                    atomicAdd(&P.refs[bid_index(id)], 1u);
+                    roots[c] = id;
+                } else {
+                    // the old roots were released first: there is no state to return to
+                    atomicOr(&P.ctl->err, kErrOom | kErrPoison);
                 }
             }
         }
-    }
-}
-
-template <typename T>
-__global__ void k_leaf_alloc_only(Pool<T> P, uint32_t nvalues) {
-    const uint32_t created = create_requested_leaves(P, nvalues);
-    if (threadIdx.x == 0) {
-        // fill released the old roots first: there is no state to return to
-        if (P.ctl->abort_) atomicOr(&P.ctl->err, kErrOom | kErrPoison);
-        atomicAdd((unsigned long long*)&P.ctl->live_leaves, (unsigned long long)created);
-        atomicAdd((unsigned long long*)stat(P.ctl, ST_LEAF_MISS), (unsigned long long)created);
     }
 }
 
