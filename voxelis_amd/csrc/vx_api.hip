@@ -92,18 +92,14 @@ struct LevelBufs {
 
 // Kernel ids of the per-kernel timer (vx_interner_profile_*).
 enum KernelId : uint32_t {
-    KID_BEGIN = 0, KID_PREPARE, KID_UNUSED0, KID_DRY_LEAVES, KID_BRICK_BUILD, KID_PROBE_BRICKS,
-    KID_UNUSED, KID_LEVEL_BUILD, KID_PROBE_UPPER, KID_COMMIT, KID_FINALIZE,
-    KID_END_ALLOC, KID_LEAF_CLEANUP, KID_GC, KID_GET, KID_CANON, KID_FILL, KID_ROLLBACK, KID_TO_VEC,
-    KID_SET_DESCEND, KID_SET_LEVEL, KID_GET_GROUPED, KID_EDIT_KEYS, KID_SORT_HIST, KID_SORT_SCAN,
-    KID_SORT_SCATTER, KID_EDIT_SCATTER, KID_COUNT
+    KID_BEGIN = 0, KID_PREPARE, KID_DRY_LEAVES, KID_BRICK_BUILD, KID_PROBE_BRICKS, KID_LEVEL_BUILD, KID_PROBE_UPPER,
+    KID_COMMIT, KID_END_ALLOC, KID_GC, KID_GET, KID_CANON, KID_FILL, KID_TO_VEC, KID_SET_DESCEND, KID_SET_LEVEL,
+    KID_GET_GROUPED, KID_EDIT_KEYS, KID_SORT_HIST, KID_SORT_SCAN, KID_SORT_SCATTER, KID_EDIT_SCATTER, KID_COUNT
 };
 const char* const kKernelNames[KID_COUNT] = {
-    "k_begin", "k_prepare", "", "k_dry_leaves", "k_brick_build", "k_probe[bricks]",
-    "", "k_level_build", "k_probe[upper]", "k_commit", "k_finish",
-    "k_end_alloc", "k_leaf_cleanup", "k_gc_round", "k_get", "k_canon", "k_fill", "k_rollback", "k_to_vec",
-    "k_set_descend", "k_set_level", "k_get_grouped", "k_edit_keys", "k_sort_hist", "k_sort_scan",
-    "k_sort_scatter", "k_edit_scatter"};
+    "k_begin", "k_prepare", "k_dry_leaves", "k_brick_build", "k_probe[bricks]", "k_level_build", "k_probe[upper]",
+    "k_commit", "k_end_alloc", "k_gc_round", "k_get", "k_canon", "k_fill", "k_to_vec", "k_set_descend", "k_set_level",
+    "k_get_grouped", "k_edit_keys", "k_sort_hist", "k_sort_scan", "k_sort_scatter", "k_edit_scatter"};
 
 struct Prof {
     bool on = false;
@@ -298,8 +294,9 @@ struct ApplyOpts {
     const void* set_values = nullptr;
 };
 
+constexpr unsigned kRebuildGrid = 512;
 template <typename T>
-int rebuild_step(vx_interner* h, bool force);
+int rebuild_step(vx_interner* h, bool force, bool reinsert);
 
 template <typename T, int TILE>
 int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* batches,
@@ -535,12 +532,13 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
         drec = (uint64_t*)h->set_rec.ptr;
         dmeta = (uint32_t*)h->set_meta.ptr;
     }
+    // u8/u16: blocks of the first kernel that re-insert into the pattern table when it is due
+    const unsigned nre = !opt.dry && !h->ltab ? kRebuildGrid : 0u;
     auto launch_set = [&]() -> int {
     const int32_t* sx = opt.set_xyz;
     const T* sv = (const T*)opt.set_values;
-    VX_LAUNCH(h, KID_SET_DESCEND, k_set_descend<T>, grid_for(n), kBlock, P, dchunks, (uint32_t)n, roots, sx, sv,
-              drec, dmeta);
-    const unsigned wpb = TILE / 64;
+    VX_LAUNCH(h, KID_SET_DESCEND, k_set_descend<T>, grid_for(n) + nre, kBlock, P, dchunks, (uint32_t)n, roots, sx, sv,
+              drec, dmeta, grid_for(n));
     for (uint32_t hh = 1; hh <= dmax; hh++) {
         unsigned th = (unsigned)ntiles[hh];
         VX_LAUNCH(h, KID_SET_LEVEL, k_set_level<T VX_COMMA TILE>, th, TILE, P, dchunks, L[hh], doff,
@@ -550,14 +548,11 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
         VX_LAUNCH(h, KID_PROBE_UPPER, k_probe<T VX_COMMA TILE>, (th + gh - 1) / gh, TILE, P, K[hh], tiles_h[hh],
                   res_ptrs_h[hh], dchunks, L[hh], th, gh);
     }
-    (void)wpb;
-    if (!opt.dry && dmax >= 1)
-        VX_LAUNCH(h, KID_COMMIT, k_commit<T VX_COMMA TILE>, h->tune.commit_grid, TILE, P, dchunks, ddrift);
     return hipGetLastError() == hipSuccess ? VX_OK : VX_E_HIP;
     };
     auto launch_all = [&]() -> int {
     if (!opt.dry) {
-        int rc = rebuild_step<T>(h, false);
+        int rc = rebuild_step<T>(h, false, nre == 0);
         if (rc) return rc;
     }
     if (setm) {
@@ -567,7 +562,7 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     // chunk set-up, plus the old-tree descent over the level-3 slots in extra blocks
     unsigned np = grid_for(n);
     unsigned nd = L[3].nslots ? grid_for(L[3].nslots) : 0u;
-    VX_LAUNCH(h, KID_PREPARE, k_prepare<T>, np + nd, kBlock, P, dchunks, (uint32_t)n, roots, pre_status, np,
+    VX_LAUNCH(h, KID_PREPARE, k_prepare<T>, np + nd + nre, kBlock, P, dchunks, (uint32_t)n, roots, pre_status, np,
               nd, L[3], doff, O);
     unsigned t1 = (unsigned)ntiles[1];
     if (dmax >= 2 && br == kBR)
@@ -592,19 +587,15 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
             VX_LAUNCH(h, KID_PROBE_UPPER, k_probe<T VX_COMMA TILE>, (th + gh - 1) / gh, TILE, P, K[hh], tiles_h[hh],
                       res_ptrs_h[hh], dchunks, L[hh], th, gh);
         }
-        // every level's new nodes, written once no probe runs any more
-        if (!opt.dry) VX_LAUNCH(h, KID_COMMIT, k_commit<T VX_COMMA TILE>, h->tune.commit_grid, TILE, P, dchunks, ddrift);
     }
     }
     uint32_t* gf0 = (uint32_t*)h->gc_front[0].ptr;
     uint32_t* gf1 = (uint32_t*)h->gc_front[1].ptr;
-    // the rollback (dry runs restore the table; an aborted apply takes its references
-    // back) and the root swap
-    unsigned rg = (unsigned)std::min<uint64_t>(std::max<uint64_t>(LT.start[LT.dmax + 1], 1), 1024);
-    unsigned fg = std::max(rg, (unsigned)((n + TILE - 1) / TILE));
-    VX_LAUNCH(h, KID_FINALIZE, k_finish<T VX_COMMA TILE>, std::min(fg, 65535u), TILE, P, dchunks, LT, ddrift,
-              (uint32_t)n, doff, (uint32_t)n, dres, dcid, roots, status, gf0);
-    VX_LAUNCH(h, KID_END_ALLOC, k_end_alloc<T>, 1, 256, P, true, opt.counts);
+    // every level's new nodes, written once no probe runs any more, and the root swap: a
+    // lane per possible owner (a slot of some level) and per tree, up to the commit grid
+    const uint64_t cg = std::max<uint64_t>(LT.start[LT.dmax + 1], (n + TILE - 1) / TILE);
+    VX_LAUNCH(h, KID_COMMIT, k_commit<T VX_COMMA TILE>, (unsigned)std::min<uint64_t>(std::max<uint64_t>(cg, 1), h->tune.commit_grid),
+              TILE, P, dchunks, ddrift, LT, (uint32_t)n, doff, (uint32_t)n, dres, dcid, roots, status, gf0, opt.counts);
     if (!opt.dry) {
         // dec_ref_recursive of the replaced roots: a tree of depth D has nodes at
         // heights D..0, one round each; the first round also releases unused new leaves.
@@ -657,20 +648,16 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
 
 // The table-rebuild step that starts every write call (enqueued on the interner's
 // stream, captured with the call's launch sequence): the device decides whether the
-// pattern table (and the i32 leaf table) is rebuilt now, and the clear and re-insert
-// kernels do it or return at once.  force: rebuild regardless.
-constexpr unsigned kRebuildGrid = 512;
+// pattern table (and the i32 leaf table) is rebuilt now, and clears it; the re-insertion is
+// a launch of its own (reinsert) or rides in the call's next kernel.  force: rebuild
+// regardless.
 template <typename T>
-int rebuild_step(vx_interner* h, bool force) {
+int rebuild_step(vx_interner* h, bool force, bool reinsert) {
     Pool<T> P = pool_of<T>(h);
     hipStream_t s = h->stream;
-    k_tab_clear<<<kRebuildGrid, kBlock, 0, s>>>(h->tab, h->tslots, h->ctl, h->ltab ? h->lslots : 0ull,
+    k_tab_clear<<<kRebuildGrid, kBlock, 0, s>>>(h->tab, h->tslots, h->ctl, h->ltab, h->ltab ? h->lslots : 0ull,
                                                 force ? 1u : 0u);
-    k_tab_reinsert<T><<<kRebuildGrid, kBlock, 0, s>>>(P);
-    if (h->ltab) {
-        k_ltab_clear<<<kRebuildGrid, kBlock, 0, s>>>(h->ltab, h->lslots, h->ctl);
-        k_ltab_reinsert<T><<<kRebuildGrid, kBlock, 0, s>>>(P);
-    }
+    if (reinsert) k_tab_reinsert<T><<<kRebuildGrid, kBlock, 0, s>>>(P);
     return hipGetLastError() == hipSuccess ? VX_OK : VX_E_HIP;
 }
 
@@ -798,14 +785,13 @@ int apply_edits_impl(vx_interner* h, size_t n, uint64_t* roots, const uint8_t* d
 
 template <typename T>
 int fill_impl(vx_interner* h, size_t n, uint64_t* roots, const uint64_t* vals) {
-    int rc = rebuild_step<T>(h, false);
+    int rc = rebuild_step<T>(h, false, true);
     if (rc) return rc;
     Pool<T> P = pool_of<T>(h);
     size_t gcap = (size_t)h->capacity + n + 16;
     if (!h->gc_front[0].ensure(gcap * 4) || !h->gc_front[1].ensure(gcap * 4)) return VX_E_HIP;
     uint32_t* gf0 = (uint32_t*)h->gc_front[0].ptr;
     uint32_t* gf1 = (uint32_t*)h->gc_front[1].ptr;
-    VX_LAUNCH(h, KID_BEGIN, k_begin, 1, 1, h->ctl);
     VX_LAUNCH(h, KID_FILL, k_fill_prepare<T>, grid_for(n), kBlock, P, (uint32_t)n, roots, gf0);
     for (uint32_t r = 0; r < (uint32_t)kLevels + 1; r++) {
         uint32_t* fr = (r & 1) ? gf1 : gf0;
@@ -816,7 +802,7 @@ int fill_impl(vx_interner* h, size_t n, uint64_t* roots, const uint64_t* vals) {
     }
     VX_LAUNCH(h, KID_BEGIN, k_begin, 1, 1, h->ctl);
     VX_LAUNCH(h, KID_FILL, k_fill_finish<T>, grid_for(n), kBlock, P, (uint32_t)n, roots, vals);
-    VX_LAUNCH(h, KID_END_ALLOC, k_end_alloc<T>, 1, 256, P, false, (uint32_t*)nullptr);
+    VX_LAUNCH(h, KID_END_ALLOC, k_end_alloc<T>, 1, 1, P);
     return hipGetLastError() == hipSuccess ? VX_OK : VX_E_HIP;
 }
 
@@ -1278,7 +1264,7 @@ int vx_interner_get_tuning(const vx_interner* h, vx_tuning* t) {
 int vx_interner_rebuild_table(vx_interner* h, uint64_t* rebuilds) {
     if (!h) return VX_E_INVALID_ARG;
     if (h->poisoned) return VX_E_POISONED;
-    int rc = VX_WIDTH_DISPATCH(h, rebuild_step, h, true);
+    int rc = VX_WIDTH_DISPATCH(h, rebuild_step, h, true, true);
     if (rc) return rc;
     Ctl c;
     rc = sync_read_ctl(h, &c);

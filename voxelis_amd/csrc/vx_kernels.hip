@@ -649,46 +649,30 @@ __global__ void k_dry_leaves(Pool<T> P) {
     }
 }
 
-// Close the allocation window of a launch sequence.  An aborted apply
-// (rollback = true) gives every allocation back instead: the allocator cursors
-// stay and reference counts of the taken indices go back to zero (the rollback took the
-// new leaves off the value map).  counts (optional): new branches, new leaves.
+// Close the allocation window of a launch sequence (one thread, once every allocation was
+// made).  An aborted apply's allocator cursors stay: its allocations are given back.  Only
+// fields that no kernel reads before the next sequence's ctl_begin, or that other lanes do
+// not read meanwhile, are written.  counts (optional): new branches, new leaves.
 template <typename T>
-__global__ void k_end_alloc(Pool<T> P, bool rollback, uint32_t* counts) {
+__device__ inline void close_allocation(const Pool<T>& P, bool abort, uint32_t* counts) {
     Ctl* ctl = P.ctl;
-    const uint32_t n = ctl->n_new_leaves + ctl->alloc_count;
-    const bool abort = rollback && !P.dry && ctl->abort_ != 0;
     if (abort) {
-        uint32_t ft0 = ctl->free_top0;
-        const uint64_t nok = alloc_done(P, n);
-        for (uint64_t i = threadIdx.x; i < nok; i += blockDim.x) {
-            uint32_t idx = i < ft0 ? P.free_stack[ft0 - 1 - i] : (uint32_t)(ctl->next0 + (i - ft0));
-            P.refs[idx] = 0;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            ctl->n_new_leaves = 0;
-            ctl->alloc_count = 0;
-            if (counts) counts[0] = counts[1] = 0xFFFFFFFFu;
-        }
+        if (counts) counts[0] = counts[1] = 0xFFFFFFFFu;
         return;
     }
-    if (threadIdx.x == 0) {
-        if (counts) {
-            counts[0] = P.dry ? ctl->dry_owners : ctl->alloc_count;
-            counts[1] = P.dry ? ctl->dry_new_leaves : ctl->n_new_leaves;
-        }
-        const uint64_t made = alloc_done(P, ctl->n_new_leaves);
-        ctl->live_leaves += made;
-        *stat(ctl, ST_LEAF_MISS) += made;
-        uint32_t used_free = n < ctl->free_top0 ? n : ctl->free_top0;
-        ctl->free_top = ctl->free_top0 - used_free;
-        uint64_t nx = (uint64_t)ctl->next0 + (n - used_free);
-        ctl->next_index = (uint32_t)(nx > 0xFFFFFFFFull ? 0xFFFFFFFFull : nx);
-        ctl->free_top0 = ctl->free_top;
-        ctl->next0 = ctl->next_index;
-        ctl->alloc_count = 0;
+    if (counts) {
+        counts[0] = P.dry ? ctl->dry_owners : ctl->alloc_count;
+        counts[1] = P.dry ? ctl->dry_new_leaves : ctl->n_new_leaves;
     }
+    const uint64_t made = alloc_done(P, ctl->n_new_leaves);
+    ctl->live_leaves += made;
+    ctl->live_branches += ctl->alloc_count;
+    *stat(ctl, ST_LEAF_MISS) += made;
+    const uint32_t n = ctl->n_new_leaves + ctl->alloc_count;
+    const uint32_t used_free = n < ctl->free_top0 ? n : ctl->free_top0;
+    ctl->free_top = ctl->free_top0 - used_free;
+    const uint64_t nx = (uint64_t)ctl->next0 + (n - used_free);
+    ctl->next_index = (uint32_t)(nx > 0xFFFFFFFFull ? 0xFFFFFFFFull : nx);
 }
 
 // The previous tree's nodes on the path to one height-3 position (level-3 slot
@@ -735,13 +719,52 @@ __device__ inline void descend_body(const Pool<T>& P, const ChunkDev* chunks, co
     for (int i = 0; i < 8; i++) dst[i] = below[i];
 }
 
+// Re-insertion of every live branch into the cleared pattern table by blocks b of nb, when
+// this call's k_tab_clear found it due; and, i32, of every live leaf (a node without a
+// types/mask word that holds a reference) into the hashed leaf table.
+template <typename T>
+__device__ inline void reinsert_body(const Pool<T>& P, uint32_t b, uint32_t nb) {
+    if (!(P.ctl->rebuild & 1u)) return;
+    // the cleared tables hold no tombstone (no other block reads the counters here)
+    if (b == 0 && threadIdx.x < kStatStripes) {
+        P.ctl->st[threadIdx.x][ST_TOMB] = 0;
+        P.ctl->st[threadIdx.x][ST_LTOMB] = 0;
+    }
+    const uint32_t top = P.ctl->next_index;
+    for (uint32_t i = b * blockDim.x + threadIdx.x; i < top; i += nb * blockDim.x) {
+        const uint32_t tm = tmg_tm(P.tmg[i]);
+        if (i == 0) continue;
+        if (tm == 0) {
+            if (sizeof(T) == 4 && P.refs[i] != 0) leaf_publish(P, (uint32_t)P.values[i], i);
+            continue;
+        }
+        uint64_t ch[8];
+        const uint64_t* src = P.children + 8ull * i;
+#pragma unroll
+        for (int j = 0; j < 8; j++) ch[j] = src[j];
+        if (P.single && tm_is_single(tm)) continue;  // in the one-leaf index, which has no tombstones
+        const uint64_t h = branch_hash(ch, tm);
+        const uint64_t want = slot_make(slot_tag(h), false, 0, i);
+        uint64_t s = h & P.tmask;
+        for (uint64_t guard = 0; guard <= P.tmask; guard++) {
+            if (atomicCAS((unsigned long long*)&P.tab[s], 0ull, (unsigned long long)want) == 0ull) break;
+            s = (s + 1) & P.tmask;
+        }
+    }
+}
+
 // Read roots and take the fill leaf (Phase 0, voxtree.rs:742-754): a tree with a fill
 // starts from it, and the fill leaf of a batch that also has patches keeps its reference
-// (H3).  Blocks nprep..nprep+ndesc run the old-tree descent over the level-3 slots instead.
+// (H3).  Blocks nprep..nprep+ndesc run the old-tree descent over the level-3 slots instead,
+// the blocks after them the table's re-insertion when it is due (nothing here reads it).
 template <typename T>
 __global__ void k_prepare(Pool<T> P, ChunkDev* chunks, uint32_t n, const uint64_t* roots,
                           const int32_t* pre_status, uint32_t nprep, uint32_t ndesc, LevelInfo L3,
                           const uint64_t* doff, OldNodes O) {
+    if (blockIdx.x >= nprep + ndesc) {
+        reinsert_body(P, blockIdx.x - nprep - ndesc, gridDim.x - nprep - ndesc);
+        return;
+    }
     if (blockIdx.x >= nprep) {
         uint64_t stride = (uint64_t)ndesc * blockDim.x;
         for (uint64_t s = (uint64_t)(blockIdx.x - nprep) * blockDim.x + threadIdx.x; s < L3.nslots; s += stride)
@@ -1796,45 +1819,44 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(5, 8))) vo
 // probe runs during the commit: until it, every new key is a pending table entry,
 // matched against its candidate.  Grid-stride over the owners, then over the brick pass's
 // queued reference-count corrections of trees that did not fail (every status is final).
-template <typename T, int TILE>
-__global__ __launch_bounds__(TILE) void k_commit(Pool<T> P, const ChunkDev* chunks, const Drift* drift) {
+template <typename T>
+__device__ inline void commit_body(const Pool<T>& P, const ChunkDev* chunks, const Drift* drift) {
     __shared__ uint32_t akey[kAggSlots], acnt[kAggSlots];
-    __shared__ uint32_t s_owned;
     // the levels' candidate arrays, from LDS (read once per owner, ahead of its loads)
     __shared__ Cands s_lv[kLevels + 1];
-    agg_init(akey, acnt);
-    if (threadIdx.x == 0) s_owned = 0;
-    if (threadIdx.x < kLevels + 1) s_lv[threadIdx.x] = P.levels[threadIdx.x];
-    __syncthreads();
-    uint32_t owned = 0;
     const uint32_t n = P.ctl->alloc_count, ndrift = P.ctl->n_drift;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const uint64_t e = P.owners[i];
-        const Cands& K = s_lv[e >> 32];
-        const uint64_t k = (uint32_t)e;
-        // the owner's record in one round of loads: the slot and id decide whether it is
-        // written, the key and hash are what it writes
-        const uint64_t ts = K.tslot[k];
-        const uint64_t id = K.id[k];
-        uint64_t key[9];
+    if (blockIdx.x * blockDim.x < n) {  // uniform over the block
+        agg_init(akey, acnt);
+        if (threadIdx.x < kLevels + 1) s_lv[threadIdx.x] = P.levels[threadIdx.x];
+        __syncthreads();
+        for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+            const uint64_t e = P.owners[i];
+            const Cands& K = s_lv[e >> 32];
+            const uint64_t k = (uint32_t)e;
+            // the owner's record in one round of loads
+            const uint64_t ts = K.tslot[k];
+            const uint64_t id = K.id[k];
+            uint64_t key[9];
 #pragma unroll
-        for (int j = 0; j < 9; j++) key[j] = key_word(K, k, j);
-        const uint64_t hk = K.hash[k];
-        asm volatile("" ::"v"(hk));  // (loaded with the rest, not after the slot test)
-        if (ts == ~0ull || id == kInvalid) continue;  // its allocation failed
-        owned++;
-        uint32_t idx = bid_index(id);
-        uint64_t* dst = P.children + 8ull * idx;
+            for (int j = 0; j < 9; j++) key[j] = key_word(K, k, j);
+            const uint64_t hk = K.hash[k];
+            asm volatile("" ::"v"(hk));  // (loaded with the rest, not where it is used)
+            uint32_t idx = bid_index(id);
+            uint64_t* dst = P.children + 8ull * idx;
 #pragma unroll
-        for (int j = 0; j < 8; j++) dst[j] = key[j];
-        P.tmg[idx] = tmg_make((uint32_t)key[8], bid_gen(id));
-        if (ts & kTslotSingle) P.single[tslot_index(ts)] = id;
-        else P.tab[tslot_index(ts)] = slot_make(slot_tag(hk), false, 0, idx);
-        for (int j = 0; j < 8; j++) {
-            if (key[j] == kEmpty) continue;
-            uint32_t ci = bid_index(key[j]);
-            if (!agg_add(akey, acnt, ci, 1u)) atomicAdd(&P.refs[ci], 1u);
+            for (int j = 0; j < 8; j++) dst[j] = key[j];
+            P.tmg[idx] = tmg_make((uint32_t)key[8], bid_gen(id));
+            if (ts & kTslotSingle) P.single[tslot_index(ts)] = id;
+            else P.tab[tslot_index(ts)] = slot_make(slot_tag(hk), false, 0, idx);
+            for (int j = 0; j < 8; j++) {
+                if (key[j] == kEmpty) continue;
+                uint32_t ci = bid_index(key[j]);
+                if (!agg_add(akey, acnt, ci, 1u)) atomicAdd(&P.refs[ci], 1u);
+            }
         }
+        __syncthreads();
+        for (int i = threadIdx.x; i < kAggSlots; i += blockDim.x)
+            if (akey[i] != kNoIdx && acnt[i]) atomicAdd(&P.refs[akey[i]], acnt[i]);
     }
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < ndrift; i += gridDim.x * blockDim.x) {
         const Drift d = drift[i];
@@ -1843,15 +1865,6 @@ __global__ __launch_bounds__(TILE) void k_commit(Pool<T> P, const ChunkDev* chun
             atomicAdd((unsigned long long*)stat(P.ctl, (int)d.stat), 1ull);
         }
     }
-    // the block's owners go to the live count with one update (a counter every block
-    // of the launch updates is a serial point)
-    const uint32_t wo = wave_sum(owned);
-    if (__lane_id() == 0 && wo) atomicAdd(&s_owned, wo);
-    __syncthreads();
-    for (int i = threadIdx.x; i < kAggSlots; i += blockDim.x)
-        if (akey[i] != kNoIdx && acnt[i]) atomicAdd(&P.refs[akey[i]], acnt[i]);
-    if (threadIdx.x == 0 && s_owned)
-        atomicAdd((unsigned long long*)&P.ctl->live_branches, (unsigned long long)s_owned);
 }
 
 // A pending result names a candidate of the level; that candidate's id is final, or
@@ -2073,16 +2086,12 @@ struct LevelTiles {
     uint32_t dmax;
 };
 
-// After the last commit: a dry run restores the table slots its owners claimed;
-// an apply that could not allocate (abort_) also takes back every reference its
-// commits and logged corrections added, so the interner is left as before.
-// Allocations themselves are undone by k_end_alloc.
+// In place of the commit, of a dry run or an apply that could not allocate (abort_): the
+// table slots that its owners claimed are restored; an aborted apply's new leaves leave the
+// value map and its logged corrections are taken back, so the interner is left as before
+// (nothing else was written: the commit did not run, close_allocation keeps the cursors).
 template <typename T, int TILE>
-__device__ inline void rollback_body(const Pool<T>& P, const ChunkDev* chunks, const LevelTiles& LT,
-                                     const Drift* drift) {
-    const bool abort = !P.dry && P.ctl->abort_ != 0;
-    if (!P.dry && !abort) return;
-    uint32_t owned = 0;
+__device__ inline void rollback_body(const Pool<T>& P, const LevelTiles& LT) {
     uint64_t total = LT.start[LT.dmax + 1];
     for (uint64_t t = blockIdx.x; t < total; t += gridDim.x) {
         uint32_t h = 1;
@@ -2097,31 +2106,14 @@ __device__ inline void rollback_body(const Pool<T>& P, const ChunkDev* chunks, c
         if (ts & kTslotSingle) P.single[tslot_index(ts)] = 0;
         else P.tab[tslot_index(ts)] = (ts & kTslotTomb) ? kSlotTomb : kSlotEmpty;
         wave_count(stat(P.ctl, ST_TOMB), (ts & kTslotTomb) != 0);
-        uint64_t id = K.id[k];
-        if (P.dry || id == kInvalid) continue;
-        owned++;
-        for (int i = 0; i < 8; i++) {
-            uint64_t c = key_word(K, k, i);
-            if (c != kEmpty) atomicSub(&P.refs[bid_index(c)], 1u);
-        }
     }
-    if (!abort) return;
-    // new leaves leave the value map
+    if (P.dry) return;
     const uint32_t nl = (uint32_t)alloc_done(P, P.ctl->n_new_leaves);
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < nl; j += gridDim.x * blockDim.x)
         leaf_remove(P, (uint32_t)P.values[P.new_leaves[j]]);
     uint32_t nu = P.ctl->n_undo < P.undo_cap ? P.ctl->n_undo : P.undo_cap;
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < nu; j += gridDim.x * blockDim.x)
         atomicSub(&P.refs[P.undo[j].idx], (uint32_t)P.undo[j].delta);
-    // queued corrections applied by the commit (trees that did not fail)
-    uint32_t ndr = P.ctl->n_drift;
-    for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < ndr; j += gridDim.x * blockDim.x) {
-        Drift d = drift[j];
-        if (chunks[d.chunk].status >= 0) atomicSub(&P.refs[d.idx], (uint32_t)d.delta);
-    }
-    uint32_t tot = wave_sum(owned);
-    if (__lane_id() == 0 && tot)
-        atomicAdd((unsigned long long*)&P.ctl->live_branches, (unsigned long long)(-(long long)tot));
 }
 
 // ------------------------------------------------------------------ finalize + GC
@@ -2167,32 +2159,35 @@ __device__ inline void finalize_body(const Pool<T>& P, const ChunkDev* chunks, u
                     st = 1;
                 }
             }
-            status[C.orig] = st;  // the record keeps its status (the rollback may read it)
+            status[C.orig] = st;
         }
         uint32_t k = wave_append(&P.ctl->gc_count[0], push);
         if (push) gc_front[k] = bid_index(old);
     }
 }
 
-// After the last probe: the rollback (dry runs: restore the table; aborted applies:
-// take references back) and the root swap, in one launch.  The swap does not touch
-// the table or reference counts of an aborted apply, and leaves the per-tree records
-// (read by the rollback) unchanged.
+// After the last probe, in one launch: the commit (or the rollback), the root swap and the
+// end of the allocation window.  Every allocation was made, so whether the apply aborts is
+// final, and none of the parts reads what another writes: the swap adds a reference to each
+// new root and queues the old ones.
 template <typename T, int TILE>
-__global__ __launch_bounds__(TILE) void k_finish(Pool<T> P, const ChunkDev* chunks, LevelTiles LT,
-                                                  const Drift* drift, uint32_t n, const uint64_t* slot_off_all,
-                                                  uint32_t n_stride, uint64_t* const* res_levels,
-                                                  uint64_t* const* cand_id_levels, uint64_t* roots,
-                                                  int32_t* status, uint32_t* gc_front) {
-    rollback_body<T, TILE>(P, chunks, LT, drift);
+__global__ __launch_bounds__(TILE) void k_commit(Pool<T> P, const ChunkDev* chunks, const Drift* drift, LevelTiles LT,
+                                                  uint32_t n, const uint64_t* slot_off_all, uint32_t n_stride,
+                                                  uint64_t* const* res_levels, uint64_t* const* cand_id_levels,
+                                                  uint64_t* roots, int32_t* status, uint32_t* gc_front,
+                                                  uint32_t* counts) {
+    const bool abort = !P.dry && P.ctl->abort_ != 0;
+    if (P.dry || abort) rollback_body<T, TILE>(P, LT);
+    else commit_body<T>(P, chunks, drift);
     finalize_body<T>(P, chunks, n, slot_off_all, n_stride, res_levels, cand_id_levels, roots, status, gc_front);
+    if (blockIdx.x == 0 && threadIdx.x == 0) close_allocation(P, abort, counts);
 }
 
 // Leaves created in this sequence that nothing references (their trees hit an
 // error) are released again so the interner is left as before for those trees.
 template <typename T>
 __device__ inline void leaf_cleanup_body(const Pool<T>& P) {
-    uint32_t n = P.ctl->n_new_leaves;
+    const uint32_t n = P.ctl->abort_ ? 0u : P.ctl->n_new_leaves;
     VX_LOOP(i, n) {
         bool freed = false;
         if (i < n) {
@@ -2518,7 +2513,8 @@ __global__ __launch_bounds__(256) void k_gc_round(Pool<T> P, uint32_t round, con
 // fuller table (measured on the 4096-tree uneven apply: 27.1 against 28.3 ms per step).
 // Every block of the clear kernel takes the decision (block 0 records it for the kernels
 // that follow); the clear and re-insert kernels return at once when no rebuild is due.
-__global__ void k_tab_clear(uint64_t* tab, uint64_t nslots, Ctl* ctl, uint64_t lslots, uint32_t force) {
+// The control block's reset for the call that follows rides in block 0.
+__global__ void k_tab_clear(uint64_t* tab, uint64_t nslots, Ctl* ctl, uint64_t* ltab, uint64_t lslots, uint32_t force) {
     static_assert(kStatStripes == 64, "one statistics stripe per lane");
     __shared__ uint32_t s_due;
     if (threadIdx.x < 64) {  // every block takes the same decision from the same counters
@@ -2533,64 +2529,29 @@ __global__ void k_tab_clear(uint64_t* tab, uint64_t nslots, Ctl* ctl, uint64_t l
             bool due = force != 0 || (t >= nslots / 16 && live + t > nslots / 2);
             if (lslots) due = due || (lt >= lslots / 16 && ll + lt > lslots / 4 * 3);
             s_due = due ? (lslots ? 3u : 1u) : 0u;
-            if (blockIdx.x == 0) {  // for the re-insert and the leaf-table kernels
+            if (blockIdx.x == 0) {  // for the re-insertion
                 ctl->rebuild = s_due;
                 if (due) ctl->rebuilds++;
+                ctl_begin(ctl);
             }
         }
     }
     __syncthreads();
     if (!(s_due & 1u)) return;
-    uint4* t4 = (uint4*)tab;
-    const uint64_t n4 = nslots / 2;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (uint64_t)gridDim.x * blockDim.x)
-        t4[i] = make_uint4(0u, 0u, 0u, 0u);
-}
-
-// The control block's reset for the call that follows rides in block 0 (the other blocks
-// read nothing that it writes).
-template <typename T>
-__global__ void k_tab_reinsert(Pool<T> P) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) ctl_begin(P.ctl);
-    if (!(P.ctl->rebuild & 1u)) return;
-    // the cleared table holds no tombstone (no other block reads the counter here)
-    if (blockIdx.x == 0 && threadIdx.x < kStatStripes) P.ctl->st[threadIdx.x][ST_TOMB] = 0;
-    const uint32_t top = P.ctl->next_index;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < top; i += gridDim.x * blockDim.x) {
-        const uint32_t tm = tmg_tm(P.tmg[i]);
-        if (i == 0 || tm == 0) continue;
-        uint64_t ch[8];
-        const uint64_t* src = P.children + 8ull * i;
-#pragma unroll
-        for (int j = 0; j < 8; j++) ch[j] = src[j];
-        if (P.single && tm_is_single(tm)) continue;  // in the one-leaf index, which has no tombstones
-        const uint64_t h = branch_hash(ch, tm);
-        const uint64_t want = slot_make(slot_tag(h), false, 0, i);
-        uint64_t s = h & P.tmask;
-        for (uint64_t guard = 0; guard <= P.tmask; guard++) {
-            if (atomicCAS((unsigned long long*)&P.tab[s], 0ull, (unsigned long long)want) == 0ull) break;
-            s = (s + 1) & P.tmask;
-        }
+    for (int k = 0; k < 2; k++) {  // both tables are rebuilt together
+        uint4* t4 = (uint4*)(k ? ltab : tab);
+        const uint64_t n4 = (k ? lslots : nslots) / 2;
+        for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (uint64_t)gridDim.x * blockDim.x)
+            t4[i] = make_uint4(0u, 0u, 0u, 0u);
     }
 }
 
-// The hashed leaf table of four-byte voxels, rebuilt the same way: every live leaf (a
-// node without a types/mask word that holds a reference) is inserted again.
-__global__ void k_ltab_clear(uint64_t* ltab, uint64_t nslots, Ctl* ctl) {
-    if (!(ctl->rebuild & 2u)) return;
-    uint4* t4 = (uint4*)ltab;
-    const uint64_t n4 = nslots / 2;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (uint64_t)gridDim.x * blockDim.x)
-        t4[i] = make_uint4(0u, 0u, 0u, 0u);
-    if (blockIdx.x == 0 && threadIdx.x < kStatStripes) ctl->st[threadIdx.x][ST_LTOMB] = 0;
-}
-
+// i32, fills and forced rebuilds: the re-insertion as a launch of its own (32-bit voxels look
+// their leaves up in the table that it fills; an apply of u8 or u16 voxels has it ride in its
+// first kernel).
 template <typename T>
-__global__ void k_ltab_reinsert(Pool<T> P) {
-    if (!(P.ctl->rebuild & 2u)) return;
-    const uint32_t top = P.ctl->next_index;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < top; i += gridDim.x * blockDim.x)
-        if (i != 0 && tmg_tm(P.tmg[i]) == 0 && P.refs[i] != 0) leaf_publish(P, (uint32_t)P.values[i], i);
+__global__ void k_tab_reinsert(Pool<T> P) {
+    reinsert_body(P, blockIdx.x, gridDim.x);
 }
 
 // ------------------------------------------------------------------ single-voxel set
@@ -2618,8 +2579,13 @@ constexpr uint32_t kSetRec = 2 * kLevels;
 
 template <typename T>
 __global__ void k_set_descend(Pool<T> P, ChunkDev* chunks, uint32_t n, const uint64_t* roots, const int32_t* xyz,
-                              const T* vals, uint64_t* rec, uint32_t* meta) {
-    VX_LOOP(c, n) {
+                              const T* vals, uint64_t* rec, uint32_t* meta, uint32_t nprep) {
+    if (blockIdx.x >= nprep) {  // the table's re-insertion, when it is due
+        reinsert_body(P, blockIdx.x - nprep, gridDim.x - nprep);
+        return;
+    }
+    for (uint64_t c0 = (uint64_t)blockIdx.x * blockDim.x; c0 < n; c0 += (uint64_t)nprep * blockDim.x) {
+        const uint64_t c = c0 + threadIdx.x;
         if (c < n) {
             ChunkDev& C = chunks[c];
             C.root_in = roots[C.orig];
@@ -2851,6 +2817,11 @@ __global__ void k_fill_finish(Pool<T> P, uint32_t n, uint64_t* roots, const uint
             }
         }
     }
+}
+
+template <typename T>
+__global__ void k_end_alloc(Pool<T> P) {
+    close_allocation(P, false, nullptr);
 }
 
 // ------------------------------------------------------------------ reads
