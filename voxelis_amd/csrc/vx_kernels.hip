@@ -2187,7 +2187,7 @@ __global__ __launch_bounds__(TILE) void k_commit(Pool<T> P, const ChunkDev* chun
 // error) are released again so the interner is left as before for those trees.
 template <typename T>
 __device__ inline void leaf_cleanup_body(const Pool<T>& P) {
-    const uint32_t n = P.ctl->abort_ ? 0u : P.ctl->n_new_leaves;
+    const uint32_t n = P.ctl->abort_ || !P.ctl->h1_fail ? 0u : P.ctl->n_new_leaves;
     VX_LOOP(i, n) {
         bool freed = false;
         if (i < n) {
@@ -2226,11 +2226,16 @@ __device__ inline void leaf_cleanup_body(const Pool<T>& P) {
 // block has to see it, and a chain of small rounds (a few thousand replaced paths) costs
 // one launch instead of one per height.  A launch frees nodes of any depth at or below
 // its round's, so the D + 1 launches of a tree of depth D still reach every node.
+//
+// The final round takes a front of any size that way and hands nothing on: children past a
+// pass wait in the block's own runs of the next queue.  It ends the rounds early
+// (gc_rounds, with the times).
 constexpr uint32_t kGcStage = 2048;      // children staged per pass (8 per lane of a 256-lane block)
 constexpr uint32_t kGcLocal = 256;       // the most nodes of one pass a block follows itself
 constexpr uint32_t kGcLocalShare = 64;   // a front up to this many nodes per block is followed
 constexpr uint32_t kGcShareMin = 16;     // ... in shares of at least this many nodes
 constexpr uint32_t kGcFreeStage = 768;   // freed nodes staged before one free-stack update
+constexpr uint32_t kGcSegs = 16;         // waiting runs of a block in the final round (heights are 8)
 
 // Frees node idx, whose count is zero: drops its pattern, marks the slot free and
 // releases its children.  Children decremented here that reach zero are staged in
@@ -2332,17 +2337,19 @@ __device__ inline void gc_agg_flush(const Pool<T>& P, uint32_t* akey, uint32_t* 
 
 template <typename T>
 __global__ __launch_bounds__(256) void k_gc_round(Pool<T> P, uint32_t round, const uint32_t* front, uint32_t* next,
-                                                  bool decrement_self, uint64_t front_cap, bool leaf_cleanup) {
+                                                  bool decrement_self, uint64_t front_cap, bool leaf_cleanup,
+                                                  bool final) {
     __shared__ uint32_t akey[kAggSlots], acnt[kAggSlots];
     __shared__ uint32_t s_next[kGcStage];
     __shared__ uint32_t s_cur[kGcLocal];
     __shared__ uint32_t s_free[kGcFreeStage];
     __shared__ uint32_t s_nnext, s_nfree, s_bnext, s_bfree;
+    __shared__ uint32_t s_seg[kGcSegs], s_seglen[kGcSegs];  // final round: the block's runs of waiting nodes
     __shared__ unsigned long long s_leaves, s_branches, s_tombs, s_recycled;
     uint64_t n = P.ctl->gc_count[round];
     if (n > front_cap) n = front_cap;
     // a small front: the block's share [lo, hi), followed locally
-    const bool local = n <= (uint64_t)gridDim.x * kGcLocalShare;
+    const bool local = final || n <= (uint64_t)gridDim.x * kGcLocalShare;
     uint64_t lo = 0, hi = 0;
     if (local) {
         const uint64_t share = max((uint64_t)kGcShareMin, (n + gridDim.x - 1) / gridDim.x);
@@ -2367,8 +2374,8 @@ __global__ __launch_bounds__(256) void k_gc_round(Pool<T> P, uint32_t round, con
     if (local) {
         // passes over the block's share, then over the children that reached zero in the
         // block, while they fit one pass (the loop is uniform over the block)
-        uint32_t cnt = (uint32_t)(hi - lo);
-        bool first = true;
+        uint32_t cnt = (uint32_t)min(hi - lo, (uint64_t)kGcLocal), nseg = 0;
+        bool first = true;  // the pass is of the front
         for (;;) {
             uint32_t idx = kNoIdx;
             if (threadIdx.x < cnt) {
@@ -2395,10 +2402,47 @@ __global__ __launch_bounds__(256) void k_gc_round(Pool<T> P, uint32_t round, con
             // those that reach zero join the children of the next pass
             gc_agg_flush(P, akey, acnt, s_next, &s_nnext, true);
             __syncthreads();
+            if (first) lo += cnt;
             const uint32_t nn = s_nnext, nf = s_nfree;
-            const bool more = nn != 0 && nn <= kGcLocal;
+            // the children past one pass wait in `next` (its counter hands out the places):
+            // in the final round as a run of this block, else for the next launch, all of them
+            const uint32_t take = nn <= kGcLocal ? nn : final ? kGcLocal : 0u, rest = nn - take;
+            if (rest) {
+                if (threadIdx.x == 0) s_bnext = atomicAdd(next_count, rest);
+                __syncthreads();
+                const uint32_t base = s_bnext;
+                for (uint32_t k = threadIdx.x; k < rest; k += blockDim.x) {
+                    if ((uint64_t)base + k < front_cap) next[base + k] = s_next[take + k];
+                    else atomicOr(&P.ctl->err, kErrPoison);
+                }
+                if (final && nseg < kGcSegs && (uint64_t)base + rest <= front_cap) {
+                    if (threadIdx.x == 0) {
+                        s_seg[nseg] = base;
+                        s_seglen[nseg] = rest;
+                    }
+                    nseg++;
+                }
+            }
+            first = false;
+            cnt = take;
+            if (cnt == 0 && nseg) {
+                // the last run's end (its nodes lie deeper than those of the runs before it,
+                // so there is at most a run per height)
+                __syncthreads();
+                const uint32_t len = s_seglen[nseg - 1];
+                cnt = min(len, kGcLocal);
+                if (threadIdx.x < cnt) s_cur[threadIdx.x] = next[s_seg[nseg - 1] + len - cnt + threadIdx.x];
+                __syncthreads();
+                if (threadIdx.x == 0) s_seglen[nseg - 1] = len - cnt;
+                if (len == cnt) nseg--;
+            } else if (cnt) {
+                for (uint32_t k = threadIdx.x; k < cnt; k += blockDim.x) s_cur[k] = s_next[k];
+            } else if (lo < hi) {
+                first = true;
+                cnt = (uint32_t)min(hi - lo, (uint64_t)kGcLocal);
+            }
             // the staged frees go to the free stack when the next pass might not fit
-            if (nf && (!more || nf + kGcLocal > kGcFreeStage)) {
+            if (nf && (cnt == 0 || nf + kGcLocal > kGcFreeStage)) {
                 if (threadIdx.x == 0) s_bfree = atomicAdd(&P.ctl->free_top, nf);
                 __syncthreads();
                 for (uint32_t k = threadIdx.x; k < nf; k += blockDim.x) {
@@ -2409,27 +2453,10 @@ __global__ __launch_bounds__(256) void k_gc_round(Pool<T> P, uint32_t round, con
                 __syncthreads();
                 if (threadIdx.x == 0) s_nfree = 0;
             }
-            if (!more) {
-                // more children than one pass: the next launch takes them
-                if (nn) {
-                    if (threadIdx.x == 0) s_bnext = atomicAdd(next_count, nn);
-                    __syncthreads();
-                    for (uint32_t k = threadIdx.x; k < nn; k += blockDim.x) {
-                        const uint32_t pos = s_bnext + k;
-                        if (pos < front_cap) next[pos] = s_next[k];
-                        else atomicOr(&P.ctl->err, kErrPoison);
-                    }
-                }
-                __syncthreads();
-                if (threadIdx.x == 0) s_nnext = 0;
-                break;
-            }
-            for (uint32_t k = threadIdx.x; k < nn; k += blockDim.x) s_cur[k] = s_next[k];
             __syncthreads();
             if (threadIdx.x == 0) s_nnext = 0;
             __syncthreads();
-            cnt = nn;
-            first = false;
+            if (cnt == 0) break;
         }
     } else {
         for (uint64_t b0 = (uint64_t)blockIdx.x * blockDim.x; b0 < n; b0 += (uint64_t)gridDim.x * blockDim.x) {
