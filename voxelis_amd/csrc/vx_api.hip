@@ -127,13 +127,11 @@ struct Plan {
     uint64_t ws_gen = 0;
     uint64_t last_use = 0;
     hipGraphExec_t exec = nullptr;
-    Grow chunks, slot_off, tables;  // the call's records, owned by the plan
+    Grow records;  // the call's records, owned by the plan
     void release() {
         if (exec) (void)hipGraphExecDestroy(exec);
         exec = nullptr;
-        chunks.release();
-        slot_off.release();
-        tables.release();
+        records.release();
     }
 };
 
@@ -162,13 +160,13 @@ struct vx_interner {
     bool own_stream = false;
     int poisoned = 0;
     // workspace
-    Grow chunks, slot_off, ptr_tables, gc_front[2], stage, scratch, drift, undo, owners;
+    Grow records, gc_front[2], stage, scratch, drift, undo, owners;
     Grow set_rec, set_meta;  // single-voxel set: the recorded path of every tree
     // edit-list path: zero-kept dense Batch buffers, sort buffers, tree records
     Grow edit_ws, edit_keys[2], edit_order[2], edit_tmp, edit_trees, edit_first, edit_status;
     LevelBufs lv[kLevels + 1];
     // pinned staging ring: a slot is reused only after its copies completed
-    static constexpr int kRing = 4;
+    static constexpr int kRing = 8;
     void* h_pinned_ring[kRing] = {nullptr};
     size_t h_pinned_cap[kRing] = {0};
     hipEvent_t ring_ev[kRing] = {nullptr};
@@ -241,7 +239,8 @@ bool pinned_ensure(vx_interner* h, size_t bytes) {
     return true;
 }
 
-// Mark the current staging slot busy until the stream passes this point.
+// Mark the current staging slot busy until the stream passes this point (the end of its
+// call: an event between the kernels of a call is a gap on the device).
 void pinned_release(vx_interner* h) {
     int i = h->ring_cur;
     if (hipEventRecord(h->ring_ev[i], h->stream) == hipSuccess) h->ring_used[i] = true;
@@ -306,7 +305,8 @@ struct ApplyOpts {
 
 constexpr unsigned kRebuildGrid = 512;
 template <typename T>
-int rebuild_step(vx_interner* h, bool force, bool reinsert);
+int rebuild_step(vx_interner* h, bool force, bool reinsert, const void* up_src = nullptr, void* up_dst = nullptr,
+                 size_t up_bytes = 0);
 
 template <typename T, int TILE>
 int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* batches,
@@ -362,53 +362,55 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
         if (b.has_patches && (!b.masks || !b.values)) return VX_E_INVALID_ARG;
         return 0;
     };
-    auto sort_key = [&](uint32_t i) -> uint32_t {
-        const vx_batch_view& b = batches[i];
-        return (b.has_patches && status_of(b) == 0 && b.reserved != kViewSkip) ? b.depth : 0u;
-    };
-    std::vector<uint32_t> perm(n);
-    for (size_t i = 0; i < n; i++) perm[i] = (uint32_t)i;
-    std::stable_sort(perm.begin(), perm.end(),
-                     [&](uint32_t a, uint32_t b) { return sort_key(a) < sort_key(b); });
-    size_t chunk_bytes = n * sizeof(ChunkDev);
-    size_t off_count = (size_t)(kLevels + 1) * n;
-    size_t tab_bytes = 2 * (kLevels + 1) * sizeof(void*) + (kLevels + 1) * sizeof(Cands);
-    size_t stage_bytes = chunk_bytes + off_count * sizeof(uint64_t) + tab_bytes;
+    // records: trees with patches by depth (others first), in the caller's order within a
+    // depth, then the tables; one staging buffer, one upload
+    const size_t chunk_bytes = n * sizeof(ChunkDev);
+    const size_t tab_bytes = 2 * (kLevels + 1) * sizeof(void*) + (kLevels + 1) * sizeof(Cands) + sizeof(SlotMap);
+    const size_t stage_bytes = (chunk_bytes + tab_bytes + 15) / 16 * 16;
     if (!pinned_ensure(h, stage_bytes)) return VX_E_HIP;
     ChunkDev* hc = (ChunkDev*)h->h_pinned;
-    uint64_t* hoff = (uint64_t*)((char*)h->h_pinned + chunk_bytes);
     uint32_t dmax = 0, dall = 0;  // deepest patched tree, deepest tree
     uint64_t old_nodes = 0;       // a bound of the branch nodes the call can free
     struct Run { uint32_t start, count, depth; };
+    const auto depth_key = [&](const vx_batch_view& b, int32_t st) -> uint32_t {
+        return b.has_patches && st == 0 && b.reserved != kViewSkip ? b.depth : 0u;
+    };
+    uint32_t of_depth[kLevels + 1] = {0}, at[kLevels + 1] = {0};
+    for (size_t i = 0; i < n; i++) of_depth[depth_key(batches[i], status_of(batches[i]))]++;
     std::vector<Run> runs;
-    for (size_t c = 0; c < n; c++) {
-        const vx_batch_view& b = batches[perm[c]];
-        ChunkDev& C = hc[c];
-        std::memset(&C, 0, sizeof(C));
+    for (uint32_t k = 1; k <= (uint32_t)kLevels; k++) {
+        at[k] = at[k - 1] + of_depth[k - 1];
+        if (k < (uint32_t)kLevels && of_depth[k]) {
+            runs.push_back({at[k], of_depth[k], k});
+            dmax = k;
+        }
+    }
+    for (size_t i = 0; i < n; i++) {
+        const vx_batch_view& b = batches[i];
+        const int32_t st = status_of(b);
+        const uint32_t key = depth_key(b, st);
+        ChunkDev C;
         C.masks = b.masks;
         C.values = b.values;
         C.fill = b.fill_value & (sizeof(T) == 1 ? 0xFFull : sizeof(T) == 2 ? 0xFFFFull : 0xFFFFFFFFull);
-        C.orig = perm[c];
+        C.root_in = C.init = 0;
+        C.orig = (uint32_t)i;
         C.depth = b.depth;
         C.has_fill = b.has_fill ? 1 : 0;
         C.skip = b.reserved == kViewSkip ? 1 : 0;
-        C.status = C.status0 = status_of(b);
-        C.has_patches = (b.has_patches && C.status == 0 && !C.skip) ? 1 : 0;
-        if (C.status == 0 && !C.skip) {
+        C.status = C.status0 = st;
+        C.has_patches = key != 0 || (b.has_patches && st == 0 && !C.skip) ? 1 : 0;
+        if (st == 0 && !C.skip) {
             dall = std::max<uint32_t>(dall, b.depth);
             old_nodes += setm || b.depth == 0 ? b.depth + 1u : slots_at(b.depth, 1) + slots_at(b.depth, 1) / 4;
         }
-        if (!C.has_patches) continue;
-        uint32_t d = b.depth;
-        dmax = std::max<uint32_t>(dmax, d);
-        if (!runs.empty() && runs.back().depth == d && runs.back().start + runs.back().count == c)
-            runs.back().count++;
-        else
-            runs.push_back({(uint32_t)c, 1, d});
+        hc[at[key]++] = C;
     }
-    for (size_t i = 0; i < off_count; i++) hoff[i] = ~0ull;
     LevelInfo L[kLevels + 1];
     std::memset(L, 0, sizeof(L));
+    SlotMap* hmap = (SlotMap*)((char*)hc + chunk_bytes + 2 * (kLevels + 1) * sizeof(void*) + (kLevels + 1) * sizeof(Cands));
+    std::memset(hmap, 0, sizeof(SlotMap));
+    for (const Run& r : runs) hmap->start[r.depth] = r.start;
     std::vector<Run> lruns[kLevels + 1];
     for (uint32_t hh = 1; hh <= dmax; hh++) {
         uint64_t base = 0;
@@ -423,9 +425,8 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
             L[hh].slot_base[g] = base;
             L[hh].chunk_base[g] = r.start;
             L[hh].depth[g] = setm ? hh : r.depth;  // set mode: slot = tree, shift 0
-            uint64_t per = setm ? 1 : slots_at(r.depth, hh);
-            for (uint32_t k = 0; k < r.count; k++) hoff[(size_t)hh * n + r.start + k] = base + k * per;
-            base += per * r.count;
+            hmap->base[hh][r.depth] = base;
+            base += (setm ? 1 : slots_at(r.depth, hh)) * r.count;
         }
         L[hh].slot_base[L[hh].ngroups] = base;
         L[hh].nslots = base;
@@ -446,11 +447,8 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
         }
     }
     // ---- workspace (a captured call owns its records)
-    Grow& g_chunks = plan ? plan->chunks : h->chunks;
-    Grow& g_off = plan ? plan->slot_off : h->slot_off;
-    Grow& g_tables = plan ? plan->tables : h->ptr_tables;
-    if (!g_chunks.ensure(chunk_bytes, !plan)) return VX_E_HIP;
-    if (!g_off.ensure(off_count * sizeof(uint64_t), !plan)) return VX_E_HIP;
+    Grow& records = plan ? plan->records : h->records;
+    if (!records.ensure(stage_bytes, !plan)) return VX_E_HIP;
     uint64_t* res_ptrs_h[kLevels + 1] = {nullptr};
     uint64_t* cid_ptrs_h[kLevels + 1] = {nullptr};
     Cands K[kLevels + 1];
@@ -496,24 +494,24 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     for (uint32_t hh = 1; hh <= dmax; hh++) nown += ntiles[hh] * TILE;
     if (!h->owners.ensure(nown * 8)) return VX_E_HIP;
     P.owners = (uint64_t*)h->owners.ptr;
-    void** hptrs = (void**)((char*)h->h_pinned + chunk_bytes + off_count * sizeof(uint64_t));
+    void** hptrs = (void**)((char*)h->h_pinned + chunk_bytes);
     for (int i = 0; i <= kLevels; i++) {
         hptrs[i] = res_ptrs_h[i];
         hptrs[kLevels + 1 + i] = cid_ptrs_h[i];
     }
     std::memcpy(hptrs + 2 * (kLevels + 1), K, (kLevels + 1) * sizeof(Cands));
-    if (!g_tables.ensure(tab_bytes, !plan)) return VX_E_HIP;
     size_t gcap = (size_t)h->capacity + n + 16;
     if (!h->gc_front[0].ensure(gcap * 4) || !h->gc_front[1].ensure(gcap * 4)) return VX_E_HIP;
-    ChunkDev* dchunks = (ChunkDev*)g_chunks.ptr;
-    uint64_t* doff = (uint64_t*)g_off.ptr;
-    uint64_t* const* dres = (uint64_t* const*)g_tables.ptr;
+    ChunkDev* dchunks = (ChunkDev*)records.ptr;
+    uint64_t* const* dres = (uint64_t* const*)((char*)records.ptr + chunk_bytes);
     uint64_t* const* dcid = dres + (kLevels + 1);
-    HIPCHK(hipMemcpyAsync(dchunks, hc, chunk_bytes, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(doff, hoff, off_count * sizeof(uint64_t), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(g_tables.ptr, hptrs, tab_bytes, hipMemcpyHostToDevice, s));
-    P.levels = (const Cands*)((void**)g_tables.ptr + 2 * (kLevels + 1));
-    pinned_release(h);
+    P.levels = (const Cands*)(dres + 2 * (kLevels + 1));
+    const SlotMap* dmap = (const SlotMap*)(P.levels + kLevels + 1);
+    // a captured sequence keeps its records; a dry run has no table step to bring them along
+    if (plan || opt.dry) {
+        HIPCHK(hipMemcpyAsync(records.ptr, hc, stage_bytes, hipMemcpyHostToDevice, s));
+        pinned_release(h);
+    }
     uint64_t nb = std::max<uint64_t>(dmax >= 2 ? L[1].nslots : 1, 1);
     if (!h->drift.ensure(nb * sizeof(Drift))) return VX_E_HIP;
     Drift* ddrift = (Drift*)h->drift.ptr;
@@ -555,8 +553,7 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
               drec, dmeta, grid_for(n));
     for (uint32_t hh = 1; hh <= dmax; hh++) {
         unsigned th = (unsigned)ntiles[hh];
-        VX_LAUNCH(h, KID_SET_LEVEL, k_set_level<T VX_COMMA TILE>, th, TILE, P, dchunks, L[hh], doff,
-                  (uint32_t)n, sx, sv, drec, dmeta, res_ptrs_h[hh - 1], cid_ptrs_h[hh - 1], res_ptrs_h[hh], K[hh],
+        VX_LAUNCH(h, KID_SET_LEVEL, k_set_level<T VX_COMMA TILE>, th, TILE, P, dchunks, L[hh], sx, sv, drec, dmeta, res_ptrs_h[hh - 1], cid_ptrs_h[hh - 1], res_ptrs_h[hh], K[hh],
                   tiles_h[hh]);
         uint32_t gh = probe_group(th, h->tune.probe_blocks);
         VX_LAUNCH(h, KID_PROBE_UPPER, k_probe<T VX_COMMA TILE>, (th + gh - 1) / gh, TILE, P, K[hh], tiles_h[hh],
@@ -566,7 +563,7 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     };
     auto launch_all = [&]() -> int {
     if (!opt.dry) {
-        int rc = rebuild_step<T>(h, false, nre == 0);
+        int rc = rebuild_step<T>(h, false, nre == 0, plan ? nullptr : hc, records.ptr, stage_bytes);
         if (rc) return rc;
     }
     if (setm) {
@@ -577,7 +574,7 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     unsigned np = grid_for(n);
     unsigned nd = L[3].nslots ? grid_for(L[3].nslots) : 0u;
     VX_LAUNCH(h, KID_PREPARE, k_prepare<T>, np + nd + nre, kBlock, P, dchunks, (uint32_t)n, roots, pre_status, np,
-              nd, L[3], doff, O);
+              nd, L[3], dmap, O);
     unsigned t1 = (unsigned)ntiles[1];
     if (dmax >= 2 && br == kBR)
         VX_LAUNCH(h, KID_BRICK_BUILD, k_brick_build<T VX_COMMA TILE VX_COMMA kBR>, t1 / kBR, TILE, P, dchunks, L[1],
@@ -609,7 +606,7 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     // lane per possible owner (a slot of some level) and per tree, up to the commit grid
     const uint64_t cg = std::max<uint64_t>(LT.start[LT.dmax + 1], (n + TILE - 1) / TILE);
     VX_LAUNCH(h, KID_COMMIT, k_commit<T VX_COMMA TILE>, (unsigned)std::min<uint64_t>(std::max<uint64_t>(cg, 1), h->tune.commit_grid),
-              TILE, P, dchunks, ddrift, LT, (uint32_t)n, doff, (uint32_t)n, dres, dcid, roots, status, gf0, opt.counts);
+              TILE, P, dchunks, ddrift, LT, (uint32_t)n, dmap, dres, dcid, roots, status, gf0, opt.counts);
     if (!opt.dry) {
         // dec_ref_recursive of the replaced roots: a tree of depth D has nodes at
         // heights D..0, one round each; the first round also releases unused new leaves.
@@ -631,7 +628,11 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     }
     return hipGetLastError() == hipSuccess ? VX_OK : VX_E_HIP;
     };
-    if (!plan) return launch_all();
+    if (!plan) {
+        const int rc = launch_all();
+        if (!opt.dry) pinned_release(h);
+        return rc;
+    }
     // capture on a private stream, then replay on the interner's stream
     if (!h->cap_stream && hipStreamCreateWithFlags(&h->cap_stream, hipStreamNonBlocking) != hipSuccess)
         return VX_E_HIP;
@@ -666,13 +667,14 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
 // stream, captured with the call's launch sequence): the device decides whether the
 // pattern table (and the i32 leaf table) is rebuilt now, and clears it; the re-insertion is
 // a launch of its own (reinsert) or rides in the call's next kernel.  force: rebuild
-// regardless.
+// regardless.  up_*: the call's records (whole 16 bytes), pinned memory to the device.
 template <typename T>
-int rebuild_step(vx_interner* h, bool force, bool reinsert) {
+int rebuild_step(vx_interner* h, bool force, bool reinsert, const void* up_src, void* up_dst, size_t up_bytes) {
     Pool<T> P = pool_of<T>(h);
     hipStream_t s = h->stream;
     k_tab_clear<<<kRebuildGrid, kBlock, 0, s>>>(h->tab, h->tslots, h->ctl, h->ltab, h->ltab ? h->lslots : 0ull,
-                                                force ? 1u : 0u);
+                                                force ? 1u : 0u, (const uint4*)up_src, (uint4*)up_dst,
+                                                up_src ? (uint32_t)(up_bytes / 16) : 0u);
     if (reinsert) k_tab_reinsert<T><<<kRebuildGrid, kBlock, 0, s>>>(P);
     return hipGetLastError() == hipSuccess ? VX_OK : VX_E_HIP;
 }
@@ -990,9 +992,7 @@ int vx_interner_destroy(vx_interner* h) {
                     h->ltab, h->need_list, h->single};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
-    h->chunks.release();
-    h->slot_off.release();
-    h->ptr_tables.release();
+    h->records.release();
     h->gc_front[0].release();
     h->gc_front[1].release();
     h->stage.release();

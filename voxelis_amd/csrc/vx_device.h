@@ -165,6 +165,17 @@ struct LevelInfo {
     uint64_t nslots;
 };
 
+// Where the slots of a tree lie: the tree of record c and depth D (records are grouped by
+// depth, the first of depth D is start[D]) owns the slots from
+// base[h][D] + ((c - start[D]) << 3 (D - h)) at height h.
+struct SlotMap {
+    uint64_t base[kLevels + 1][kLevels];
+    uint32_t start[kLevels];
+};
+__device__ inline uint64_t slot_of(const SlotMap* M, uint32_t h, uint32_t c, uint32_t D) {
+    return M->base[h][D] + ((uint64_t)(c - M->start[D]) << (3 * (D - h)));
+}
+
 // Per height h >= 2: the previous tree's node at every level-h slot (a branch,
 // the leaf that covers the position from above, or empty), written by one
 // descent pass at the start of an apply for trees without a fill.

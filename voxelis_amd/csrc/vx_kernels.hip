@@ -684,7 +684,7 @@ __device__ inline void close_allocation(const Pool<T>& P, bool abort, uint32_t* 
 // skipped; a depth-2 tree's height-2 node is its root (recorded by k_prepare).
 template <typename T>
 __device__ inline void descend_body(const Pool<T>& P, const ChunkDev* chunks, const LevelInfo& L3,
-                                    const uint64_t* doff, uint32_t n, const OldNodes& O,
+                                    const SlotMap* M, const OldNodes& O,
                                     const uint64_t* roots, uint64_t slot) {
     const GroupPos G = group_pos(L3, slot);
     uint64_t local = slot - G.base;
@@ -705,7 +705,7 @@ __device__ inline void descend_body(const Pool<T>& P, const ChunkDev* chunks, co
             }
         }
         uint32_t sub = 3 * (uint32_t)(hh - 3);
-        if ((q & ((1u << sub) - 1u)) == 0) O.at[hh][doff[(size_t)hh * n + c] + (q >> sub)] = cur;
+        if ((q & ((1u << sub) - 1u)) == 0) O.at[hh][slot_of(M, hh, c, D) + (q >> sub)] = cur;
     }
     uint64_t below[8];
     const bool branch = cur != kEmpty && !bid_is_leaf(cur);
@@ -714,7 +714,7 @@ __device__ inline void descend_body(const Pool<T>& P, const ChunkDev* chunks, co
     const uint64_t* src = P.children + 8ull * (ok ? bid_index(cur) : 0u);
 #pragma unroll
     for (int i = 0; i < 8; i++) below[i] = ok ? src[i] : (branch ? kEmpty : cur);
-    uint64_t* dst = O.at[2] + doff[(size_t)2 * n + c] + 8ull * q;
+    uint64_t* dst = O.at[2] + slot_of(M, 2, c, D) + 8ull * q;
 #pragma unroll
     for (int i = 0; i < 8; i++) dst[i] = below[i];
 }
@@ -760,7 +760,7 @@ __device__ inline void reinsert_body(const Pool<T>& P, uint32_t b, uint32_t nb) 
 template <typename T>
 __global__ void k_prepare(Pool<T> P, ChunkDev* chunks, uint32_t n, const uint64_t* roots,
                           const int32_t* pre_status, uint32_t nprep, uint32_t ndesc, LevelInfo L3,
-                          const uint64_t* doff, OldNodes O) {
+                          const SlotMap* M, OldNodes O) {
     if (blockIdx.x >= nprep + ndesc) {
         reinsert_body(P, blockIdx.x - nprep - ndesc, gridDim.x - nprep - ndesc);
         return;
@@ -768,7 +768,7 @@ __global__ void k_prepare(Pool<T> P, ChunkDev* chunks, uint32_t n, const uint64_
     if (blockIdx.x >= nprep) {
         uint64_t stride = (uint64_t)ndesc * blockDim.x;
         for (uint64_t s = (uint64_t)(blockIdx.x - nprep) * blockDim.x + threadIdx.x; s < L3.nslots; s += stride)
-            descend_body(P, chunks, L3, doff, n, O, roots, s);
+            descend_body(P, chunks, L3, M, O, roots, s);
         return;
     }
     // a dry run's control-block reset rides in block 0 (nothing else here reads it); any
@@ -780,7 +780,7 @@ __global__ void k_prepare(Pool<T> P, ChunkDev* chunks, uint32_t n, const uint64_
         C.init = C.root_in;
         C.status = C.status0;
         // a depth-2 tree's height-2 node is its root (deeper trees: the descent)
-        if (C.depth == 2 && C.has_patches && !C.has_fill) O.at[2][doff[(size_t)2 * n + c]] = C.root_in;
+        if (C.depth == 2 && C.has_patches && !C.has_fill) O.at[2][slot_of(M, 2, (uint32_t)c, 2)] = C.root_in;
         if (P.per_tree) P.per_tree[C.orig] = 0;
         if (pre_status && pre_status[C.orig] < 0 && C.status >= 0) C.status = pre_status[C.orig];
         if (C.status >= 0 && C.has_fill) {
@@ -2122,8 +2122,7 @@ __device__ inline void rollback_body(const Pool<T>& P, const LevelTiles& LT) {
 // queue the old root for dec_ref_recursive.
 template <typename T>
 __device__ inline void finalize_body(const Pool<T>& P, const ChunkDev* chunks, uint32_t n,
-                                     const uint64_t* slot_off_all, uint32_t n_stride,
-                                     uint64_t* const* res_levels, uint64_t* const* cand_id_levels,
+                                     const SlotMap* M, uint64_t* const* res_levels, uint64_t* const* cand_id_levels,
                                      uint64_t* roots, int32_t* status, uint32_t* gc_front) {
     const uint32_t ab = P.ctl->abort_;
     VX_LOOP(c, n) {
@@ -2142,7 +2141,7 @@ __device__ inline void finalize_body(const Pool<T>& P, const ChunkDev* chunks, u
                     nw = C.init;
                 } else {
                     uint32_t D = C.depth;
-                    uint64_t r = res_levels[D][slot_off_all[(uint64_t)D * n_stride + c]];
+                    uint64_t r = res_levels[D][slot_of(M, D, (uint32_t)c, D)];
                     nw = r != kInvalid ? resolve(r, cand_id_levels[D]) : r;
                 }
                 old = C.root_in;
@@ -2172,14 +2171,14 @@ __device__ inline void finalize_body(const Pool<T>& P, const ChunkDev* chunks, u
 // new root and queues the old ones.
 template <typename T, int TILE>
 __global__ __launch_bounds__(TILE) void k_commit(Pool<T> P, const ChunkDev* chunks, const Drift* drift, LevelTiles LT,
-                                                  uint32_t n, const uint64_t* slot_off_all, uint32_t n_stride,
+                                                  uint32_t n, const SlotMap* M,
                                                   uint64_t* const* res_levels, uint64_t* const* cand_id_levels,
                                                   uint64_t* roots, int32_t* status, uint32_t* gc_front,
                                                   uint32_t* counts) {
     const bool abort = !P.dry && P.ctl->abort_ != 0;
     if (P.dry || abort) rollback_body<T, TILE>(P, LT);
     else commit_body<T>(P, chunks, drift);
-    finalize_body<T>(P, chunks, n, slot_off_all, n_stride, res_levels, cand_id_levels, roots, status, gc_front);
+    finalize_body<T>(P, chunks, n, M, res_levels, cand_id_levels, roots, status, gc_front);
     if (blockIdx.x == 0 && threadIdx.x == 0) close_allocation(P, abort, counts);
 }
 
@@ -2541,7 +2540,13 @@ __global__ __launch_bounds__(256) void k_gc_round(Pool<T> P, uint32_t round, con
 // Every block of the clear kernel takes the decision (block 0 records it for the kernels
 // that follow); the clear and re-insert kernels return at once when no rebuild is due.
 // The control block's reset for the call that follows rides in block 0.
-__global__ void k_tab_clear(uint64_t* tab, uint64_t nslots, Ctl* ctl, uint64_t* ltab, uint64_t lslots, uint32_t force) {
+// The call's records come along: copied from pinned host memory to the device by this launch.
+// Two copy commands of 0.3 MB each, for 4096 trees, held the stream for 40 us, in some
+// processes for three times that (a set of one voxel in each: 233 or 320 us a call; 177 so,
+// with the slots' places computed and not uploaded).
+__global__ void k_tab_clear(uint64_t* tab, uint64_t nslots, Ctl* ctl, uint64_t* ltab, uint64_t lslots, uint32_t force,
+                            const uint4* up_src, uint4* up_dst, uint32_t up_n) {
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < up_n; i += gridDim.x * blockDim.x) up_dst[i] = up_src[i];
     static_assert(kStatStripes == 64, "one statistics stripe per lane");
     __shared__ uint32_t s_due;
     if (threadIdx.x < 64) {  // every block takes the same decision from the same counters
@@ -2695,7 +2700,7 @@ __global__ void k_set_descend(Pool<T> P, ChunkDev* chunks, uint32_t n, const uin
 // voxtree.rs:597-705 (remove) build it.  Blocks nbuild.. commit height h-1.
 template <typename T, int TILE>
 __global__ __launch_bounds__(TILE) void k_set_level(
-    Pool<T> P, const ChunkDev* chunks, LevelInfo L, const uint64_t* doff, uint32_t n, const int32_t* xyz,
+    Pool<T> P, const ChunkDev* chunks, LevelInfo L, const int32_t* xyz,
     const T* vals, const uint64_t* rec, const uint32_t* meta, const uint64_t* res_prev,
     const uint64_t* cand_id_prev, uint64_t* res, Cands K, uint32_t* tile_cnt) {
     __shared__ uint32_t s_cnt;
@@ -2732,7 +2737,7 @@ __global__ __launch_bounds__(TILE) void k_set_level(
                     cur = kEmpty;
                 }
             } else {
-                uint64_t r = res_prev[doff[(uint64_t)(L.h - 1) * n + c]];
+                uint64_t r = res_prev[G.prev + (slot - G.base)];
                 cur = res_is_pending(r) ? cand_id_prev[(uint32_t)r] : r;
             }
             if (cur != kInvalid && v != 0) {
