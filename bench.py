@@ -1383,9 +1383,8 @@ def bench_calib(a):
 def bench_edits(a):
     """Edit lists through vx_trees_apply_edits: the served stream's sphere edits (radius
     uniform 2-40 voxels, random centres, u16 ids, a quarter carving) on the 16384-tree
-    depth-5 u16 world, --spheres per apply.  The device radix sort of the edits by (tree,
-    Morton path), the scatter into Batch buffers and the apply are timed per kernel (HIP
-    events on the library's stream)."""
+    depth-5 u16 world, --spheres per apply.  The making of the Batch buffers (the last write
+    to each voxel) and the apply are timed per kernel (HIP events on the library's stream)."""
     import torch
     from voxelis_amd import api, serve
     from voxelis_amd import workloads as W
@@ -1428,19 +1427,16 @@ def bench_edits(a):
     world.it.sync()
     E = sum(b[3] for b in batches[a.warmup:])
     kern = {k: round(v[0] / a.steps, 4) for k, v in sorted(prof.items(), key=lambda kv: -kv[1][0])}
-    sort_ms = sum(prof[k][0] for k in ("k_sort_hist", "k_sort_scan", "k_sort_scatter") if k in prof) / a.steps
-    passes = prof.get("k_sort_scatter", (0, 0))[1] / a.steps
+    batch_ms = sum(prof[k][0] for k in ("k_edit_mark", "k_edit_build") if k in prof) / a.steps
     res = {"edits_per_apply": E / a.steps, "trees_per_apply": float(np.mean([b[4] for b in batches[a.warmup:]])),
            "edits_per_s": E / wall, "ms_per_apply": 1e3 * wall / a.steps,
-           "sort_ms_per_apply": sort_ms, "sort_passes": passes,
-           "sort_keys_per_s": (E / a.steps) / (sort_ms / 1e3) if sort_ms else None,
-           "sort_bytes_per_key_per_pass": 2 * (8 + 4) + 8,
+           "batch_ms_per_apply": batch_ms, "batch_edits_per_s": (E / a.steps) / (batch_ms / 1e3) if batch_ms else None,
            "kernels_ms_per_apply": kern,
            "note": "each apply runs with profiling events around every kernel (launched one by one)"}
     print(f"[edits] {E / a.steps / 1e6:.2f} M edits per apply over {res['trees_per_apply']:.0f} trees: "
-          f"{res['edits_per_s'] / 1e6:.1f} M edits/s, {res['ms_per_apply']:.3f} ms per apply; sort {sort_ms:.3f} ms "
-          f"({passes:.0f} passes, {res['sort_keys_per_s'] / 1e9:.2f} G keys/s)", file=sys.stderr, flush=True)
-    print(json.dumps({"metric": "edit lists: sorted on the device and applied", "config": {
+          f"{res['edits_per_s'] / 1e6:.1f} M edits/s, {res['ms_per_apply']:.3f} ms per apply; "
+          f"Batch buffers {batch_ms:.3f} ms", file=sys.stderr, flush=True)
+    print(json.dumps({"metric": "edit lists: Batch buffers made on the device and applied", "config": {
         "workload": f"{a.spheres} sphere edits per apply (radius 2-40, u16 ids, a quarter carving) on the "
                     f"16384-tree depth-5 u16 world"}, "results": res}))
 

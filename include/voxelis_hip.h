@@ -174,8 +174,8 @@ int vx_tree_apply_batch_host(vx_interner* h, uint64_t* root, const vx_batch_view
  * xyz[3e..3e+3) / values[e] for e in [edit_offsets[t], edit_offsets[t+1]) in
  * submission order, as if Batch::just_set (core/batch.rs:145-175) had been called
  * for each on a fresh Batch of that tree; a tree with no edits is not applied
- * (status 0).  The edits are radix-sorted by (tree, Morton path) on the device;
- * the last write to a voxel wins.  depths and edit_offsets (n+1 entries) are
+ * (status 0).  The last write to a voxel wins (the device takes the maximum of the
+ * submission indices of each voxel).  depths and edit_offsets (n+1 entries) are
  * host arrays; roots, xyz, values and status are device arrays.  A coordinate
  * outside the tree fails that tree with VX_E_RANGE (the reference's Vec index
  * panics).  Asynchronous. */

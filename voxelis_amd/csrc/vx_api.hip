@@ -104,12 +104,12 @@ struct LevelBufs {
 enum KernelId : uint32_t {
     KID_BEGIN = 0, KID_PREPARE, KID_DRY_LEAVES, KID_BRICK_BUILD, KID_PROBE_BRICKS, KID_LEVEL_BUILD, KID_PROBE_UPPER,
     KID_COMMIT, KID_END_ALLOC, KID_GC, KID_GET, KID_CANON, KID_FILL, KID_TO_VEC, KID_SET_DESCEND, KID_SET_LEVEL,
-    KID_GET_GROUPED, KID_EDIT_KEYS, KID_SORT_HIST, KID_SORT_SCAN, KID_SORT_SCATTER, KID_EDIT_SCATTER, KID_COUNT
+    KID_GET_GROUPED, KID_EDIT_MARK, KID_EDIT_BUILD, KID_COUNT
 };
 const char* const kKernelNames[KID_COUNT] = {
     "k_begin", "k_prepare", "k_dry_leaves", "k_brick_build", "k_probe[bricks]", "k_level_build", "k_probe[upper]",
     "k_commit", "k_end_alloc", "k_gc_round", "k_get", "k_canon", "k_fill", "k_to_vec", "k_set_descend", "k_set_level",
-    "k_get_grouped", "k_edit_keys", "k_sort_hist", "k_sort_scan", "k_sort_scatter", "k_edit_scatter"};
+    "k_get_grouped", "k_edit_mark", "k_edit_build"};
 
 struct Prof {
     bool on = false;
@@ -162,8 +162,8 @@ struct vx_interner {
     // workspace
     Grow records, gc_front[2], stage, scratch, drift, undo, owners;
     Grow set_rec, set_meta;  // single-voxel set: the recorded path of every tree
-    // edit-list path: zero-kept dense Batch buffers, sort buffers, tree records
-    Grow edit_ws, edit_keys[2], edit_order[2], edit_tmp, edit_trees, edit_first, edit_status;
+    // edit lists: the winners of every voxel and the dirty cells (kept zero), Batch buffers
+    Grow edit_win, edit_dirty, edit_masks, edit_values;
     LevelBufs lv[kLevels + 1];
     // pinned staging ring: a slot is reused only after its copies completed
     static constexpr int kRing = 8;
@@ -261,9 +261,6 @@ int err_to_status(uint32_t err) {
 
 uint64_t slots_at(uint32_t d, uint32_t h) { return 1ull << (3 * (d - h)); }
 
-// vx_batch_view.reserved value used internally for trees that are not applied
-constexpr uint8_t kViewSkip = 0x5A;
-
 hipEvent_t prof_event(vx_interner* h) {
     Prof& p = h->prof;
     if (p.used == p.pool.size()) {
@@ -301,6 +298,14 @@ struct ApplyOpts {
     // single-voxel set mode (vx_trees_set): one voxel per tree, device xyz[3n] and values[n]
     const int32_t* set_xyz = nullptr;
     const void* set_values = nullptr;
+    // edit lists: the views are the edited trees', orig[i] their index in the caller's arrays
+    // of nall trees, edits[i] their records; nedits edits (device) and nbricks workspace bricks
+    const EditTree* edits = nullptr;
+    const uint32_t* orig = nullptr;
+    size_t nall = 0;
+    uint64_t nedits = 0, nbricks = 0;
+    const int32_t* edit_xyz = nullptr;
+    const void* edit_values = nullptr;
 };
 
 constexpr unsigned kRebuildGrid = 512;
@@ -310,7 +315,7 @@ int rebuild_step(vx_interner* h, bool force, bool reinsert, const void* up_src =
 
 template <typename T, int TILE>
 int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* batches,
-                int32_t* status, const int32_t* pre_status, const ApplyOpts& opt) {
+                int32_t* status, const ApplyOpts& opt) {
     constexpr int kBR = brick_rounds<TILE>();
     hipStream_t s = h->stream;
     Pool<T> P = pool_of<T>(h);
@@ -322,7 +327,7 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     // ---- a repeated call replays its captured launch sequence
     Plan* plan = nullptr;
     uint64_t key = 0;
-    if (h->graphs && !h->prof.on && !pre_status && !setm) {
+    if (h->graphs && !h->prof.on && !opt.edits && !setm) {
         key = mix64(0x5650u ^ (uint64_t)n ^ ((uint64_t)sizeof(T) << 40));
         const uint64_t head[] = {(uint64_t)roots, (uint64_t)status, (uint64_t)opt.dry,
                                  (uint64_t)opt.alloc_limit, (uint64_t)opt.counts, (uint64_t)TILE,
@@ -365,7 +370,9 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     // records: trees with patches by depth (others first), in the caller's order within a
     // depth, then the tables; one staging buffer, one upload
     const size_t chunk_bytes = n * sizeof(ChunkDev);
-    const size_t tab_bytes = 2 * (kLevels + 1) * sizeof(void*) + (kLevels + 1) * sizeof(Cands) + sizeof(SlotMap);
+    const size_t map_at = 2 * (kLevels + 1) * sizeof(void*) + (kLevels + 1) * sizeof(Cands);
+    const size_t edits_at = map_at + sizeof(SlotMap);
+    const size_t tab_bytes = edits_at + (opt.edits ? n * sizeof(EditTree) : 0);
     const size_t stage_bytes = (chunk_bytes + tab_bytes + 15) / 16 * 16;
     if (!pinned_ensure(h, stage_bytes)) return VX_E_HIP;
     ChunkDev* hc = (ChunkDev*)h->h_pinned;
@@ -373,7 +380,7 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     uint64_t old_nodes = 0;       // a bound of the branch nodes the call can free
     struct Run { uint32_t start, count, depth; };
     const auto depth_key = [&](const vx_batch_view& b, int32_t st) -> uint32_t {
-        return b.has_patches && st == 0 && b.reserved != kViewSkip ? b.depth : 0u;
+        return b.has_patches && st == 0 ? b.depth : 0u;
     };
     uint32_t of_depth[kLevels + 1] = {0}, at[kLevels + 1] = {0};
     for (size_t i = 0; i < n; i++) of_depth[depth_key(batches[i], status_of(batches[i]))]++;
@@ -394,13 +401,15 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
         C.values = b.values;
         C.fill = b.fill_value & (sizeof(T) == 1 ? 0xFFull : sizeof(T) == 2 ? 0xFFFFull : 0xFFFFFFFFull);
         C.root_in = C.init = 0;
-        C.orig = (uint32_t)i;
+        C.orig = opt.orig ? opt.orig[i] : (uint32_t)i;
+        C.sub = (uint32_t)i;
+        C.pad = 0;
         C.depth = b.depth;
         C.has_fill = b.has_fill ? 1 : 0;
-        C.skip = b.reserved == kViewSkip ? 1 : 0;
+        C.skip = 0;
         C.status = C.status0 = st;
-        C.has_patches = key != 0 || (b.has_patches && st == 0 && !C.skip) ? 1 : 0;
-        if (st == 0 && !C.skip) {
+        C.has_patches = b.has_patches && st == 0 ? 1 : 0;
+        if (st == 0) {
             dall = std::max<uint32_t>(dall, b.depth);
             old_nodes += setm || b.depth == 0 ? b.depth + 1u : slots_at(b.depth, 1) + slots_at(b.depth, 1) / 4;
         }
@@ -408,7 +417,8 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     }
     LevelInfo L[kLevels + 1];
     std::memset(L, 0, sizeof(L));
-    SlotMap* hmap = (SlotMap*)((char*)hc + chunk_bytes + 2 * (kLevels + 1) * sizeof(void*) + (kLevels + 1) * sizeof(Cands));
+    SlotMap* hmap = (SlotMap*)((char*)hc + chunk_bytes + map_at);
+    if (opt.edits && n) std::memcpy((char*)hc + chunk_bytes + edits_at, opt.edits, n * sizeof(EditTree));
     std::memset(hmap, 0, sizeof(SlotMap));
     for (const Run& r : runs) hmap->start[r.depth] = r.start;
     std::vector<Run> lruns[kLevels + 1];
@@ -507,6 +517,7 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     uint64_t* const* dcid = dres + (kLevels + 1);
     P.levels = (const Cands*)(dres + 2 * (kLevels + 1));
     const SlotMap* dmap = (const SlotMap*)(P.levels + kLevels + 1);
+    EditTree* dedits = opt.edits ? (EditTree*)(dmap + 1) : nullptr;
     // a captured sequence keeps its records; a dry run has no table step to bring them along
     if (plan || opt.dry) {
         HIPCHK(hipMemcpyAsync(records.ptr, hc, stage_bytes, hipMemcpyHostToDevice, s));
@@ -570,10 +581,21 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
         int rc = launch_set();
         if (rc) return rc;
     } else {
+    if (dedits) {
+        // runs of up to 2048 edits per block, while there are eight blocks for each CU
+        const uint32_t per = (uint32_t)std::min<uint64_t>(8, std::max<uint64_t>(1, opt.nedits / (2048 * 256)));
+        VX_LAUNCH(h, KID_EDIT_MARK, k_edit_mark, grid_for(std::max<uint64_t>(opt.nedits / per, opt.nall)), 256, opt.nedits, per, dedits,
+                  (uint32_t)n, opt.edit_xyz, (uint32_t*)h->edit_win.ptr, (uint8_t*)h->edit_dirty.ptr, (uint32_t)opt.nall,
+                  status, P.per_tree);
+        if (opt.nbricks)
+            VX_LAUNCH(h, KID_EDIT_BUILD, k_edit_build<T>, grid_for(opt.nbricks), 256, opt.nbricks,
+                      (const T*)opt.edit_values, (uint32_t*)h->edit_win.ptr, (uint8_t*)h->edit_dirty.ptr,
+                      (uint16_t*)h->edit_masks.ptr, (T*)h->edit_values.ptr);
+    }
     // chunk set-up, plus the old-tree descent over the level-3 slots in extra blocks
     unsigned np = grid_for(n);
     unsigned nd = L[3].nslots ? grid_for(L[3].nslots) : 0u;
-    VX_LAUNCH(h, KID_PREPARE, k_prepare<T>, np + nd + nre, kBlock, P, dchunks, (uint32_t)n, roots, pre_status, np,
+    VX_LAUNCH(h, KID_PREPARE, k_prepare<T>, np + nd + nre, kBlock, P, dchunks, (uint32_t)n, roots, dedits, np,
               nd, L[3], dmap, O);
     unsigned t1 = (unsigned)ntiles[1];
     if (dmax >= 2 && br == kBR)
@@ -688,117 +710,66 @@ uint64_t tombstones_of(const Ctl& c, int which = ST_TOMB) {
 
 template <typename T>
 int apply_impl(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* batches,
-               int32_t* status, const int32_t* pre_status = nullptr, const ApplyOpts& opt = ApplyOpts()) {
+               int32_t* status, const ApplyOpts& opt = ApplyOpts()) {
     int rc = VX_OK;
     switch (h->tune.tile) {
-        case 128: rc = apply_tiled<T, 128>(h, n, roots, batches, status, pre_status, opt); break;
-        case 512: rc = apply_tiled<T, 512>(h, n, roots, batches, status, pre_status, opt); break;
-        default: rc = apply_tiled<T, 256>(h, n, roots, batches, status, pre_status, opt); break;
+        case 128: rc = apply_tiled<T, 128>(h, n, roots, batches, status, opt); break;
+        case 512: rc = apply_tiled<T, 512>(h, n, roots, batches, status, opt); break;
+        default: rc = apply_tiled<T, 256>(h, n, roots, batches, status, opt); break;
     }
     return rc;
 }
 
+// A workspace array that is zero between calls.
+int ensure_zero(vx_interner* h, Grow& g, size_t bytes) {
+    if (bytes <= g.cap) return VX_OK;
+    if (!g.ensure(bytes)) return VX_E_HIP;
+    if (hipMemsetAsync(g.ptr, 0, g.cap, h->stream) == hipSuccess) return VX_OK;
+    g.release();
+    return VX_E_HIP;
+}
+
+// Only the trees with edits are planned, uploaded and applied.
 template <typename T>
 int apply_edits_impl(vx_interner* h, size_t n, uint64_t* roots, const uint8_t* depths,
                      const uint64_t* offsets, const int32_t* xyz, const void* values, int32_t* status,
-                     const ApplyOpts& opt = ApplyOpts()) {
-    hipStream_t s = h->stream;
-    uint64_t E = offsets[n];
-    std::vector<EditTree> trees(n);
-    std::vector<uint64_t> first(n);
-    uint64_t mbytes = 0, vcount = 0;
+                     const ApplyOpts& opts = ApplyOpts()) {
+    ApplyOpts opt = opts;
+    std::vector<EditTree> trees;
+    std::vector<uint32_t> orig;
+    uint64_t nvox = 0;
+    if (offsets[n] >= 0xFFFFFFFFull) return VX_E_INVALID_ARG;  // submission indices are 32 bits
     for (size_t t = 0; t < n; t++) {
-        uint32_t d = depths[t];
         if (offsets[t + 1] < offsets[t]) return VX_E_INVALID_ARG;
-        uint64_t P = d > 0 ? (1ull << (3 * (d - 1))) : 1ull;
-        trees[t].first = offsets[t];
-        trees[t].depth = d;
-        trees[t].status = 0;
-        bool has = offsets[t + 1] > offsets[t];
-        if (d > (uint32_t)kMaxDepth || (has && d < 2)) trees[t].status = VX_E_DEPTH;
-        trees[t].mbase = mbytes;
-        trees[t].vbase = vcount;
-        first[t] = offsets[t];
-        if (d <= (uint32_t)kMaxDepth) {
-            mbytes += ((2 * P + 255) / 256) * 256;
-            vcount += ((8 * P + 255) / 256) * 256;
+        if (offsets[t + 1] == offsets[t]) continue;
+        const uint32_t d = depths[t];
+        EditTree e{t ? offsets[t] : 0, ~0ull, d, 0};  // (edits before the first tree's are its own)
+        if (d >= 2 && d <= (uint32_t)kMaxDepth) {  // (others fail with VX_E_DEPTH when planned)
+            e.vbase = nvox;
+            nvox += std::max<uint64_t>(slots_at(d, 0), 512);
         }
+        trees.push_back(e);
+        orig.push_back((uint32_t)t);
     }
-    size_t ws_bytes = mbytes + vcount * sizeof(T);
-    if (ws_bytes > h->edit_ws.cap) {
-        if (!h->edit_ws.ensure(ws_bytes)) return VX_E_HIP;
-        HIPCHK(hipMemsetAsync(h->edit_ws.ptr, 0, h->edit_ws.cap, s));  // kept zero from here on
-    }
-    uint8_t* mws = (uint8_t*)h->edit_ws.ptr;
-    T* vws = (T*)(mws + mbytes);
-    uint64_t En = std::max<uint64_t>(E, 1);
-    if (!h->edit_keys[0].ensure(En * 8) || !h->edit_keys[1].ensure(En * 8) ||
-        !h->edit_order[0].ensure(En * 4) || !h->edit_order[1].ensure(En * 4) ||
-        !h->edit_trees.ensure(n * sizeof(EditTree)) || !h->edit_first.ensure(n * 8) ||
-        !h->edit_status.ensure(n * 4))
-        return VX_E_HIP;
-    EditTree* dtrees = (EditTree*)h->edit_trees.ptr;
-    uint64_t* dfirst = (uint64_t*)h->edit_first.ptr;
-    int32_t* dpre = (int32_t*)h->edit_status.ptr;
-    // the tree records travel through a pinned staging slot, reused only once these
-    // copies completed (no wait for earlier work on the stream)
-    if (!pinned_ensure(h, n * (sizeof(EditTree) + 8))) return VX_E_HIP;
-    std::memcpy(h->h_pinned, trees.data(), n * sizeof(EditTree));
-    std::memcpy((char*)h->h_pinned + n * sizeof(EditTree), first.data(), n * 8);
-    HIPCHK(hipMemcpyAsync(dtrees, h->h_pinned, n * sizeof(EditTree), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dfirst, (char*)h->h_pinned + n * sizeof(EditTree), n * 8, hipMemcpyHostToDevice, s));
-    pinned_release(h);
-    uint64_t* k0 = (uint64_t*)h->edit_keys[0].ptr;
-    uint64_t* k1 = (uint64_t*)h->edit_keys[1].ptr;
-    uint32_t* o0 = (uint32_t*)h->edit_order[0].ptr;
-    uint32_t* o1 = (uint32_t*)h->edit_order[1].ptr;
-    unsigned tree_bits = 1;
-    while ((1ull << tree_bits) <= n) tree_bits++;
-    unsigned end_bit = kPathBits + tree_bits;
-    if (E > 0) {
-        VX_LAUNCH(h, KID_EDIT_KEYS, k_edit_keys, grid_for(E), kBlock, E, dfirst, (uint32_t)n, dtrees, xyz, k0, o0);
-        // stable LSD radix sort, 8 bits per pass, ping-ponging between the two buffers
-        const unsigned G = (unsigned)std::min<uint64_t>(2048, (E + kSortBlock - 1) / kSortBlock);
-        const uint64_t per = (E + G - 1) / G;
-        const uint32_t M = 256u * G;  // digit counts of a pass, digit-major
-        const uint32_t ntile = (M + kScanTileN - 1) / kScanTileN;
-        if (!h->edit_tmp.ensure((size_t)(M + ntile + 1) * 4)) return VX_E_HIP;
-        uint32_t* hist = (uint32_t*)h->edit_tmp.ptr;
-        uint32_t* tile_off = hist + M;
-        for (unsigned shift = 0; shift < end_bit; shift += 8) {
-            VX_LAUNCH(h, KID_SORT_HIST, k_sort_hist, G, kSortBlock, k0, E, per, shift, hist);
-            VX_LAUNCH(h, KID_SORT_SCAN, k_sort_scan_tiles, ntile, kSortScanBlock, hist, M, tile_off);
-            VX_LAUNCH(h, KID_SORT_SCAN, k_sort_scan, 1, kSortScanBlock, tile_off, ntile);
-            VX_LAUNCH(h, KID_SORT_SCATTER, k_sort_scatter, G, kSortBlock, k0, o0, k1, o1, E, per, shift, hist,
-                      tile_off);
-            std::swap(k0, k1);
-            std::swap(o0, o1);
-        }
-        std::swap(k0, k1);  // the sorted pairs are in (k1, o1)
-        std::swap(o0, o1);
-        VX_LAUNCH(h, KID_EDIT_SCATTER, k_edit_scatter<T>, grid_for(E), kBlock, E, (uint32_t)n, dtrees, k1, o1,
-                  (const T*)values, mws, vws, false);
-    }
-    // per-tree failures recorded by k_edit_keys go in as pre-statuses
-    k_edit_status<<<grid_for(n), kBlock, 0, s>>>((uint32_t)n, dtrees, dpre);
-    std::vector<vx_batch_view> views(n);
-    for (size_t t = 0; t < n; t++) {
-        vx_batch_view& v = views[t];
-        std::memset(&v, 0, sizeof(v));
-        v.depth = depths[t];
-        v.has_patches = offsets[t + 1] > offsets[t] ? 1 : 0;
-        if (!v.has_patches) v.reserved = kViewSkip;
-        v.masks = mws + trees[t].mbase;
-        v.values = vws + trees[t].vbase;
-    }
-    int rc = apply_impl<T>(h, n, roots, views.data(), status, dpre, opt);
-    // the touched bricks are cleared again on every path, a failed apply included, so
-    // the workspace stays zero for the next call
-    if (E > 0)
-        VX_LAUNCH(h, KID_EDIT_SCATTER, k_edit_scatter<T>, grid_for(E), kBlock, E, (uint32_t)n, dtrees, k1, o1,
-                  (const T*)values, mws, vws, true);
+    int rc = ensure_zero(h, h->edit_win, nvox * 4);
+    if (!rc) rc = ensure_zero(h, h->edit_dirty, nvox / 512);
     if (rc) return rc;
-    return hipGetLastError() == hipSuccess ? VX_OK : VX_E_HIP;
+    if (!h->edit_masks.ensure(nvox / 4) || !h->edit_values.ensure(nvox * sizeof(T))) return VX_E_HIP;
+    std::vector<vx_batch_view> views(trees.size());
+    for (size_t i = 0; i < trees.size(); i++) {
+        const uint64_t v0 = trees[i].vbase == ~0ull ? 0 : trees[i].vbase;
+        views[i] = vx_batch_view{(const uint8_t*)h->edit_masks.ptr + v0 / 4, (const T*)h->edit_values.ptr + v0, 0,
+                                 (uint8_t)trees[i].depth, 0, 1, 0};
+    }
+    static const EditTree none{};
+    opt.edits = trees.empty() ? &none : trees.data();
+    opt.orig = orig.data();
+    opt.nall = n;
+    opt.nedits = trees.empty() ? 0 : offsets[n];
+    opt.nbricks = nvox / 8;
+    opt.edit_xyz = xyz;
+    opt.edit_values = values;
+    return apply_impl<T>(h, trees.size(), roots, views.data(), status, opt);
 }
 
 template <typename T>
@@ -1002,8 +973,7 @@ int vx_interner_destroy(vx_interner* h) {
     h->owners.release();
     for (Plan& pl : h->plans) pl.release();
     if (h->cap_stream) (void)hipStreamDestroy(h->cap_stream);
-    for (Grow* g : {&h->edit_ws, &h->edit_keys[0], &h->edit_keys[1], &h->edit_order[0], &h->edit_order[1],
-                    &h->edit_tmp, &h->edit_trees, &h->edit_first, &h->edit_status})
+    for (Grow* g : {&h->edit_win, &h->edit_dirty, &h->edit_masks, &h->edit_values})
         g->release();
     for (auto& b : h->lv) {
         b.res.release();
@@ -1168,7 +1138,7 @@ int vx_trees_set(vx_interner* h, size_t n, uint64_t* roots, const uint8_t* depth
     ApplyOpts o;
     o.set_xyz = xyz;
     o.set_values = values;
-    return VX_WIDTH_DISPATCH(h, apply_impl, h, n, roots, views.data(), status, nullptr, o);
+    return VX_WIDTH_DISPATCH(h, apply_impl, h, n, roots, views.data(), status, o);
 }
 
 int opts_of(const vx_interner* h, const vx_apply_opts* o, ApplyOpts* out) {
@@ -1194,7 +1164,7 @@ int vx_trees_apply_batches_ex(vx_interner* h, size_t n, uint64_t* roots, const v
     ApplyOpts o;
     int rc = opts_of(h, opts, &o);
     if (rc) return rc;
-    return VX_WIDTH_DISPATCH(h, apply_impl, h, n, roots, batches, status, nullptr, o);
+    return VX_WIDTH_DISPATCH(h, apply_impl, h, n, roots, batches, status, o);
 }
 
 int vx_trees_apply_edits_ex(vx_interner* h, size_t n, uint64_t* roots, const uint8_t* depths,

@@ -147,10 +147,20 @@ struct ChunkDev {  // 8-byte aligned; depth .. skip form one dword (read as such
     uint8_t has_patches;
     uint8_t skip;  // not applied at all (an edit-list tree without edits)
     int32_t status0;  // status before the launch (a replayed launch starts from it)
+    uint32_t sub;     // index among the call's records as the caller listed them (its EditTree)
+    uint32_t pad;
 };
 static_assert(offsetof(ChunkDev, depth) % 4 == 0 && offsetof(ChunkDev, has_fill) == offsetof(ChunkDev, depth) + 1 &&
                   offsetof(ChunkDev, has_patches) == offsetof(ChunkDev, depth) + 2,
               "the flag bytes are read as one dword");
+
+// One edited tree of an edit-list call.
+struct EditTree {
+    uint64_t first;  // its first edit
+    uint64_t vbase;  // its first voxel in the workspace (a multiple of 512); ~0: rejected
+    uint32_t depth;
+    int32_t status;
+};
 
 // Slot space of one level: groups of trees of equal depth, each tree owning
 // 8^(depth-h) consecutive slots at height h (h = 1: bricks, h = depth: root).

@@ -759,7 +759,7 @@ __device__ inline void reinsert_body(const Pool<T>& P, uint32_t b, uint32_t nb) 
 // the blocks after them the table's re-insertion when it is due (nothing here reads it).
 template <typename T>
 __global__ void k_prepare(Pool<T> P, ChunkDev* chunks, uint32_t n, const uint64_t* roots,
-                          const int32_t* pre_status, uint32_t nprep, uint32_t ndesc, LevelInfo L3,
+                          const EditTree* edits, uint32_t nprep, uint32_t ndesc, LevelInfo L3,
                           const SlotMap* M, OldNodes O) {
     if (blockIdx.x >= nprep + ndesc) {
         reinsert_body(P, blockIdx.x - nprep - ndesc, gridDim.x - nprep - ndesc);
@@ -782,7 +782,7 @@ __global__ void k_prepare(Pool<T> P, ChunkDev* chunks, uint32_t n, const uint64_
         // a depth-2 tree's height-2 node is its root (deeper trees: the descent)
         if (C.depth == 2 && C.has_patches && !C.has_fill) O.at[2][slot_of(M, 2, (uint32_t)c, 2)] = C.root_in;
         if (P.per_tree) P.per_tree[C.orig] = 0;
-        if (pre_status && pre_status[C.orig] < 0 && C.status >= 0) C.status = pre_status[C.orig];
+        if (edits && edits[C.sub].status < 0 && C.status >= 0) C.status = edits[C.sub].status;
         if (C.status >= 0 && C.has_fill) {
             const uint32_t v = (uint32_t)C.fill;
             const uint32_t li = leaf_index(P, v);
