@@ -106,31 +106,37 @@ constexpr int kStatStripes = 64;
 // TILE = 128, 256 or 512, a tuning choice); a tile's candidates are compacted into
 // its own region of the candidate arrays.
 
+// Counters that every block of a launch updates have a cache line each: an update of one
+// does not wait behind the others', or behind the loads of the fields that every block reads.
+struct alignas(128) HotCounter {
+    uint32_t v;
+};
+
 struct Ctl {
-    uint32_t free_top;    // entries on the free stack
+    // read by every block, changed between launches
     uint32_t next_index;  // bump cursor (interner/macros.rs:16-34)
     uint32_t free_top0;   // snapshot at the start of a launch sequence
     uint32_t next0;
-    uint32_t alloc_count;  // branch nodes allocated in the current sequence (ranks after its new leaves)
-    uint32_t err;
-    uint32_t n_new_leaves;  // leaves created in the current sequence: allocation ranks [0, n_new_leaves)
-    uint32_t epoch;         // counts launch sequences: marks the leaf claims of the current one
+    uint32_t epoch;       // counts launch sequences: marks the leaf claims of the current one
     uint64_t live_leaves;
     uint64_t live_branches;
     uint32_t rebuild;   // this call rebuilds the pattern table (bit 0) and the i32 leaf table (bit 1)
     uint32_t rebuilds;  // table rebuilds so far
-    uint32_t n_drift;  // queued reference-count corrections of the reference's quirks
-    uint32_t dry_owners;      // dry run: branch keys that would be new
-    uint32_t dry_new_leaves;  // dry run: leaves that would be new
+    // rare events
+    uint32_t err;
     uint32_t abort_;          // this apply could not allocate: 1 capacity, 2 reservation
     uint32_t n_undo;          // entries of the undo log (reference-count deltas applied)
     uint32_t h1_fail;         // a tree of this apply failed in the brick pass (leaf-brick panic)
     uint32_t n_need;          // i32: values a dry run requested (need_list entries)
-    uint32_t ncand[kLevels + 1];
-    uint32_t gc_count[kLevels + 2];
-    uint32_t pad1;
+    uint32_t dry_new_leaves;  // dry run: leaves that would be new
+    alignas(128) uint32_t free_top;      // entries on the free stack
+    alignas(128) uint32_t alloc_count;   // branch nodes allocated in the current sequence (ranks after its new leaves)
+    alignas(128) uint32_t n_new_leaves;  // leaves created in the current sequence: allocation ranks [0, n_new_leaves)
+    alignas(128) uint32_t n_drift;       // queued reference-count corrections of the reference's quirks
+    alignas(128) uint32_t dry_owners;    // dry run: branch keys that would be new
+    HotCounter gc_count[kLevels + 2];
     // statistics, striped over 64 cache lines by block index (summed when read)
-    uint64_t st[kStatStripes][32];
+    alignas(128) uint64_t st[kStatStripes][32];
 };
 
 // Per-tree record of one apply launch sequence (trees sorted by depth on the host).

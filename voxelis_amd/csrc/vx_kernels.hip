@@ -356,7 +356,7 @@ __device__ inline uint64_t leaf_now(const Pool<T>& P, uint32_t v) {
 // A new leaf used to be requested here and created by one block of a later launch, and its
 // bricks rebuilt by a third one: a new id written everywhere (64 x 64 terrain trees, u8)
 // took 1.24 ms of brick passes and takes 0.14 ms here; 0.85 M new 32-bit ids took 56 ms of
-// creation and as much again to take their requests back, and are 1.2 ms of the 1.6 ms pass.
+// creation and as much again to take their requests back; the whole brick pass is 0.47 ms now.
 //
 // A lane that claims a value (its epoch word, or the i32 table's slot) publishes the id
 // without waiting for anyone, and every claim of a wavefront is published before one of its
@@ -619,8 +619,7 @@ __device__ inline void ctl_begin(Ctl* ctl) {
         ctl->abort_ = 0;
         ctl->n_undo = 0;
         ctl->h1_fail = 0;
-        for (int i = 0; i <= kLevels; i++) ctl->ncand[i] = 0;
-        for (int i = 0; i < kLevels + 2; i++) ctl->gc_count[i] = 0;
+        for (int i = 0; i < kLevels + 2; i++) ctl->gc_count[i].v = 0;
     }
 }
 
@@ -944,7 +943,7 @@ __device__ inline int brick_work(const Pool<T>& P, const ChunkDev& C, uint32_t m
     }
     bool split = bid_is_leaf(base);
     uint32_t split_value = 0;
-    if (split) split_value = fill_split ? (uint32_t)C.fill : (uint32_t)P.values[bid_index(base)];
+    if (split && sizeof(T) <= 2) split_value = fill_split ? (uint32_t)C.fill : (uint32_t)P.values[bid_index(base)];
     // A completely written brick replaces every child of an old brick-level node: its key
     // is (the leaves of its values, types = mask = 0xFF) whatever the old children were, so
     // they are not loaded.  The old children only tell whether the brick is unchanged (every
@@ -970,7 +969,8 @@ __device__ inline int brick_work(const Pool<T>& P, const ChunkDev& C, uint32_t m
         // is that leaf (the children of a brick are leaves)
         uint64_t lid = lids[i];
         if (ch[i] != kEmpty) {
-            bool same = split ? split_value == v[i] : (lid != kEmpty && ch[i] == lid);
+            // (i32: v holds leaf indices by now, and a value's leaf is its identity too)
+            bool same = split && sizeof(T) <= 2 ? split_value == v[i] : (lid != kEmpty && ch[i] == lid);
             if (same) continue;
         }
         if (lid == kEmpty) {
@@ -1186,6 +1186,13 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
     }
     __syncthreads();
     const uint32_t nq = s_nq;
+    // i32: one round's edited voxels (lane << 3 | slot), whose leaves are looked up, and
+    // created, by a lane each: taken slot by slot, a brick of one or two edits makes every
+    // wavefront wait for eight look-ups in a row (0.87 M scattered voxels in 333 trees of
+    // 64^3, all ids new: a pass of 1.58 ms, 1.31 so, 0.47 with the counters in lines of their
+    // own)
+    __shared__ uint16_t s_list[sizeof(T) == 4 ? TILE * 8 : 1];
+    __shared__ uint32_t s_nl;
     // the queue's rounds; bricks that miss a leaf are left out, and once their leaves were
     // created (by this block or another) they alone are taken by a second pass
     for (int pass = 0; pass < 2; pass++) {
@@ -1204,7 +1211,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
             mm = s_m[q];
             const Vox8 w = s_v[q];
             const uint64_t upq = s_up[q];
-            uint32_t v[8];
+            [[maybe_unused]] uint32_t v[8];
             load8<T>((const T*)&w, v);
             const GroupPos G = group_of(L, BG, slot);
             const uint64_t local = slot - G.base;
@@ -1223,12 +1230,6 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
             if constexpr (sizeof(T) <= 2) {
 #pragma unroll
                 for (int i = 0; i < 8; i++) lids[i] = leaf_ids[v[i]];
-            } else {
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    lids[i] = kEmpty;
-                    if ((mm >> i) & 1u) lids[i] = pass == 0 ? leaf_lookup(P, leaf_ids, v[i]) : leaf_now(P, v[i]);
-                }
             }
             const bool up_branch = D >= 2 && upq != kEmpty && !bid_is_leaf(upq);
             const bool up_ok = up_branch && bid_index(upq) < P.capacity;
@@ -1266,10 +1267,67 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
                 P.ctl->h1_fail = 1u;
                 live = false;
             } else {
+                need = all_same ? 1u : mm;
+                if constexpr (sizeof(T) <= 2) {
 #pragma unroll
-                for (int i = 0; i < 8; i++) need |= (lids[i] == kEmpty ? 1u : 0u) << i;
-                need &= all_same ? 1u : mm;
+                    for (int i = 0; i < 8; i++) need &= ~((lids[i] != kEmpty ? 1u : 0u) << i);
+                }
             }
+        }
+        if constexpr (sizeof(T) == 4) {
+            // the voxels' values give way to their leaves' indices (0: none)
+            if (threadIdx.x == 0) s_nl = 0;
+            __syncthreads();
+            {
+                uint32_t x = (uint32_t)__popc(need);
+                const uint32_t cnt = x;
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const uint32_t y = __shfl_up(x, o);
+                    if ((int)__lane_id() >= o) x += y;
+                }
+                uint32_t at = 0;
+                if (__lane_id() == 63) at = atomicAdd(&s_nl, x);
+                at = __shfl(at, 63) + x - cnt;
+                for (uint32_t m = need; m; m &= m - 1)
+                    s_list[at++] = (uint16_t)(threadIdx.x << 3 | ((uint32_t)__ffs(m) - 1u));
+            }
+            __syncthreads();
+            const uint32_t nl = s_nl;
+            for (uint32_t k0 = 0; k0 < nl; k0 += TILE) {  // uniform
+                const uint32_t k = k0 + threadIdx.x;
+                uint32_t idx = 0;
+                T* cell = nullptr;
+                if (k < nl) {
+                    cell = (T*)&s_v[(uint32_t)r * TILE + (s_list[k] >> 3)] + (s_list[k] & 7u);
+                    idx = leaf_index(P, (uint32_t)*cell);
+                    if (idx == 0 && P.dry) idx = P.capacity + leaf_request(P, (uint32_t)*cell);
+                }
+                const bool miss = k < nl && idx == 0;
+                if (__ballot(miss)) {
+                    const uint32_t vv = miss ? (uint32_t)*cell : 0u;
+                    leaf_ensure(P, miss ? 1u : 0u, 1, [&](int) { return vv; });
+                    if (miss) idx = bid_index(leaf_now(P, vv));
+                }
+                if (cell) {
+                    *cell = (T)idx;
+                    if (s_idx[(uint32_t)r * TILE + (s_list[k] >> 3)] & kSame)
+                        for (int i = 1; i < 8; i++) cell[i] = (T)idx;
+                }
+            }
+            __syncthreads();
+            if (live) {
+                const Vox8 w = s_v[q];
+                uint32_t ix[8];
+                load8<T>((const T*)&w, ix);
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const bool on = (need >> i) & 1u && ix[i] != 0;
+                    const uint32_t g = P.tmg[on && ix[i] < P.capacity ? ix[i] : 0u];
+                    lids[i] = on ? make_leaf(ix[i], ix[i] < P.capacity ? tmg_gen(g) : 0u) : kEmpty;
+                }
+            }
+            need = 0;
         }
         // (a leaf created in this launch is seen past the caches)
         if (__ballot(need != 0)) {
@@ -1365,7 +1423,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
         tile_count(s_st, 3, follow);
     }
     __syncthreads();
-    if (!s_miss) break;  // uniform
+    if (sizeof(T) == 4 || !s_miss) break;  // uniform
     if (pass == 0) {
         for (uint32_t q0 = 0; q0 < nq; q0 += TILE) {
             const uint32_t q = q0 + threadIdx.x;
@@ -2160,7 +2218,7 @@ __device__ inline void finalize_body(const Pool<T>& P, const ChunkDev* chunks, u
             }
             status[C.orig] = st;
         }
-        uint32_t k = wave_append(&P.ctl->gc_count[0], push);
+        uint32_t k = wave_append(&P.ctl->gc_count[0].v, push);
         if (push) gc_front[k] = bid_index(old);
     }
 }
@@ -2345,7 +2403,7 @@ __global__ __launch_bounds__(256) void k_gc_round(Pool<T> P, uint32_t round, con
     __shared__ uint32_t s_nnext, s_nfree, s_bnext, s_bfree;
     __shared__ uint32_t s_seg[kGcSegs], s_seglen[kGcSegs];  // final round: the block's runs of waiting nodes
     __shared__ unsigned long long s_leaves, s_branches, s_tombs, s_recycled;
-    uint64_t n = P.ctl->gc_count[round];
+    uint64_t n = P.ctl->gc_count[round].v;
     if (n > front_cap) n = front_cap;
     // a small front: the block's share [lo, hi), followed locally
     const bool local = final || n <= (uint64_t)gridDim.x * kGcLocalShare;
@@ -2367,7 +2425,7 @@ __global__ __launch_bounds__(256) void k_gc_round(Pool<T> P, uint32_t round, con
     // new leaves nothing references (their trees failed) are released in the first
     // round; no node that this GC visits references them
     if (leaf_cleanup) leaf_cleanup_body(P);
-    uint32_t* next_count = &P.ctl->gc_count[round + 1];
+    uint32_t* next_count = &P.ctl->gc_count[round + 1].v;
     const int lane = (int)__lane_id();
     const uint64_t below = (1ull << lane) - 1ull;
     if (local) {
@@ -2823,7 +2881,7 @@ __global__ void k_fill_prepare(Pool<T> P, uint32_t n, const uint64_t* roots, uin
             r = roots[c];
             push = r != kEmpty;
         }
-        uint32_t k = wave_append(&P.ctl->gc_count[0], push);
+        uint32_t k = wave_append(&P.ctl->gc_count[0].v, push);
         if (push) gc_front[k] = bid_index(r);
     }
 }
