@@ -696,7 +696,7 @@ int rebuild_step(vx_interner* h, bool force, bool reinsert, const void* up_src, 
     hipStream_t s = h->stream;
     k_tab_clear<<<kRebuildGrid, kBlock, 0, s>>>(h->tab, h->tslots, h->ctl, h->ltab, h->ltab ? h->lslots : 0ull,
                                                 force ? 1u : 0u, (const uint4*)up_src, (uint4*)up_dst,
-                                                up_src ? (uint32_t)(up_bytes / 16) : 0u);
+                                                up_src ? (uint32_t)(up_bytes / 16) : 0u, h->tmg, h->free_stack);
     if (reinsert) k_tab_reinsert<T><<<kRebuildGrid, kBlock, 0, s>>>(P);
     return hipGetLastError() == hipSuccess ? VX_OK : VX_E_HIP;
 }

@@ -36,8 +36,11 @@ __host__ __device__ inline bool bid_is_leaf(uint64_t id) { return (id >> 63) != 
 __host__ __device__ inline uint32_t bid_index(uint64_t id) { return (uint32_t)id; }
 // A node's types/mask word and its generation share one 32-bit column entry, so a free or
 // a commit touches one sector for both.
+// Bit 31 (generations are 15 bits) marks a node that lies on the free stack, or was allocated
+// from it and is not written yet.
+constexpr uint32_t kTmgFree = 1u << 31;
 __host__ __device__ inline uint32_t tmg_tm(uint32_t w) { return w & 0xFFFFu; }
-__host__ __device__ inline uint32_t tmg_gen(uint32_t w) { return w >> 16; }
+__host__ __device__ inline uint32_t tmg_gen(uint32_t w) { return (w >> 16) & 0x7FFFu; }
 __host__ __device__ inline uint32_t tmg_make(uint32_t tm, uint32_t gen) { return (gen << 16) | (tm & 0xFFFFu); }
 __host__ __device__ inline uint32_t bid_gen(uint64_t id) { return (uint32_t)(id >> 32) & 0x7FFFu; }
 __host__ __device__ inline uint32_t bid_tm(uint64_t id) { return (uint32_t)(id >> 47) & 0xFFFFu; }
@@ -129,11 +132,14 @@ struct Ctl {
     uint32_t h1_fail;         // a tree of this apply failed in the brick pass (leaf-brick panic)
     uint32_t n_need;          // i32: values a dry run requested (need_list entries)
     uint32_t dry_new_leaves;  // dry run: leaves that would be new
+    uint32_t free_base;       // free_top when the last allocation window closed
+    uint32_t unsorted;        // nodes freed before that since the free stack was last put in order
     alignas(128) uint32_t free_top;      // entries on the free stack
     alignas(128) uint32_t alloc_count;   // branch nodes allocated in the current sequence (ranks after its new leaves)
     alignas(128) uint32_t n_new_leaves;  // leaves created in the current sequence: allocation ranks [0, n_new_leaves)
     alignas(128) uint32_t n_drift;       // queued reference-count corrections of the reference's quirks
     alignas(128) uint32_t dry_owners;    // dry run: branch keys that would be new
+    alignas(128) uint32_t sort_cur;      // entries of the free stack being put in order
     HotCounter gc_count[kLevels + 2];
     // statistics, striped over 64 cache lines by block index (summed when read)
     alignas(128) uint64_t st[kStatStripes][32];

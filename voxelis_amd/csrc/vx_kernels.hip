@@ -648,6 +648,57 @@ __global__ void k_dry_leaves(Pool<T> P) {
     }
 }
 
+// The free stack is put in index order when enough of it is not: nodes freed together lie
+// anywhere in the pool after a few replaced worlds, and so do then the nodes allocated
+// together, whose columns the probe, the commit and the next GC write and read one sector
+// each.  From 2^18 frees on, and a quarter of the stack: 2048 uneven u16 trees (13 M nodes
+// replaced per call) take 11.9 ms per call in the order of their frees and 10.75 ms so (GC 2.17
+// -> 1.89, commit 1.85 -> 1.53, probes 3.10 -> 2.60), 333 scattered i32 trees 1.80 -> 1.65 ms.
+__device__ inline bool sort_due(const Ctl* ctl) {
+    const uint32_t u = ctl->unsorted + (ctl->free_top - ctl->free_base);
+    return u >= 1u << 18 && u >= ctl->free_top / 4;
+}
+
+// The stack written anew from the nodes marked free, in runs of index order (one run per
+// block and turn; the runs' places come from a counter).  Nothing else of the launch reads
+// it.  A 256-lane block.
+__device__ inline void sort_free(Ctl* ctl, const uint32_t* tmg, uint32_t* free_stack) {
+    __shared__ uint32_t s_w[4], s_base;
+    constexpr uint32_t kPer = 32;
+    const uint32_t top = ctl->next_index, nfree = ctl->free_top, lane = __lane_id(), w = threadIdx.x >> 6;
+    for (uint64_t i0 = (uint64_t)blockIdx.x * 256 * kPer; i0 < top; i0 += (uint64_t)gridDim.x * 256 * kPer) {
+        const uint64_t i = i0 + (uint64_t)threadIdx.x * kPer;
+        uint32_t m = 0;
+        if (i + kPer <= top) {
+            uint4 t[kPer / 4];
+#pragma unroll
+            for (uint32_t k = 0; k < kPer / 4; k++) t[k] = ((const uint4*)(tmg + i))[k];
+#pragma unroll
+            for (uint32_t k = 0; k < kPer / 4; k++)
+                m |= ((t[k].x >> 31) | (t[k].y >> 31) << 1 | (t[k].z >> 31) << 2 | (t[k].w >> 31) << 3) << (4 * k);
+        } else {
+            for (uint32_t k = 0; k < kPer; k++)
+                if (i + k < top) m |= (tmg[i + k] >> 31) << k;
+        }
+        const uint32_t cnt = (uint32_t)__popc(m);
+        uint32_t x = cnt;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o);
+            if ((int)lane >= o) x += y;
+        }
+        if (lane == 63) s_w[w] = x;
+        __syncthreads();
+        if (threadIdx.x == 0) s_base = atomicAdd(&ctl->sort_cur, s_w[0] + s_w[1] + s_w[2] + s_w[3]);
+        __syncthreads();
+        uint32_t at = s_base + x - cnt;
+        for (uint32_t k = 0; k < w; k++) at += s_w[k];
+        for (; m; m &= m - 1, at++)
+            if (at < nfree) free_stack[at] = (uint32_t)(i + (uint32_t)__ffs(m) - 1u);
+        __syncthreads();  // s_w and s_base are written again
+    }
+}
+
 // Close the allocation window of a launch sequence (one thread, once every allocation was
 // made).  An aborted apply's allocator cursors stay: its allocations are given back.  Only
 // fields that no kernel reads before the next sequence's ctl_begin, or that other lanes do
@@ -655,6 +706,7 @@ __global__ void k_dry_leaves(Pool<T> P) {
 template <typename T>
 __device__ inline void close_allocation(const Pool<T>& P, bool abort, uint32_t* counts) {
     Ctl* ctl = P.ctl;
+    ctl->sort_cur = 0;
     if (abort) {
         if (counts) counts[0] = counts[1] = 0xFFFFFFFFu;
         return;
@@ -667,9 +719,12 @@ __device__ inline void close_allocation(const Pool<T>& P, bool abort, uint32_t* 
     ctl->live_leaves += made;
     ctl->live_branches += ctl->alloc_count;
     *stat(ctl, ST_LEAF_MISS) += made;
+    if (P.dry) return;
+    // (free_top is still what the sequence began with: the frees come after this)
+    ctl->unsorted = sort_due(ctl) ? 0u : ctl->unsorted + (ctl->free_top - ctl->free_base);
     const uint32_t n = ctl->n_new_leaves + ctl->alloc_count;
     const uint32_t used_free = n < ctl->free_top0 ? n : ctl->free_top0;
-    ctl->free_top = ctl->free_top0 - used_free;
+    ctl->free_top = ctl->free_base = ctl->free_top0 - used_free;
     const uint64_t nx = (uint64_t)ctl->next0 + (n - used_free);
     ctl->next_index = (uint32_t)(nx > 0xFFFFFFFFull ? 0xFFFFFFFFull : nx);
 }
@@ -2168,7 +2223,11 @@ __device__ inline void rollback_body(const Pool<T>& P, const LevelTiles& LT) {
     if (P.dry) return;
     const uint32_t nl = (uint32_t)alloc_done(P, P.ctl->n_new_leaves);
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < nl; j += gridDim.x * blockDim.x)
-        leaf_remove(P, (uint32_t)P.values[P.new_leaves[j]]);
+    {
+        const uint32_t idx = P.new_leaves[j];
+        leaf_remove(P, (uint32_t)P.values[idx]);
+        P.tmg[idx] |= kTmgFree;
+    }
     uint32_t nu = P.ctl->n_undo < P.undo_cap ? P.ctl->n_undo : P.undo_cap;
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < nu; j += gridDim.x * blockDim.x)
         atomicSub(&P.refs[P.undo[j].idx], (uint32_t)P.undo[j].delta);
@@ -2254,7 +2313,7 @@ __device__ inline void leaf_cleanup_body(const Pool<T>& P) {
                 leaf_remove(P, (uint32_t)P.values[idx]);
                 P.values[idx] = 0;
                 const uint32_t g = tmg_gen(P.tmg[idx]) + 1u;
-                P.tmg[idx] = tmg_make(0u, g >= kMaxGeneration ? 0u : g);
+                P.tmg[idx] = tmg_make(0u, g >= kMaxGeneration ? 0u : g) | kTmgFree;
                 uint32_t pos = atomicAdd(&P.ctl->free_top, 1u);
                 if (pos < P.capacity) P.free_stack[pos] = idx;
                 else atomicOr(&P.ctl->err, kErrPoison);
@@ -2334,7 +2393,7 @@ __device__ inline void gc_free(const Pool<T>& P, uint32_t idx, uint32_t* akey, u
         for (int j = 0; j < 8; j++) old[j] = ((gmask >> j) & 1u) ? atomicSub(&P.refs[bid_index(ch[j])], 1u) : 0u;
         // remove the pattern (mod.rs:518): a one-leaf key from its index (the leaf is
         // still live: this node's reference is still being dropped), any other from the
-        // table, leaving a tombstone
+        // table
         if (P.single && tm_is_single(tm)) {
             P.single[single_index(P, tm, ch)] = 0;
         } else {
@@ -2344,8 +2403,16 @@ __device__ inline void gc_free(const Pool<T>& P, uint32_t idx, uint32_t* akey, u
             for (uint64_t guard = 0; guard <= P.tmask; guard++) {
                 uint64_t e = P.tab[s];
                 if (e == want) {
-                    P.tab[s] = kSlotTomb;
-                    *tomb = true;
+                    // Before an empty slot no scan goes on through this one (every slot
+                    // between a key's home and its place is taken), so it becomes empty
+                    // itself; only removals run meanwhile, which never fill a slot.  At low
+                    // load that is nearly every removal (2048 uneven u16 trees: 0.5 M tombstones
+                    // per call instead of 1.6 M, the brick probe after 36 calls 1.66 instead of
+                    // 1.88 ms for 0.1 ms more GC).  Clearing the tombstones before an emptied
+                    // slot as well cost the GC what it gave the probes.
+                    const bool end = P.tab[(s + 1) & P.tmask] == kSlotEmpty;
+                    P.tab[s] = end ? kSlotEmpty : kSlotTomb;
+                    *tomb = !end;
                     break;
                 }
                 if (e == kSlotEmpty) break;
@@ -2362,7 +2429,7 @@ __device__ inline void gc_free(const Pool<T>& P, uint32_t idx, uint32_t* akey, u
         for (int j = 0; j < 8; j++)
             if (((gmask >> j) & 1u) && old[j] == one) s_next[atomicAdd(s_nnext, 1u)] = bid_index(ch[j]);
     }
-    P.tmg[idx] = tmg_make(0u, g >= kMaxGeneration ? 0u : g);  // no types/mask: free
+    P.tmg[idx] = tmg_make(0u, g >= kMaxGeneration ? 0u : g) | kTmgFree;  // no types/mask
 }
 
 // Applies the block's combined decrements (a 256-lane block: every lane takes
@@ -2603,7 +2670,8 @@ __global__ __launch_bounds__(256) void k_gc_round(Pool<T> P, uint32_t round, con
 // processes for three times that (a set of one voxel in each: 233 or 320 us a call; 177 so,
 // with the slots' places computed and not uploaded).
 __global__ void k_tab_clear(uint64_t* tab, uint64_t nslots, Ctl* ctl, uint64_t* ltab, uint64_t lslots, uint32_t force,
-                            const uint4* up_src, uint4* up_dst, uint32_t up_n) {
+                            const uint4* up_src, uint4* up_dst, uint32_t up_n, const uint32_t* tmg,
+                            uint32_t* free_stack) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < up_n; i += gridDim.x * blockDim.x) up_dst[i] = up_src[i];
     static_assert(kStatStripes == 64, "one statistics stripe per lane");
     __shared__ uint32_t s_due;
@@ -2626,6 +2694,7 @@ __global__ void k_tab_clear(uint64_t* tab, uint64_t nslots, Ctl* ctl, uint64_t* 
             }
         }
     }
+    if (!force && sort_due(ctl)) sort_free(ctl, tmg, free_stack);  // uniform over the launch
     __syncthreads();
     if (!(s_due & 1u)) return;
     for (int k = 0; k < 2; k++) {  // both tables are rebuilt together
