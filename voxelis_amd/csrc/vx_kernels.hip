@@ -902,16 +902,17 @@ __device__ inline uint32_t emit_candidate(const Cands& K, uint32_t* s_cnt, bool 
 // confirms it; the merge crosses trees, since a key's node is the same for every tree.
 // Returns the set slot (*lead when this lane inserted it), or -1 when no slot was found
 // within a bounded scan (the key is then emitted on its own).  Hash 0 marks a free slot.
-template <uint32_t N>
-__device__ inline int keyset_insert(uint64_t* s_h, uint64_t h, bool* lead) {
-    const uint64_t hk = h ? h : 1ull;
+template <uint32_t N, typename H>
+__device__ inline int keyset_insert(H* s_h, H h, bool* lead) {
+    typedef typename std::conditional<sizeof(H) == 8, unsigned long long, unsigned int>::type Word;
+    const H hk = h ? h : (H)1;
     uint32_t s = (uint32_t)hk & (N - 1);
     *lead = false;
 #pragma unroll 1
     for (uint32_t g = 0; g < 32; g++) {
-        uint64_t cur = s_h[s];
+        H cur = s_h[s];
         if (cur == 0) {
-            cur = atomicCAS((unsigned long long*)&s_h[s], 0ull, (unsigned long long)hk);
+            cur = (H)atomicCAS((Word*)&s_h[s], (Word)0, (Word)hk);
             if (cur == 0) {
                 *lead = true;
                 return (int)s;
@@ -933,6 +934,20 @@ __device__ inline bool vox8_equal(const V& a, const V& b) {
 #pragma unroll
     for (int i = 0; i < (int)(sizeof(V) / 4); i++) eq &= x[i] == y[i];
     return eq;
+}
+
+// Hash of a brick's eight values (products of pairs of words, as in branch_hash).
+template <typename V>
+__device__ inline uint32_t vox8_hash(const V& v) {
+    const uint32_t* w = (const uint32_t*)&v;
+    uint64_t s = 0;
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(V) / 4); i += 2)
+        s += (uint64_t)(w[i] + 0x4ABEA221u + 0x3A1B5D06u * i) * (w[i + 1] + 0x23148989u + 0x5DCE1B54u * i);
+    uint32_t x = (uint32_t)s ^ (uint32_t)(s >> 32);
+    x ^= x >> 15;
+    x *= 0x2C1B3C6Du;
+    return x ^ (x >> 13);
 }
 
 // Tile statistics in LDS, flushed with one striped atomic per counter per block.
@@ -1074,7 +1089,12 @@ constexpr int brick_rounds() { return TILE >= 512 ? 2 : 4; }
 // block start + j*TILE + lane in round j).  Phase 1 issues every round's loads at
 // once (edit mask, the 8 values and the old height-2 node above the brick) and
 // settles the bricks that need no old tree: untouched ones and all-same ones whose
-// leaf exists.  The rest (mixed bricks; all-same ones whose leaf is missing) are queued in
+// leaf exists.  A completely written brick of different values over a branch or nothing has
+// a result that follows from its values: of those with equal values in the block (found by a
+// hash of the values, in registers) only the first goes on, and the others copy its result at
+// the end.  (Merged by their finished keys, each took eight leaf look-ups, the build and the
+// key's hash: 2048 trees of 64^3 and 128^3 u16, half of them dense, a pass of 3.42 ms, 3.00 so.)
+// The rest (mixed bricks; all-same ones whose leaf is missing) are queued in
 // LDS with their loaded data and take phase 2, one per lane, in rounds of TILE: the
 // old-tree descent, the leaves that do not exist yet (leaf_ensure), and brick_work.  Round r of phase 2
 // emits into candidate tile blk*R + r.  The pass is bound by memory latency, so it runs
@@ -1088,26 +1108,32 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
     typedef typename std::conditional<sizeof(T) == 1, uint2, typename std::conditional<sizeof(T) == 2, uint4,
                                                                                           Vox8x4>::type>::type Vox8;
     static_assert(sizeof(Vox8) == 8 * sizeof(T), "8 voxels");
-    static_assert(R * TILE <= 0x4000, "queued brick index is 14 bits");
-    constexpr uint32_t kSame = 0x8000u, kMiss = 0x4000u;  // all eight values equal; a leaf is missing
+    static_assert(R * TILE <= 0x2000, "queued brick index is 13 bits");
+    // all eight values equal; a leaf is missing; its equals were found by its values
+    constexpr uint32_t kSame = 0x8000u, kMiss = 0x4000u, kByValue = 0x2000u;
+    constexpr uint32_t kOwn = 0xFFFFu;
+    // a wavefront merges by value from here on: fewer such bricks fit one round of phase 2
+    // anyway (4096 trees of 32^3 terrain, their surface: a pass of 143 us, 159 without the rule)
+    constexpr uint32_t kManyFull = 16 * R;
     __shared__ uint32_t s_nq, s_miss;
     __shared__ uint32_t s_cnt[R];
     __shared__ uint32_t s_st[8];
     // u8: the leaf id of every value, from LDS (loaded past the caches, so that a leaf
     // created by an earlier block of the launch is seen)
     __shared__ uint64_t s_leaf[sizeof(T) == 1 ? 256 : 1];
-    __shared__ uint64_t s_up[R * TILE];
+    __shared__ uint64_t s_up[R * TILE];  // the node above the brick; once built, its result
     __shared__ Vox8 s_v[R * TILE];
     __shared__ uint16_t s_idx[R * TILE];
+    __shared__ uint16_t s_of[R * TILE];  // per slot the queue entry whose result it has (kOwn: none)
     __shared__ uint8_t s_m[R * TILE];
-    // the block's key set (keyset_insert): a quarter as many slots as the block has
+    // the block's set (keyset_insert) of value hashes (top bit set) and, for the bricks not
+    // merged by value, key hashes: a quarter as many slots as the block has
     // bricks, enough for the few distinct keys of a dense region (a block of all-distinct
     // keys fills it and emits the rest unmerged), and small enough that five blocks of
     // 256 lanes with u16 values share a CU's LDS
     constexpr uint32_t kSetB = R * TILE / 4;
-    __shared__ uint64_t s_kh[kSetB];
-    __shared__ uint32_t s_kc[kSetB];
-    __shared__ uint16_t s_kq[kSetB];  // the leader's queue entry (its mask and values in LDS)
+    __shared__ uint32_t s_kh[kSetB];
+    __shared__ uint16_t s_kq[kSetB];  // the leader's queue entry
     for (uint32_t i = threadIdx.x; i < kSetB; i += TILE) s_kh[i] = 0;
     uint64_t lm[sizeof(T) == 1 ? (256 + TILE - 1) / TILE : 1];
     if (sizeof(T) == 1)
@@ -1121,10 +1147,12 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
     uint32_t m[R];
     Vox8 vw[R];
     uint64_t up[R];
+    bool free[R];       // the tree is deep enough and has no fill: may be merged by value
+    uint32_t place[R];  // the brick's place in its height-2 node
     {
         uint32_t cj[R], pj[R];
         uint64_t uj[R];
-        bool lj[R];
+        bool lj[R], deep[R];
         bool uni = true;  // every slot's chunk is one per wavefront: scalar loads
 #pragma unroll
         for (int j = 0; j < R; j++) {
@@ -1140,11 +1168,13 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
             // the height-2 slot above this brick follows from the slot (a depth-1 tree
             // has none; a tree with a fill does not use it)
             uj[j] = D >= 2 ? G.next + (local >> 3) : 0;
+            deep[j] = D >= 2;
             uni = uni && __ballot(cj[j] != __builtin_amdgcn_readfirstlane(cj[j])) == 0;
         }
         const uint8_t* hm[R];
         const void* hv[R];
         int32_t hs[R];
+        bool hf[R];
         if (uni) {
 #pragma unroll
             for (int j = 0; j < R; j++) {
@@ -1152,6 +1182,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
                 hm[j] = r.masks;
                 hv[j] = r.values;
                 hs[j] = r.status;
+                hf[j] = r.has_fill != 0;
             }
         } else {
 #pragma unroll
@@ -1160,6 +1191,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
                 hm[j] = r.masks;
                 hv[j] = r.values;
                 hs[j] = r.status;
+                hf[j] = r.has_fill != 0;
             }
         }
         // (global-memory loads: a generic load may return out of order with the others,
@@ -1180,7 +1212,11 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
         for (int j = 0; j < R; j++) asm volatile("" ::"v"(m[j]));
 #pragma unroll
         for (int j = 0; j < R; j++)
-            if (!lj[j] || hs[j] < 0) m[j] = 0;
+            {
+                if (!lj[j] || hs[j] < 0) m[j] = 0;
+                free[j] = !hf[j] && deep[j];
+                place[j] = pj[j] & 7u;
+            }
     }
     if (sizeof(T) == 1)
         for (uint32_t i = 0, vv = threadIdx.x; vv < 256; i++, vv += TILE) s_leaf[vv] = lm[i];
@@ -1219,18 +1255,53 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
         for (int j = 0; j < R; j++)
             if (asj[j] && lidj[j] == kEmpty) lidj[j] = leaf_now(P, (uint32_t)*(const T*)&vw[j]);
     }
+    // the old child a completely written brick replaces is looked at only for the panic of a
+    // leaf at brick level; such bricks, and those under a leaf, go to phase 2 unmerged
+    bool full[R], any_of = false;
+    uint32_t nfull = 0;  // of the wavefront
+    int ks[R];
+    bool lead[R];
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        full[j] = m[j] == 0xFFu && !asj[j];
+        nfull += (uint32_t)__popcll(__ballot(full[j]));
+        ks[j] = -1;
+        lead[j] = false;
+    }
+    const bool by_value = nfull > kManyFull && P.brick_merge_rounds;
+    if (by_value) {
+        uint64_t below[R];
+#pragma unroll
+        for (int j = 0; j < R; j++) {
+            full[j] = full[j] && free[j] &&
+                      (up[j] == kEmpty || (!bid_is_leaf(up[j]) && bid_index(up[j]) < P.capacity));
+            below[j] = P.children[8ull * (full[j] ? bid_index(up[j]) : 0u) + place[j]];
+        }
+#pragma unroll
+        for (int j = 0; j < R; j++) {
+            full[j] = full[j] && (up[j] == kEmpty || below[j] == kEmpty || !bid_is_leaf(below[j]));
+            if (full[j]) ks[j] = keyset_insert<kSetB>(s_kh, vox8_hash(vw[j]) | 0x80000000u, &lead[j]);
+            any_of = any_of || (ks[j] >= 0 && !lead[j]);
+        }
+    }
+    const bool wave_of = __ballot(any_of) != 0;
+    const auto enqueue = [&](int j, uint32_t q) {
+        s_idx[q] = (uint16_t)((j * TILE + threadIdx.x) | (asj[j] ? kSame : 0u) | (by_value && full[j] ? kByValue : 0u));
+        s_m[q] = (uint8_t)m[j];
+        s_v[q] = vw[j];
+        s_up[q] = up[j];
+    };
 #pragma unroll
     for (int j = 0; j < R; j++) {
         const uint64_t slot = b0 + (uint64_t)j * TILE + threadIdx.x;
         const uint64_t lid = lidj[j];
-        const bool queue = m[j] != 0 && lid == kEmpty;
+        const bool follow = ks[j] >= 0 && !lead[j];
+        const bool queue = m[j] != 0 && lid == kEmpty && !follow;
         const uint32_t q = wave_append(&s_nq, queue);
         if (queue) {
-            s_idx[q] = (uint16_t)((j * TILE + threadIdx.x) | (asj[j] ? kSame : 0u));
-            s_m[q] = (uint8_t)m[j];
-            s_v[q] = vw[j];
-            s_up[q] = up[j];
-        } else if (slot < L.nslots) {
+            enqueue(j, q);
+            if (lead[j]) s_kq[ks[j]] = (uint16_t)q;
+        } else if (!follow && slot < L.nslots) {
             res1[slot] = m[j] != 0 ? lid : kInvalid;
             ncollapse += m[j] != 0;
         }
@@ -1238,6 +1309,20 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
     {
         const uint32_t t = wave_sum(ncollapse);
         if (__lane_id() == 0 && t) atomicAdd(&s_st[1], t);
+    }
+    __syncthreads();
+    if (wave_of) {
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        const bool follow = ks[j] >= 0 && !lead[j];
+        const uint32_t lq = follow ? s_kq[ks[j]] : kOwn;
+        const bool differ = follow && !vox8_equal(vw[j], s_v[lq]);  // another brick with the same hash
+        if (__ballot(differ)) {
+            const uint32_t q = wave_append(&s_nq, differ);
+            if (differ) enqueue(j, q);
+        }
+        s_of[j * TILE + threadIdx.x] = (uint16_t)(differ ? kOwn : lq);
+    }
     }
     __syncthreads();
     const uint32_t nq = s_nq;
@@ -1262,7 +1347,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
         uint32_t tm = 0, c = 0, mm = 0, need = 0;
         if (live) {
             const uint32_t qi = s_idx[q];
-            slot = b0 + (qi & (kMiss - 1));
+            slot = b0 + (qi & (kByValue - 1));
             mm = s_m[q];
             const Vox8 w = s_v[q];
             const uint64_t upq = s_up[q];
@@ -1385,6 +1470,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
             need = 0;
         }
         // (a leaf created in this launch is seen past the caches)
+        bool wait = false;  // for the second pass
         if (__ballot(need != 0)) {
             if constexpr (sizeof(T) <= 2) {
                 asm volatile("" ::: "memory");  // (the values again from LDS, below too: no registers hold them)
@@ -1400,6 +1486,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
                 if (pass == 0) {
                     s_idx[q] |= kMiss;
                     s_miss = 1;
+                    wait = true;
                 }
             }
         }
@@ -1445,28 +1532,21 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
         key[8] = tm;
         const uint64_t hk = cand ? branch_hash(ch, tm) : 0ull;
         bool lead = false;
-        const int ks = cand && P.brick_merge_rounds ? keyset_insert<kSetB>(s_kh, hk, &lead) : -1;
+        const int ks = cand && P.brick_merge_rounds && !(s_idx[q] & kByValue)
+                           ? keyset_insert<kSetB>(s_kh, (uint32_t)(hk >> 32) & 0x7FFFFFFFu, &lead) : -1;
         const uint32_t tile = blockIdx.x * R + (uint32_t)r;
-        const uint32_t pos = emit_candidate<TILE>(K, &s_cnt[r], cand && (lead || ks < 0), ch, tm, slot, tile, hk);
-        if (lead) {
-            s_kc[ks] = (uint32_t)((uint64_t)tile * TILE) + pos;
-            s_kq[ks] = (uint16_t)q;
-        }
+        const bool emit = cand && (lead || ks < 0);
+        const uint32_t pos = emit_candidate<TILE>(K, &s_cnt[r], emit, ch, tm, slot, tile, hk);
+        if (mine && !wait) s_up[q] = emit ? res_pending((uint32_t)((uint64_t)tile * TILE) + pos) : out;
+        if (lead) s_kq[ks] = (uint16_t)q;
         __syncthreads();  // the leaders' candidates and their indices are visible to the block
         bool follow = false;
         if (cand && ks >= 0 && !lead) {
-            const uint32_t k2 = s_kc[ks];
-            // Two completely written bricks have equal keys exactly when their values are
-            // equal: every child is then the leaf of its value (a live leaf is the one leaf
-            // of its value; a dry run's placeholder is a function of the value too) and
-            // types = mask = 0xFF, whatever the old brick was.  Such a pair is compared in
-            // LDS; any other pair compares the leader's candidate key.
-            const uint32_t lq = s_kq[ks];
-            const bool both_full = s_m[q] == 0xFFu && s_m[lq] == 0xFFu;
-            if (both_full ? vox8_equal(s_v[q], s_v[lq]) : key_matches_cand(K, k2, key)) {
+            const uint32_t k2 = (uint32_t)s_up[s_kq[ks]];
+            if (key_matches_cand(K, k2, key)) {
                 out = res_pending(k2);
                 follow = true;
-            } else {  // another key with the same 64-bit hash: a candidate of its own
+            } else {  // another key with the same hash: a candidate of its own
                 const uint32_t p2 = atomicAdd(&s_cnt[r], 1u);
                 write_candidate(K, (uint64_t)tile * TILE + p2, ch, tm, hk, slot);
             }
@@ -1490,6 +1570,21 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
             }
             leaf_ensure(P, need, 8, [&](int i) { return (uint32_t)((const T*)&s_v[q])[i]; });
         }
+    }
+    }
+    // (the leaders' results are visible: a barrier ended the last pass)
+    if (wave_of) {
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        const uint32_t lq = s_of[j * TILE + threadIdx.x];
+        bool pend = false;
+        if (lq != kOwn) {
+            const uint64_t out = s_up[lq];
+            res1[b0 + (uint64_t)j * TILE + threadIdx.x] = out;
+            pend = res_is_pending(out);
+        }
+        tile_count(s_st, 0, pend);
+        tile_count(s_st, 3, pend);
     }
     }
     __syncthreads();
