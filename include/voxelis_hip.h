@@ -95,7 +95,7 @@ int vx_interner_set_stream(vx_interner* h, void* hip_stream);
  * its keys become candidates (0-16; equal keys of one tree share a candidate);
  * brick_rounds: brick slots per lane of the brick pass (1, 2 or 4; 0: 4 when the
  * pass has at least 512 blocks of them, else 1).
- * Defaults {256, 8, 1024, 1024, 32768, 512, 4, 0}.  Synchronizes the interner's
+ * Defaults {256, 8, 1024, 1024, 2048, 512, 4, 0}.  Synchronizes the interner's
  * stream. */
 typedef struct {
     uint32_t tile;

@@ -46,7 +46,7 @@ def _time(step, steps, warmup):
 
 def autotune(make_case, load_factors=(0.5, 0.6, 0.7, 0.85), tiles=(128, 256, 512), dedups=(0, 2, 4, 8),
              commit_grids=(256, 1024, 4096), gc_grids=(256, 1024, 4096),
-             probe_blocks_bricks=(0, 8192, 16384, 32768), probe_blocks=(0, 256, 512, 1024),
+             probe_blocks_bricks=(0, 1024, 2048, 8192, 32768), probe_blocks=(0, 256, 512, 1024),
              brick_merge_rounds=(0, 2, 4, 8), brick_rounds=(0, 1, 2, 4), steps=6, warmup=2, log=None):
     """make_case(load_factor) -> (interner, step(k), close()); returns (best point, all points).
 
@@ -60,10 +60,10 @@ def autotune(make_case, load_factors=(0.5, 0.6, 0.7, 0.85), tiles=(128, 256, 512
             for tile in tiles:
                 for dd in dedups:
                     it.set_tuning(tile=tile, dedup_rounds=dd, commit_grid=1024, gc_grid=1024,
-                                  probe_blocks_bricks=32768, probe_blocks=512, brick_merge_rounds=4, brick_rounds=0)
+                                  probe_blocks_bricks=2048, probe_blocks=512, brick_merge_rounds=4, brick_rounds=0)
                     t = _time(step, steps, warmup)
                     pt = {"load_factor": lf, "tile": tile, "dedup_rounds": dd, "commit_grid": 1024,
-                          "gc_grid": 1024, "probe_blocks_bricks": 32768, "probe_blocks": 512,
+                          "gc_grid": 1024, "probe_blocks_bricks": 2048, "probe_blocks": 512,
                           "brick_merge_rounds": 4, "brick_rounds": 0, "s_per_step": t}
                     points.append(pt)
                     if log:

@@ -36,7 +36,11 @@ constexpr uint64_t kMaxGrid = 8192;
 
 // Tiles per probe block: candidates of sparse tiles are packed into full
 // wavefronts, and the owners' allocation takes one update of the shared counter per
-// block; at least `blocks` blocks stay so the launch still spreads over the chip.
+// block; at least `blocks` blocks stay so the launch still spreads over the chip.  The brick
+// level's default is 2048, eight blocks for each CU: the counter's updates, about 20 ns each,
+// are what bounds a probe of many sparse tiles (333 scattered i32 trees of 64^3, 42 k tiles:
+// 430 us with 32768 blocks, 243 with 16384, 173 with 8192, 122 with 2048, 125 with 1024; 4096
+// trees of 32^3 terrain 84, 54, 45 and 43 us, the last with 16 tiles to a block).
 inline uint32_t probe_group(uint32_t ntiles, uint32_t blocks) {
     if (blocks == 0) return 1;
     return std::max<uint32_t>(1u, std::min<uint32_t>(kProbeTiles, ntiles / blocks));
@@ -175,7 +179,7 @@ struct vx_interner {
     int ring_cur = 0;
     void* h_pinned = nullptr;  // the slot of the current call
     Prof prof;
-    vx_tuning tune = {256, 8, 1024, 1024, 32768, 512, 4, 0};
+    vx_tuning tune = {256, 8, 1024, 1024, 2048, 512, 4, 0};
     // captured launch sequences of repeated calls (vx_interner_set_graphs)
     bool graphs = false;
     hipStream_t cap_stream = nullptr;
