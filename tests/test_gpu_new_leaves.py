@@ -143,3 +143,29 @@ def test_failed_tree_beside_new_ids(vx, width, brick_rounds):
     assert (st == -5).all()
     assert it.counts() == before
     assert_same(it, f, it_o, trees, what="every tree failed")
+
+
+@pytest.mark.parametrize("width", [2, 4])
+def test_applies_out_of_nodes_leave_no_request_behind(vx, width):
+    """Many new ids at once, in a used table, with a reservation that runs out at once: again and
+    again nothing is left of it, and then the same ids are created."""
+    api, W = vx
+    rng = np.random.default_rng(width)
+    trees, depth = 48, 5
+    n = 8 ** (depth - 1)
+    it = api.VoxInterner(width, 64 * MB)
+    f = api.Forest(it, [depth] * trees)
+    top = (1 << 16) - 1 if width == 2 else 1 << 24
+    for step in range(3):
+        v = rng.integers(1, top, (trees, n, 8)).astype(NP[width])
+        v[rng.random(v.shape) >= 0.1] = 0
+        m = np.zeros((trees, n, 2), dtype=np.uint8)
+        m[:, :, 0] = np.packbits(v != 0, axis=2, bitorder="little")[:, :, 0]
+        f.fill([0] * trees)  # (their leaves' places in the table are free again)
+        dev = [[api.to_device(a[t]) for t in range(trees)] for a in (m, v)]
+        before = (it.counts(), it.alive_nodes())
+        for k in range(12):
+            assert (f.apply(*dev, node_limit=1 + 40 * k) == -8).all()
+            assert (it.counts(), it.alive_nodes()) == before, (step, k)
+        assert (f.apply(*dev) == 1).all()
+        assert it.counts()[0] == len(np.unique(v[v != 0]))

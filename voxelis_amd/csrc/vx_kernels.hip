@@ -299,13 +299,12 @@ __device__ inline uint64_t ltab_claim(const Pool<T>& P, uint32_t v, bool* won, u
     return ~0ull;
 }
 
-// i32: the slot and current entry of value v (0: none).
+// i32: the current entry of value v (0: none).
 template <typename T>
-__device__ inline uint64_t ltab_peek(const Pool<T>& P, uint32_t v, uint64_t* slot) {
+__device__ inline uint64_t ltab_peek(const Pool<T>& P, uint32_t v) {
     uint64_t s = leaf_hash(v) & P.lmask;
     for (uint64_t g = 0; g <= P.lmask; g++) {
         const uint64_t e = load_agent(&P.ltab[s]);
-        *slot = s;
         if (e == 0 || (e != kLeafTomb && (uint32_t)(e >> 32) == v)) return e;
         s = (s + 1) & P.lmask;
     }
@@ -342,8 +341,7 @@ __device__ inline uint64_t leaf_now(const Pool<T>& P, uint32_t v) {
     if constexpr (sizeof(T) <= 2) {
         return load_agent(&P.leaf_ids[v]);
     } else {
-        uint64_t slot;
-        const uint64_t e = ltab_peek(P, v, &slot);
+        const uint64_t e = ltab_peek(P, v);
         return e && (uint32_t)e != kLeafNeed ? make_leaf((uint32_t)e, tmg_gen(P.tmg[(uint32_t)e])) : kEmpty;
     }
 }
@@ -369,6 +367,10 @@ __device__ inline void leaf_ensure(const Pool<T>& P, uint32_t need, int n, V val
     const uint32_t lane = __lane_id();
     const uint64_t below = (1ull << lane) - 1ull;
     uint32_t won = 0, wait = 0;
+    // i32 (n is 1): the table slot that the lane claimed.  It is not looked for again: an apply
+    // that runs out of nodes puts tombstones in front of other claims of the launch, so that
+    // one value may have two entries, and each claimant has to give back its own.
+    [[maybe_unused]] uint64_t claimed = 0;
     if (!__ballot(need != 0)) return;
 #pragma unroll 1
     for (int i = 0; i < n; i++) {
@@ -398,7 +400,8 @@ __device__ inline void leaf_ensure(const Pool<T>& P, uint32_t need, int n, V val
                 }
             } else {
                 uint64_t e;
-                if (ltab_claim(P, v, &w, &e) != ~0ull) wait |= (w ? 0u : 1u) << i;
+                claimed = ltab_claim(P, v, &w, &e);
+                if (claimed != ~0ull) wait |= (w ? 0u : 1u) << i;
             }
             won |= (w ? 1u : 0u) << i;
         }
@@ -418,8 +421,6 @@ __device__ inline void leaf_ensure(const Pool<T>& P, uint32_t need, int n, V val
                 const uint32_t rank = k + (uint32_t)__popcll(b & below), v = value(i);
                 bool ok;
                 const uint32_t idx = alloc_at(P, rank, &ok, ft0, next0);
-                uint64_t slot = 0;
-                if constexpr (sizeof(T) == 4) ltab_peek(P, v, &slot);
                 if (ok) {
                     const uint32_t gen = tmg_gen(P.tmg[idx]);
                     // a recycled node keeps its old children (the free does not clear
@@ -430,9 +431,9 @@ __device__ inline void leaf_ensure(const Pool<T>& P, uint32_t need, int n, V val
                     P.tmg[idx] = tmg_make(0u, gen);
                     P.new_leaves[rank] = idx;
                     if constexpr (sizeof(T) <= 2) store_agent(&P.leaf_ids[v], make_leaf(idx, gen));
-                    else store_agent(&P.ltab[slot], ((uint64_t)v << 32) | idx);
+                    else store_agent(&P.ltab[claimed], ((uint64_t)v << 32) | idx);
                 } else if constexpr (sizeof(T) == 4) {
-                    store_agent(&P.ltab[slot], kLeafTomb);
+                    store_agent(&P.ltab[claimed], kLeafTomb);
                 }
             }
             k += (uint32_t)__popcll(b);
