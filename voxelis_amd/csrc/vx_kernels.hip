@@ -491,7 +491,7 @@ __device__ inline void leaf_remove(const Pool<T>& P, uint32_t v) {
 
 // The index of the launch sequence's k-th allocation: the free stack first, then
 // fresh indices.  ft0 / next0: the allocation window's snapshot (free_top0, next0), which
-// no kernel of the sequence changes before k_end_alloc.
+// no kernel of the sequence changes before the window is closed.
 template <typename T>
 __device__ inline uint32_t alloc_at(const Pool<T>& P, uint32_t k, bool* ok, uint32_t ft0, uint32_t next0) {
     if (k >= P.alloc_limit) {
@@ -3148,7 +3148,7 @@ __global__ void k_get(Pool<T> P, uint64_t nq, uint64_t ntrees, const uint64_t* r
 }
 
 // get for queries grouped by tree: tree t's queries are [qoff[t], qoff[t+1]).  A block
-// takes `per` consecutive queries.  For each tree its range meets, the block first walks
+// takes `per` consecutive queries, one from the nlong-th on `per2`.  For each tree its range meets, the block first walks
 // every path of the tree's top k levels (k = 3 for a segment of at least 256 queries,
 // 2 from 32, else none) and keeps the node each path reaches in LDS; a query then takes
 // the node of its first k child digits from there and walks the rest in HBM
@@ -3159,12 +3159,15 @@ template <typename T, int TILE>
 __global__ __launch_bounds__(TILE) void k_get_grouped(Pool<T> P, uint64_t nq, uint32_t ntrees,
                                                       const uint64_t* roots, const uint8_t* depths,
                                                       const uint64_t* qoff, const int32_t* xyz, T* out,
-                                                      uint8_t* present, uint8_t* stop, uint64_t per) {
+                                                      uint8_t* present, uint8_t* stop, uint32_t per,
+                                                      uint32_t nlong, uint32_t per2) {
     __shared__ uint64_t s_node[1u << (3 * kGetTop)];
     __shared__ uint8_t s_dep[1u << (3 * kGetTop)];
     __shared__ uint32_t s_lo;
-    const uint64_t q1 = min(nq, (uint64_t)(blockIdx.x + 1) * per);
-    uint64_t q0 = (uint64_t)blockIdx.x * per;
+    const uint32_t n = blockIdx.x < nlong ? per : per2;
+    uint64_t q0 = blockIdx.x < nlong ? (uint64_t)blockIdx.x * per
+                                     : (uint64_t)nlong * per + (uint64_t)(blockIdx.x - nlong) * n;
+    const uint64_t q1 = min(nq, q0 + n);
     if (q0 >= q1) return;
     // the tree holding q0, the last t with qoff[t] <= q0: a TILE-way search per round
     {
@@ -3192,6 +3195,11 @@ __global__ __launch_bounds__(TILE) void k_get_grouped(Pool<T> P, uint64_t nq, ui
         const bool tree_ok = seg_ok && D <= (uint32_t)kMaxDepth;
         const uint64_t n_seg = e - q0;
         const uint32_t k = !tree_ok ? 0u : min(D, n_seg >= 256 ? kGetTop : n_seg >= 32 ? 2u : 0u);
+        // the first query's coordinates, and later each next one's, are on their way while the
+        // paths, or the query before it, are walked (a lane past the end takes the last query)
+        const uint64_t q_last = e - 1;
+        uint64_t qn = min(q0 + threadIdx.x, q_last);
+        int32_t xn = xyz[3 * qn], yn = xyz[3 * qn + 1], zn = xyz[3 * qn + 2];
         if (k) {
             const uint32_t np = 1u << (3 * k);
             for (uint32_t p = threadIdx.x; p < np; p += TILE) {
@@ -3214,7 +3222,11 @@ __global__ __launch_bounds__(TILE) void k_get_grouped(Pool<T> P, uint64_t nq, ui
             __syncthreads();
         }
         for (uint64_t q = q0 + threadIdx.x; q < e; q += TILE) {
-            const int32_t x = xyz[3 * q], y = xyz[3 * q + 1], z = xyz[3 * q + 2];
+            const int32_t x = xn, y = yn, z = zn;
+            qn = min(q + TILE, q_last);
+            xn = xyz[3 * qn];
+            yn = xyz[3 * qn + 1];
+            zn = xyz[3 * qn + 2];
             const int32_t lim = tree_ok ? 1 << D : 0;
             uint32_t v = 0;
             uint8_t pr = 0xFF, sd = 0;
