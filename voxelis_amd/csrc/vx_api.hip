@@ -47,13 +47,15 @@ inline uint32_t probe_group(uint32_t ntiles, uint32_t blocks) {
 }
 
 // The GC round that ends a call (the first is 0): its blocks follow their shares of the front
-// to the leaves themselves, with no launch per height.  A large call takes four rounds of
-// fronts before it, so that the shares are many and even: 2048 uneven u16 trees (250 M places,
-// 12 M frees) 2.09 ms, against 2.21 with a round per height, 2.77 with three rounds and 4.98
-// with one; 333 scattered i32 trees (14 M places, 1.7 M frees) 0.33 ms with one round, 0.43
-// with a round per height; one 32^3 tree 32 against 57 us.
+// to the leaves themselves, with no launch per height.  The deeper the trees, the more a share
+// of few nodes may hold, so deep trees take rounds of fronts before it, until the shares are
+// many and even.  us of the GC with the last round 1, 2, 3, 4: one 32^3 tree 31, 37, 43, 50;
+// 4096 terrain trees of 32^3 54, 60, 65, 72; 64^3, 60 uneven trees 167, 89, 97, 104, 333
+// scattered i32 trees 284, 309, 343, 363; 128^3 uneven trees, 8 of them 308, 82, 81, 88, 256 of
+// them 715, 367, 312, 319.  Above 2^25 old places (2048 uneven trees, 250 M places, 12 M frees)
+// four rounds: 2.09 ms, against 2.21 with a round per height and 2.77 with three.
 inline uint32_t gc_rounds(uint32_t deepest, uint64_t old_nodes) {
-    return std::min<uint32_t>(deepest, old_nodes <= (1u << 25) ? 1u : 4u);
+    return std::min<uint32_t>(deepest, old_nodes > (1u << 25) ? 4u : deepest <= 5 ? 1u : deepest == 6 ? 2u : 3u);
 }
 
 inline unsigned grid_for(uint64_t work) {
