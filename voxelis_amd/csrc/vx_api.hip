@@ -579,7 +579,9 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     return hipGetLastError() == hipSuccess ? VX_OK : VX_E_HIP;
     };
     auto launch_all = [&]() -> int {
-    if (!opt.dry) {
+    if (opt.dry) {
+        VX_LAUNCH(h, KID_BEGIN, k_begin, 1, 1, h->ctl);
+    } else {
         int rc = rebuild_step<T>(h, false, nre == 0, plan ? nullptr : hc, records.ptr, stage_bytes);
         if (rc) return rc;
     }

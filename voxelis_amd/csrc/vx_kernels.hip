@@ -826,9 +826,8 @@ __global__ void k_prepare(Pool<T> P, ChunkDev* chunks, uint32_t n, const uint64_
             descend_body(P, chunks, L3, M, O, roots, s);
         return;
     }
-    // a dry run's control-block reset rides in block 0 (nothing else here reads it); any
-    // other call's came with its table maintenance, since leaves are created here
-    if (P.dry && blockIdx.x == 0 && threadIdx.x == 0) ctl_begin(P.ctl);
+    // (the control block's reset came with a launch before this one: leaves are created, or
+    // by a dry run requested, here)
     for (uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (uint64_t)nprep * blockDim.x) {
         ChunkDev& C = chunks[c];
         C.root_in = roots[C.orig];
