@@ -255,11 +255,12 @@ __device__ inline void store_agent(V* p, V v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// i32: the entry of value v, inserted as kLeafNeed when there is none (*won).  Returns its
-// slot, or ~0 when the table is full.
+// i32: the entry of value v, inserted as kLeafNeed when there is none (*won; *reused: in
+// place of a tombstone, which the caller takes off their count).  Returns its slot, or ~0
+// when the table is full.
 template <typename T>
-__device__ inline uint64_t ltab_claim(const Pool<T>& P, uint32_t v, bool* won, uint64_t* entry) {
-    *won = false;
+__device__ inline uint64_t ltab_claim(const Pool<T>& P, uint32_t v, bool* won, bool* reused, uint64_t* entry) {
+    *won = *reused = false;
     *entry = 0;
     uint64_t s = leaf_hash(v) & P.lmask;
     uint64_t first_tomb = ~0ull;
@@ -282,6 +283,7 @@ __device__ inline uint64_t ltab_claim(const Pool<T>& P, uint32_t v, bool* won, u
                                  (unsigned long long)want);
             if (seen == expected) {
                 *won = true;
+                *reused = expected == kLeafTomb;
                 *entry = want;
                 return target;
             }
@@ -320,9 +322,10 @@ __device__ inline uint32_t leaf_request(const Pool<T>& P, uint32_t v) {
         P.leaf_need[v] = 1;
         return v;
     } else {
-        bool won;
+        bool won, reused;
         uint64_t e;
-        const uint64_t s = ltab_claim(P, v, &won, &e);
+        const uint64_t s = ltab_claim(P, v, &won, &reused, &e);
+        if (reused) atomicAdd((unsigned long long*)stat(P.ctl, ST_LTOMB), ~0ull);
         if (won) {
             const uint32_t pos = atomicAdd(&P.ctl->n_need, 1u);
             if (pos < P.need_cap) P.need_list[pos] = v;
@@ -361,9 +364,10 @@ __device__ inline uint64_t leaf_now(const Pool<T>& P, uint32_t v) {
 // lanes waits, so every wait ends; it also ends when an allocation fails, and it is bounded.
 // Ids are exchanged with agent-scope accesses; the new node's columns are read by later
 // launches only.  (The loops are kept rolled: this is the rare path of kernels whose
-// registers are full.)
+// registers are full.)  i32: the change in the table's tombstones goes to *s_tomb in LDS,
+// when the caller has one for its block, else to the counter.
 template <typename T, typename V>
-__device__ inline void leaf_ensure(const Pool<T>& P, uint32_t need, int n, V value) {
+__device__ inline void leaf_ensure(const Pool<T>& P, uint32_t need, int n, V value, uint32_t* s_tomb = nullptr) {
     const uint32_t lane = __lane_id();
     const uint64_t below = (1ull << lane) - 1ull;
     uint32_t won = 0, wait = 0;
@@ -371,6 +375,7 @@ __device__ inline void leaf_ensure(const Pool<T>& P, uint32_t need, int n, V val
     // that runs out of nodes puts tombstones in front of other claims of the launch, so that
     // one value may have two entries, and each claimant has to give back its own.
     [[maybe_unused]] uint64_t claimed = 0;
+    [[maybe_unused]] bool reused = false, gave = false;  // a tombstone taken, one left
     if (!__ballot(need != 0)) return;
 #pragma unroll 1
     for (int i = 0; i < n; i++) {
@@ -400,7 +405,7 @@ __device__ inline void leaf_ensure(const Pool<T>& P, uint32_t need, int n, V val
                 }
             } else {
                 uint64_t e;
-                claimed = ltab_claim(P, v, &w, &e);
+                claimed = ltab_claim(P, v, &w, &reused, &e);
                 if (claimed != ~0ull) wait |= (w ? 0u : 1u) << i;
             }
             won |= (w ? 1u : 0u) << i;
@@ -434,9 +439,17 @@ __device__ inline void leaf_ensure(const Pool<T>& P, uint32_t need, int n, V val
                     else store_agent(&P.ltab[claimed], ((uint64_t)v << 32) | idx);
                 } else if constexpr (sizeof(T) == 4) {
                     store_agent(&P.ltab[claimed], kLeafTomb);
+                    gave = true;
                 }
             }
             k += (uint32_t)__popcll(b);
+        }
+        if constexpr (sizeof(T) == 4) {
+            const int d = __popcll(__ballot(gave)) - __popcll(__ballot(reused));
+            if (d != 0 && (int)lane == leader) {
+                if (s_tomb) atomicAdd(s_tomb, (uint32_t)d);
+                else atomicAdd((unsigned long long*)stat(P.ctl, ST_LTOMB), (unsigned long long)(long long)d);
+            }
         }
     }
 #pragma unroll 1
@@ -645,6 +658,7 @@ __global__ void k_dry_leaves(Pool<T> P) {
                 created = P.leaf_ids[i] == kEmpty;
             }
         }
+        if (sizeof(T) == 4) wave_count(stat(P.ctl, ST_LTOMB), created);
         wave_append(&P.ctl->dry_new_leaves, created);
     }
 }
@@ -1446,7 +1460,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
                 const bool miss = k < nl && idx == 0;
                 if (__ballot(miss)) {
                     const uint32_t vv = miss ? (uint32_t)*cell : 0u;
-                    leaf_ensure(P, miss ? 1u : 0u, 1, [&](int) { return vv; });
+                    leaf_ensure(P, miss ? 1u : 0u, 1, [&](int) { return vv; }, &s_st[4]);
                     if (miss) idx = bid_index(leaf_now(P, vv));
                 }
                 if (cell) {
@@ -1589,10 +1603,10 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(R > 1 && s
     }
     __syncthreads();
     if (threadIdx.x < R) tile_cnt[blockIdx.x * R + threadIdx.x] = s_cnt[threadIdx.x];
-    const int ids[6] = {ST_CAND, ST_COLLAPSE, ST_H2, ST_MERGED, ST_CAND1, ST_MERGED1};
-    const int src[6] = {0, 1, 2, 3, 0, 3};
-    if (threadIdx.x < 6 && s_st[src[threadIdx.x]])
-        atomicAdd((unsigned long long*)stat(P.ctl, ids[threadIdx.x]), (unsigned long long)s_st[src[threadIdx.x]]);
+    const int ids[7] = {ST_CAND, ST_COLLAPSE, ST_H2, ST_MERGED, ST_CAND1, ST_MERGED1, ST_LTOMB};
+    const int src[7] = {0, 1, 2, 3, 0, 3, 4};
+    if (threadIdx.x < 7 && s_st[src[threadIdx.x]])  // (signed: the tombstones may become fewer)
+        atomicAdd((unsigned long long*)stat(P.ctl, ids[threadIdx.x]), (unsigned long long)(long long)(int32_t)s_st[src[threadIdx.x]]);
 }
 
 // ------------------------------------------------------------------ interning
