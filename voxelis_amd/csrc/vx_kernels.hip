@@ -2766,11 +2766,15 @@ __global__ __launch_bounds__(256) void k_gc_round(Pool<T> P, uint32_t round, con
 //
 // Every write call starts with the decision, made on the device in stream order
 // (so it stays current however many calls the host has queued): rebuild when the
-// tombstones take a sixteenth of the slots and live keys plus tombstones half of them
-// in the pattern table, or three quarters in the i32 leaf table (force: always).  Half
-// keeps a miss's scan to the next empty slot at about two probes; the rebuild (a clear
-// of the table and one insert per live branch) costs less than the longer scans of a
-// fuller table (measured on the 4096-tree uneven apply: 27.1 against 28.3 ms per step).
+// tombstones take a sixteenth of the slots and live keys plus tombstones half of them, or a
+// quarter when there are half as many tombstones as live keys (force: always).  A rebuild (a
+// clear of the table and one insert per live branch) is paid for by the frees since the last
+// one, so it may come early where the live keys are few beside them.  us of an apply, the mean
+// over whole rebuild cycles, at a half only, and so: 2048 uneven trees 10740, 10460; 400
+// uneven trees of 32^3 and 64^3 863, 785 (with half the memory, so twice the live share, 863
+// and 793); 200 scattered u16 trees of 64^3 642, 607; 333 scattered i32 trees 1429, 1397.  (At
+// three sixteenths for a quarter: 10395, 770, 602, 1400; but 824 with half the memory.)
+// The i32 leaf table holds three quarters, or a half when it has as many tombstones as leaves.
 // Every block of the clear kernel takes the decision (block 0 records it for the kernels
 // that follow); the clear and re-insert kernels return at once when no rebuild is due.
 // The control block's reset for the call that follows rides in block 0.
@@ -2793,8 +2797,8 @@ __global__ void k_tab_clear(uint64_t* tab, uint64_t nslots, Ctl* ctl, uint64_t* 
         }
         if (lane == 0) {
             const uint64_t live = ctl->live_branches, ll = ctl->live_leaves;
-            bool due = force != 0 || (t >= nslots / 16 && live + t > nslots / 2);
-            if (lslots) due = due || (lt >= lslots / 16 && ll + lt > lslots / 4 * 3);
+            bool due = force != 0 || (t >= nslots / 16 && live + t > (2 * t >= live ? nslots / 4 : nslots / 2));
+            if (lslots) due = due || (lt >= lslots / 16 && ll + lt > (lt >= ll ? lslots / 2 : lslots / 4 * 3));
             s_due = due ? (lslots ? 3u : 1u) : 0u;
             if (blockIdx.x == 0) {  // for the re-insertion
                 ctl->rebuild = s_due;
