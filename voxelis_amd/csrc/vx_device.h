@@ -134,6 +134,8 @@ struct Ctl {
     uint32_t dry_new_leaves;  // dry run: leaves that would be new
     uint32_t free_base;       // free_top when the last allocation window closed
     uint32_t unsorted;        // nodes freed before that since the free stack was last put in order
+    uint32_t sorted;          // the call's first kernel put it in order,
+    uint32_t sorted_top;      // ... with this many entries
     alignas(128) uint32_t free_top;      // entries on the free stack
     alignas(128) uint32_t alloc_count;   // branch nodes allocated in the current sequence (ranks after its new leaves)
     alignas(128) uint32_t n_new_leaves;  // leaves created in the current sequence: allocation ranks [0, n_new_leaves)

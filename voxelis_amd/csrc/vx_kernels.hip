@@ -722,6 +722,11 @@ template <typename T>
 __device__ inline void close_allocation(const Pool<T>& P, bool abort, uint32_t* counts) {
     Ctl* ctl = P.ctl;
     ctl->sort_cur = 0;
+    if (!P.dry) {
+        // (an apply's frees come after this; those of a fill came before, past its sort)
+        ctl->unsorted = ctl->sorted ? ctl->free_top - ctl->sorted_top : ctl->unsorted + (ctl->free_top - ctl->free_base);
+        ctl->free_base = ctl->free_top;
+    }
     if (abort) {
         if (counts) counts[0] = counts[1] = 0xFFFFFFFFu;
         return;
@@ -735,8 +740,6 @@ __device__ inline void close_allocation(const Pool<T>& P, bool abort, uint32_t* 
     ctl->live_branches += ctl->alloc_count;
     *stat(ctl, ST_LEAF_MISS) += made;
     if (P.dry) return;
-    // (free_top is still what the sequence began with: the frees come after this)
-    ctl->unsorted = sort_due(ctl) ? 0u : ctl->unsorted + (ctl->free_top - ctl->free_base);
     const uint32_t n = ctl->n_new_leaves + ctl->alloc_count;
     const uint32_t used_free = n < ctl->free_top0 ? n : ctl->free_top0;
     ctl->free_top = ctl->free_base = ctl->free_top0 - used_free;
@@ -2788,6 +2791,7 @@ __global__ void k_tab_clear(uint64_t* tab, uint64_t nslots, Ctl* ctl, uint64_t* 
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < up_n; i += gridDim.x * blockDim.x) up_dst[i] = up_src[i];
     static_assert(kStatStripes == 64, "one statistics stripe per lane");
     __shared__ uint32_t s_due;
+    const bool sort = !force && sort_due(ctl);  // uniform over the launch, which changes nothing it depends on
     if (threadIdx.x < 64) {  // every block takes the same decision from the same counters
         const int lane = (int)threadIdx.x;
         uint64_t t = ctl->st[lane][ST_TOMB], lt = ctl->st[lane][ST_LTOMB];
@@ -2803,11 +2807,13 @@ __global__ void k_tab_clear(uint64_t* tab, uint64_t nslots, Ctl* ctl, uint64_t* 
             if (blockIdx.x == 0) {  // for the re-insertion
                 ctl->rebuild = s_due;
                 if (due) ctl->rebuilds++;
+                ctl->sorted = sort ? 1u : 0u;
+                ctl->sorted_top = ctl->free_top;
                 ctl_begin(ctl);
             }
         }
     }
-    if (!force && sort_due(ctl)) sort_free(ctl, tmg, free_stack);  // uniform over the launch
+    if (sort) sort_free(ctl, tmg, free_stack);
     __syncthreads();
     if (!(s_due & 1u)) return;
     for (int k = 0; k < 2; k++) {  // both tables are rebuilt together
