@@ -669,9 +669,12 @@ __global__ void k_dry_leaves(Pool<T> P) {
 // each.  From 2^18 frees on, and a quarter of the stack: 2048 uneven u16 trees (13 M nodes
 // replaced per call) take 11.9 ms per call in the order of their frees and 10.75 ms so (GC 2.17
 // -> 1.89, commit 1.85 -> 1.53, probes 3.10 -> 2.60), 333 scattered i32 trees 1.80 -> 1.65 ms.
+// And a 32nd of the pool, whose column the sort reads: with 11.5 M nodes resident, calls that
+// free 45 k, 180 k and 830 k of them take 244, 405 and 1190 us unsorted, 247, 410 and 1145
+// sorted from 2^18 frees on, and 245, 404 and 1145 by this rule.
 __device__ inline bool sort_due(const Ctl* ctl) {
     const uint32_t u = ctl->unsorted + (ctl->free_top - ctl->free_base);
-    return u >= 1u << 18 && u >= ctl->free_top / 4;
+    return u >= 1u << 18 && u >= ctl->free_top / 4 && u >= ctl->next_index / 32;
 }
 
 // The stack written anew from the nodes marked free, in runs of index order (one run per
