@@ -305,11 +305,12 @@ struct ApplyOpts {
     const int32_t* set_xyz = nullptr;
     const void* set_values = nullptr;
     // edit lists: the views are the edited trees', orig[i] their index in the caller's arrays
-    // of nall trees, edits[i] their records; nedits edits (device) and nbricks workspace bricks
+    // of nall trees, edits[i] their records; nedits edits (device) from edit0 on and nbricks
+    // workspace bricks
     const EditTree* edits = nullptr;
     const uint32_t* orig = nullptr;
     size_t nall = 0;
-    uint64_t nedits = 0, nbricks = 0;
+    uint64_t edit0 = 0, nedits = 0, nbricks = 0;
     const int32_t* edit_xyz = nullptr;
     const void* edit_values = nullptr;
 };
@@ -592,12 +593,12 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     if (dedits) {
         // runs of up to 2048 edits per block, while there are eight blocks for each CU
         const uint32_t per = (uint32_t)std::min<uint64_t>(8, std::max<uint64_t>(1, opt.nedits / (2048 * 256)));
-        VX_LAUNCH(h, KID_EDIT_MARK, k_edit_mark, grid_for(std::max<uint64_t>(opt.nedits / per, opt.nall)), 256, opt.nedits, per, dedits,
+        VX_LAUNCH(h, KID_EDIT_MARK, k_edit_mark, grid_for(std::max<uint64_t>(opt.nedits / per, opt.nall)), 256, opt.edit0, opt.edit0 + opt.nedits, per, dedits,
                   (uint32_t)n, opt.edit_xyz, (uint32_t*)h->edit_win.ptr, (uint8_t*)h->edit_dirty.ptr, (uint32_t)opt.nall,
                   status, P.per_tree);
         if (opt.nbricks)
             VX_LAUNCH(h, KID_EDIT_BUILD, k_edit_build<T>, grid_for(opt.nbricks), 256, opt.nbricks,
-                      (const T*)opt.edit_values, (uint32_t*)h->edit_win.ptr, (uint8_t*)h->edit_dirty.ptr,
+                      (const T*)opt.edit_values + opt.edit0, (uint32_t*)h->edit_win.ptr, (uint8_t*)h->edit_dirty.ptr,
                       (uint16_t*)h->edit_masks.ptr, (T*)h->edit_values.ptr);
     }
     // chunk set-up, plus the old-tree descent over the level-3 slots in extra blocks
@@ -746,12 +747,11 @@ int apply_edits_impl(vx_interner* h, size_t n, uint64_t* roots, const uint8_t* d
     std::vector<EditTree> trees;
     std::vector<uint32_t> orig;
     uint64_t nvox = 0;
-    if (offsets[n] >= 0xFFFFFFFFull) return VX_E_INVALID_ARG;  // submission indices are 32 bits
     for (size_t t = 0; t < n; t++) {
         if (offsets[t + 1] < offsets[t]) return VX_E_INVALID_ARG;
         if (offsets[t + 1] == offsets[t]) continue;
         const uint32_t d = depths[t];
-        EditTree e{t ? offsets[t] : 0, ~0ull, d, 0};  // (edits before the first tree's are its own)
+        EditTree e{offsets[t], ~0ull, d, 0};
         if (d >= 2 && d <= (uint32_t)kMaxDepth) {  // (others fail with VX_E_DEPTH when planned)
             e.vbase = nvox;
             nvox += std::max<uint64_t>(slots_at(d, 0), 512);
@@ -759,6 +759,7 @@ int apply_edits_impl(vx_interner* h, size_t n, uint64_t* roots, const uint8_t* d
         trees.push_back(e);
         orig.push_back((uint32_t)t);
     }
+    if (offsets[n] - offsets[0] >= 0xFFFFFFFFull) return VX_E_INVALID_ARG;  // submission indices are 32 bits
     int rc = ensure_zero(h, h->edit_win, nvox * 4);
     if (!rc) rc = ensure_zero(h, h->edit_dirty, nvox / 512);
     if (rc) return rc;
@@ -773,7 +774,8 @@ int apply_edits_impl(vx_interner* h, size_t n, uint64_t* roots, const uint8_t* d
     opt.edits = trees.empty() ? &none : trees.data();
     opt.orig = orig.data();
     opt.nall = n;
-    opt.nedits = trees.empty() ? 0 : offsets[n];
+    opt.edit0 = offsets[0];
+    opt.nedits = offsets[n] - offsets[0];
     opt.nbricks = nvox / 8;
     opt.edit_xyz = xyz;
     opt.edit_values = values;

@@ -37,12 +37,12 @@ __device__ inline uint32_t tree_of_edit(const EditTree* trees, uint32_t lo, uint
     return lo;
 }
 
-// Per edit: win[voxel] = the largest submission index + 1, and the voxel's cell of 8^3 is
-// marked dirty.  A coordinate outside its tree (a panic in the reference's Vec indexing)
+// Per edit e of [first, n): win[voxel] = the largest submission index (counted from first) + 1,
+// and the voxel's cell of 8^3 is marked dirty.  A coordinate outside its tree (a panic in the reference's Vec indexing)
 // fails the tree.  A block's run of edits (per * 256) mostly lies in one tree, found once.
 // Bound by the rate of the atomics.  Lanes also reset the status and count of every tree of
 // the call, edited or not (a tree without edits is not applied: status 0).
-__global__ __launch_bounds__(256) void k_edit_mark(uint64_t n, uint32_t per, EditTree* trees, uint32_t ntrees,
+__global__ __launch_bounds__(256) void k_edit_mark(uint64_t first, uint64_t n, uint32_t per, EditTree* trees, uint32_t ntrees,
                                                    const int32_t* xyz, uint32_t* win, uint8_t* dirty, uint32_t nall,
                                                    int32_t* status, uint32_t* per_tree) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nall; i += gridDim.x * blockDim.x) {
@@ -51,7 +51,7 @@ __global__ __launch_bounds__(256) void k_edit_mark(uint64_t n, uint32_t per, Edi
     }
     __shared__ uint32_t s_t[2];
     const uint64_t run = (uint64_t)per * 256;
-    for (uint64_t e0 = (uint64_t)blockIdx.x * run; e0 < n; e0 += (uint64_t)gridDim.x * run) {
+    for (uint64_t e0 = first + (uint64_t)blockIdx.x * run; e0 < n; e0 += (uint64_t)gridDim.x * run) {
         const uint64_t e1 = min(e0 + run, n);
         if (threadIdx.x < 2) s_t[threadIdx.x] = tree_of_edit(trees, 0, ntrees, threadIdx.x ? e1 - 1 : e0);
         __syncthreads();
@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) void k_edit_mark(uint64_t n, uint32_t per, Edi
         for (uint64_t e = e0 + threadIdx.x; e < e1; e += 256) {
             const uint32_t t = t0 == t1 ? t0 : tree_of_edit(trees, t0, t1 + 1, e);
             const EditTree tr = trees[t];
-            if (tr.vbase == ~0ull || e < tr.first) continue;  // rejected on the host; of no tree
+            if (tr.vbase == ~0ull) continue;  // rejected on the host
             const uint32_t x = (uint32_t)xyz[3 * e], y = (uint32_t)xyz[3 * e + 1], z = (uint32_t)xyz[3 * e + 2];
             const uint32_t lim = 1u << tr.depth;
             if (x >= lim || y >= lim || z >= lim) {  // (negative coordinates too)
@@ -68,7 +68,7 @@ __global__ __launch_bounds__(256) void k_edit_mark(uint64_t n, uint32_t per, Edi
                 continue;
             }
             const uint64_t v = tr.vbase + (spread3(x) | (spread3(y) << 1) | (spread3(z) << 2));
-            atomicMax(&win[v], (uint32_t)e + 1u);
+            atomicMax(&win[v], (uint32_t)(e - first) + 1u);
             dirty[v >> 9] = 1;
         }
     }
