@@ -179,7 +179,9 @@ int vx_tree_apply_batch_host(vx_interner* h, uint64_t* root, const vx_batch_view
  * submission indices of each voxel).  depths and edit_offsets (n+1 entries) are
  * host arrays; roots, xyz, values and status are device arrays.  A coordinate
  * outside the tree fails that tree with VX_E_RANGE (the reference's Vec index
- * panics).  Asynchronous. */
+ * panics).  The call keeps value_size + 1/4 bytes of workspace per voxel of an edited
+ * tree, and 4 per voxel of up to 2^27 of them; a tree with 2^32 - 1 edits or more is
+ * refused (VX_E_INVALID_ARG).  Asynchronous. */
 int vx_trees_apply_edits(vx_interner* h, size_t n, uint64_t* roots, const uint8_t* depths,
                          const uint64_t* edit_offsets, const int32_t* xyz, const void* values,
                          int32_t* status);

@@ -297,6 +297,12 @@ hipEvent_t prof_event(vx_interner* h) {
     } while (0)
 
 // Options of one apply (vx_apply_opts, validated by the caller).
+// Consecutive edited trees [t0, t1) of an edit-list call, their edits and workspace voxels.
+struct EditWindow {
+    uint64_t e0, e1, v0, v1;
+    uint32_t t0, t1;
+};
+
 struct ApplyOpts {
     bool dry = false;
     uint32_t alloc_limit = 0xFFFFFFFFu;
@@ -305,15 +311,20 @@ struct ApplyOpts {
     const int32_t* set_xyz = nullptr;
     const void* set_values = nullptr;
     // edit lists: the views are the edited trees', orig[i] their index in the caller's arrays
-    // of nall trees, edits[i] their records; nedits edits (device) from edit0 on and nbricks
-    // workspace bricks
+    // of nall trees, edits[i] their records; edit_windows: the windows that they are taken in
     const EditTree* edits = nullptr;
     const uint32_t* orig = nullptr;
     size_t nall = 0;
-    uint64_t edit0 = 0, nedits = 0, nbricks = 0;
+    const std::vector<EditWindow>* edit_windows = nullptr;
     const int32_t* edit_xyz = nullptr;
     const void* edit_values = nullptr;
 };
+
+// Voxels of one window of an edit-list call: 512 MiB of winners (64 trees of 128^3, 4096 of
+// 32^3), beside which a window's two launches are short.  The dense batch form needs the Batch
+// buffers only, so the winners of all of a large call at once would keep worlds from being
+// edited that fit otherwise (u16: 4 bytes per voxel beside 2.25).
+constexpr uint64_t kEditWindow = 1ull << 27;
 
 constexpr unsigned kRebuildGrid = 512;
 template <typename T>
@@ -591,15 +602,20 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
         if (rc) return rc;
     } else {
     if (dedits) {
-        // runs of up to 2048 edits per block, while there are eight blocks for each CU
-        const uint32_t per = (uint32_t)std::min<uint64_t>(8, std::max<uint64_t>(1, opt.nedits / (2048 * 256)));
-        VX_LAUNCH(h, KID_EDIT_MARK, k_edit_mark, grid_for(std::max<uint64_t>(opt.nedits / per, opt.nall)), 256, opt.edit0, opt.edit0 + opt.nedits, per, dedits,
-                  (uint32_t)n, opt.edit_xyz, (uint32_t*)h->edit_win.ptr, (uint8_t*)h->edit_dirty.ptr, (uint32_t)opt.nall,
-                  status, P.per_tree);
-        if (opt.nbricks)
-            VX_LAUNCH(h, KID_EDIT_BUILD, k_edit_build<T>, grid_for(opt.nbricks), 256, opt.nbricks,
-                      (const T*)opt.edit_values + opt.edit0, (uint32_t*)h->edit_win.ptr, (uint8_t*)h->edit_dirty.ptr,
-                      (uint16_t*)h->edit_masks.ptr, (T*)h->edit_values.ptr);
+        uint32_t nall = (uint32_t)opt.nall;  // (the first launch resets every tree's status)
+        for (const EditWindow& w : *opt.edit_windows) {
+            // runs of up to 2048 edits per block, while there are eight blocks for each CU
+            const uint64_t ne = w.e1 - w.e0, nbr = (w.v1 - w.v0) / 8;
+            const uint32_t per = (uint32_t)std::min<uint64_t>(8, std::max<uint64_t>(1, ne / (2048 * 256)));
+            VX_LAUNCH(h, KID_EDIT_MARK, k_edit_mark, grid_for(std::max<uint64_t>(ne / per, nall)), 256, w.e0, w.e1, per,
+                      dedits + w.t0, w.t1 - w.t0, opt.edit_xyz, w.v0, (uint32_t*)h->edit_win.ptr,
+                      (uint8_t*)h->edit_dirty.ptr, nall, status, P.per_tree);
+            nall = 0;
+            if (nbr)
+                VX_LAUNCH(h, KID_EDIT_BUILD, k_edit_build<T>, grid_for(nbr), 256, nbr, (const T*)opt.edit_values + w.e0,
+                          (uint32_t*)h->edit_win.ptr, (uint8_t*)h->edit_dirty.ptr,
+                          (uint16_t*)h->edit_masks.ptr + w.v0 / 8, (T*)h->edit_values.ptr + w.v0);
+        }
     }
     // chunk set-up, plus the old-tree descent over the level-3 slots in extra blocks
     unsigned np = grid_for(n);
@@ -746,22 +762,35 @@ int apply_edits_impl(vx_interner* h, size_t n, uint64_t* roots, const uint8_t* d
     ApplyOpts opt = opts;
     std::vector<EditTree> trees;
     std::vector<uint32_t> orig;
-    uint64_t nvox = 0;
+    std::vector<EditWindow> windows(1, EditWindow{offsets[0], offsets[0], 0, 0, 0, 0});
+    uint64_t nvox = 0, most = 0;  // voxels of all edited trees, of the largest window
     for (size_t t = 0; t < n; t++) {
         if (offsets[t + 1] < offsets[t]) return VX_E_INVALID_ARG;
         if (offsets[t + 1] == offsets[t]) continue;
         const uint32_t d = depths[t];
         EditTree e{offsets[t], ~0ull, d, 0};
+        uint64_t nv = 0;
         if (d >= 2 && d <= (uint32_t)kMaxDepth) {  // (others fail with VX_E_DEPTH when planned)
             e.vbase = nvox;
-            nvox += std::max<uint64_t>(slots_at(d, 0), 512);
+            nv = std::max<uint64_t>(slots_at(d, 0), 512);
         }
+        // submission indices are 32 bits, counted from the window's first edit
+        if (offsets[t + 1] - offsets[t] >= 0xFFFFFFFFull) return VX_E_INVALID_ARG;
+        if (nvox + nv - windows.back().v0 > kEditWindow || offsets[t + 1] - windows.back().e0 >= 0xFFFFFFFFull) {
+            const uint32_t i = (uint32_t)trees.size();
+            windows.push_back(EditWindow{offsets[t], offsets[t], nvox, nvox, i, i});
+        }
+        nvox += nv;
         trees.push_back(e);
         orig.push_back((uint32_t)t);
+        EditWindow& w = windows.back();
+        w.e1 = offsets[t + 1];
+        w.v1 = nvox;
+        w.t1 = (uint32_t)trees.size();
+        most = std::max(most, w.v1 - w.v0);
     }
-    if (offsets[n] - offsets[0] >= 0xFFFFFFFFull) return VX_E_INVALID_ARG;  // submission indices are 32 bits
-    int rc = ensure_zero(h, h->edit_win, nvox * 4);
-    if (!rc) rc = ensure_zero(h, h->edit_dirty, nvox / 512);
+    int rc = ensure_zero(h, h->edit_win, most * 4);
+    if (!rc) rc = ensure_zero(h, h->edit_dirty, most / 512);
     if (rc) return rc;
     if (!h->edit_masks.ensure(nvox / 4) || !h->edit_values.ensure(nvox * sizeof(T))) return VX_E_HIP;
     std::vector<vx_batch_view> views(trees.size());
@@ -774,9 +803,7 @@ int apply_edits_impl(vx_interner* h, size_t n, uint64_t* roots, const uint8_t* d
     opt.edits = trees.empty() ? &none : trees.data();
     opt.orig = orig.data();
     opt.nall = n;
-    opt.edit0 = offsets[0];
-    opt.nedits = offsets[n] - offsets[0];
-    opt.nbricks = nvox / 8;
+    opt.edit_windows = &windows;
     opt.edit_xyz = xyz;
     opt.edit_values = values;
     return apply_impl<T>(h, trees.size(), roots, views.data(), status, opt);

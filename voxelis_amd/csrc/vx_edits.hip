@@ -10,6 +10,8 @@
 // its eight winners and leaves their array zero again.  (A stable radix sort by (tree, Morton
 // path), whose run ends were scattered and later cleared, took 23 launches and 640 us on 4.4 M
 // sphere edits over 700 trees of 32^3 against 93 us here; 18 launches against 2 on 3000 edits.)
+// The winners take four bytes per voxel, so a call of very many voxels goes in windows of
+// consecutive trees, two launches each, that share one array of them (kEditWindow).
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -37,13 +39,13 @@ __device__ inline uint32_t tree_of_edit(const EditTree* trees, uint32_t lo, uint
     return lo;
 }
 
-// Per edit e of [first, n): win[voxel] = the largest submission index (counted from first) + 1,
-// and the voxel's cell of 8^3 is marked dirty.  A coordinate outside its tree (a panic in the reference's Vec indexing)
+// Per edit e of [first, n): win[voxel - v0] = the largest submission index (counted from first)
+// + 1, and the voxel's cell of 8^3 is marked dirty.  A coordinate outside its tree (a panic in the reference's Vec indexing)
 // fails the tree.  A block's run of edits (per * 256) mostly lies in one tree, found once.
 // Bound by the rate of the atomics.  Lanes also reset the status and count of every tree of
 // the call, edited or not (a tree without edits is not applied: status 0).
 __global__ __launch_bounds__(256) void k_edit_mark(uint64_t first, uint64_t n, uint32_t per, EditTree* trees, uint32_t ntrees,
-                                                   const int32_t* xyz, uint32_t* win, uint8_t* dirty, uint32_t nall,
+                                                   const int32_t* xyz, uint64_t v0, uint32_t* win, uint8_t* dirty, uint32_t nall,
                                                    int32_t* status, uint32_t* per_tree) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nall; i += gridDim.x * blockDim.x) {
         status[i] = 0;
@@ -67,7 +69,7 @@ __global__ __launch_bounds__(256) void k_edit_mark(uint64_t first, uint64_t n, u
                 trees[t].status = -4;
                 continue;
             }
-            const uint64_t v = tr.vbase + (spread3(x) | (spread3(y) << 1) | (spread3(z) << 2));
+            const uint64_t v = tr.vbase - v0 + (spread3(x) | (spread3(y) << 1) | (spread3(z) << 2));
             atomicMax(&win[v], (uint32_t)(e - first) + 1u);
             dirty[v >> 9] = 1;
         }
