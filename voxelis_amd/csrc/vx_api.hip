@@ -861,10 +861,7 @@ int get_grouped_impl(vx_interner* h, hipStream_t st, size_t ntrees, const uint64
     // about 4096 blocks for large batches; at least 512 queries per block
     uint64_t per = std::min<uint64_t>(4096, std::max<uint64_t>(512, (nq + 4095) / 4096));
     per = (per + kGetTile - 1) / kGetTile * kGetTile;
-    // the last quarter of the queries in runs half as long: blocks over deep, dense trees take
-    // several times as long as the rest, and as the last ones they left the chip idle (9 M
-    // queries of 777 uneven u16 trees 148 us, 134 so; 16 M of 4096 terrain trees 127 and 121;
-    // runs of a quarter 133 and 123, the whole call in runs of 1024 135 and 147)
+    // the last quarter of the queries in runs half as long, where the kernel finds deep trees
     const uint64_t per2 = std::max<uint64_t>(512, per / 2 / kGetTile * kGetTile);
     const uint64_t nlong = nq / per * 3 / 4;
     const uint64_t blocks = nlong + (nq - nlong * per + per2 - 1) / per2;

@@ -3174,13 +3174,23 @@ __global__ void k_get(Pool<T> P, uint64_t nq, uint64_t ntrees, const uint64_t* r
 }
 
 // get for queries grouped by tree: tree t's queries are [qoff[t], qoff[t+1]).  A block
-// takes `per` consecutive queries, one from the nlong-th on `per2`.  For each tree its range meets, the block first walks
+// takes a run of `per` consecutive queries; from the nlong-th on one of `per2`, when there are
+// deep trees, of kGetDeep levels or more.  Blocks over deep, dense trees take several times as
+// long as the others, and as the last ones they left the chip idle; over shallow trees more
+// stagings of a tree cost more than they give (the blocks that are not needed then are the
+// last of the grid).  The trees are looked at by a sample of TILE.  us, the last quarter in
+// whole runs, in half ones, and so: 9 M queries of 777 uneven u16 trees 153, 142, 142; 15 M of 300
+// uneven trees of 32^3 and 64^3 170, 155, 155; 16 M of 4096 terrain trees of 32^3 150, 155, 150; 10.4 M of 4 of
+// them 89, 92, 89.
+//
+// For each tree its range meets, the block first walks
 // every path of the tree's top k levels (k = 3 for a segment of at least 256 queries,
 // 2 from 32, else none) and keeps the node each path reaches in LDS; a query then takes
 // the node of its first k child digits from there and walks the rest in HBM
 // (utils/common.rs:122-156): a depth-5 read makes three dependent loads instead of six.
 // A query outside its tree, or beyond qoff[ntrees], is VX_E_RANGE (present 0xFF).
 constexpr uint32_t kGetTop = 3;
+constexpr uint32_t kGetDeep = 6;
 template <typename T, int TILE>
 __global__ __launch_bounds__(TILE) void k_get_grouped(Pool<T> P, uint64_t nq, uint32_t ntrees,
                                                       const uint64_t* roots, const uint8_t* depths,
@@ -3190,9 +3200,15 @@ __global__ __launch_bounds__(TILE) void k_get_grouped(Pool<T> P, uint64_t nq, ui
     __shared__ uint64_t s_node[1u << (3 * kGetTop)];
     __shared__ uint8_t s_dep[1u << (3 * kGetTop)];
     __shared__ uint32_t s_lo;
-    const uint32_t n = blockIdx.x < nlong ? per : per2;
-    uint64_t q0 = blockIdx.x < nlong ? (uint64_t)blockIdx.x * per
-                                     : (uint64_t)nlong * per + (uint64_t)(blockIdx.x - nlong) * n;
+    uint32_t n = per;
+    uint64_t q0 = (uint64_t)blockIdx.x * per;
+    if (blockIdx.x >= nlong && ntrees) {
+        const bool deep = depths[(uint64_t)threadIdx.x * ntrees / TILE] >= kGetDeep;
+        if (__syncthreads_or(deep)) {
+            n = per2;
+            q0 = (uint64_t)nlong * per + (uint64_t)(blockIdx.x - nlong) * n;
+        }
+    }
     const uint64_t q1 = min(nq, q0 + n);
     if (q0 >= q1) return;
     // the tree holding q0, the last t with qoff[t] <= q0: a TILE-way search per round
