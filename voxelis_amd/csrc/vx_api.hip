@@ -883,8 +883,10 @@ int to_vec_impl(vx_interner* h, size_t n, const uint64_t* roots, const uint8_t* 
     Pool<T> P = pool_of<T>(h);
     // a lane per voxel for trees of at most 4^3 voxels, and for extractions that give every
     // CU's lanes at most a few voxels each: their time is one walk's, and the cells' kernel
-    // has two more loads in a row (one tree of 32^3: 1.5 us longer)
-    if (stride <= 64 || (uint64_t)n * stride <= (1u << 19)) {
+    // has two more loads in a row.  us by lanes and by cells, 20, 24 and 28 uneven trees of 64^3
+    // at half resolution (32^3 places each, half of them in use) 4.8 and 5.6, 5.2 and 5.5, 5.8
+    // and 5.5; 16, 24 and 32 terrain trees of 32^3 4.6 and 4.9, 5.2 and 4.9, 6.1 and 4.9
+    if (stride <= 64 || (uint64_t)n * stride <= 25u << 15) {
         VX_LAUNCH(h, KID_TO_VEC, k_to_vec_small<T>, grid_for((uint64_t)n * stride), kBlock, P, (uint64_t)n, roots, depths,
                   lod, stride, (T*)out);
     } else {
