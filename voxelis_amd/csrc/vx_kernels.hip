@@ -3447,7 +3447,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
             }
             // lane l: the node of the brick with digits l >> 3 and l & 7 (x | y << 1 | z << 2)
             uint64_t nd = dense_step(P, dense_step(P, cn, lane >> 3), lane & 7u);
-            if (nd != kEmpty && bid_index(nd) >= P.capacity) nd = kEmpty;
+            if (nd != kEmpty && bid_index(nd) >= P.capacity) {
+                if (!bid_is_leaf(nd)) atomicOr(&P.ctl->err, kErrPoison);  // as dense_step
+                nd = kEmpty;
+            }
             // its eight values, two per lane of four: bricks 16 j + lane / 4 in round j
             ulonglong2 ch[4];
 #pragma unroll
