@@ -1016,7 +1016,7 @@ int vx_interner_destroy(vx_interner* h) {
     h->owners.release();
     for (Plan& pl : h->plans) pl.release();
     if (h->cap_stream) (void)hipStreamDestroy(h->cap_stream);
-    for (Grow* g : {&h->edit_win, &h->edit_dirty, &h->edit_masks, &h->edit_values})
+    for (Grow* g : {&h->set_rec, &h->set_meta, &h->edit_win, &h->edit_dirty, &h->edit_masks, &h->edit_values})
         g->release();
     for (auto& b : h->lv) {
         b.res.release();
