@@ -655,8 +655,8 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
     VX_LAUNCH(h, KID_COMMIT, k_commit<T VX_COMMA TILE>, (unsigned)std::min<uint64_t>(std::max<uint64_t>(cg, 1), h->tune.commit_grid),
               TILE, P, dchunks, ddrift, LT, (uint32_t)n, dmap, dres, dcid, roots, status, gf0, opt.counts);
     if (!opt.dry) {
-        // dec_ref_recursive of the replaced roots: a tree of depth D has nodes at
-        // heights D..0, one round each; the first round also releases unused new leaves.
+        // dec_ref_recursive of the replaced roots in a few rounds (gc_rounds), the last of
+        // which goes down to the leaves; the first also releases unused new leaves.
         // A small front is split over the blocks in shares of kGcShareMin nodes and
         // followed locally: the first round takes one block per share of the replaced
         // roots (every block of that round also runs the leaf release), the later ones

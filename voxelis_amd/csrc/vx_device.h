@@ -148,7 +148,7 @@ struct Ctl {
 };
 
 // Per-tree record of one apply launch sequence (trees sorted by depth on the host).
-struct ChunkDev {  // 8-byte aligned; depth .. skip form one dword (read as such)
+struct ChunkDev {  // 8-byte aligned
     const uint8_t* masks;
     const void* values;
     uint64_t fill;
@@ -159,15 +159,11 @@ struct ChunkDev {  // 8-byte aligned; depth .. skip form one dword (read as such
     uint8_t depth;
     uint8_t has_fill;
     uint8_t has_patches;
-    uint8_t skip;  // not applied at all (an edit-list tree without edits)
+    uint8_t skip;  // nothing changes (a set of a voxel that holds the value already)
     int32_t status0;  // status before the launch (a replayed launch starts from it)
     uint32_t sub;     // index among the call's records as the caller listed them (its EditTree)
     uint32_t pad;
 };
-static_assert(offsetof(ChunkDev, depth) % 4 == 0 && offsetof(ChunkDev, has_fill) == offsetof(ChunkDev, depth) + 1 &&
-                  offsetof(ChunkDev, has_patches) == offsetof(ChunkDev, depth) + 2,
-              "the flag bytes are read as one dword");
-
 // One edited tree of an edit-list call.
 struct EditTree {
     uint64_t first;  // its first edit

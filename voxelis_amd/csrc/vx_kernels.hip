@@ -83,24 +83,7 @@ __device__ inline void wave_add64(uint64_t* st, uint32_t v) {
 constexpr uint32_t kNoIdx = 0xFFFFFFFFu;
 constexpr int kMatchRounds = 4;
 
-// refs[idx] += 1 for every lane with idx != kNoIdx; lanes with equal idx share one
-// atomic (hot leaves are referenced from most new nodes).
-__device__ inline void wave_ref_inc(uint32_t* refs, uint32_t idx) {
-    bool pending = idx != kNoIdx;
-    for (int r = 0; r < kMatchRounds; r++) {
-        uint64_t act = __ballot(pending);
-        if (!act) return;
-        int leader = __ffsll((unsigned long long)act) - 1;
-        uint32_t li = __shfl(idx, leader);
-        bool same = pending && idx == li;
-        uint64_t sm = __ballot(same);
-        if ((int)__lane_id() == leader) atomicAdd(&refs[li], (uint32_t)__popcll(sm));
-        if (same) pending = false;
-    }
-    if (pending) atomicAdd(&refs[idx], 1u);
-}
-
-// refs[idx] -= 1 for every lane with idx != kNoIdx (aggregated like wave_ref_inc).
+// refs[idx] -= 1 for every lane with idx != kNoIdx; lanes with equal idx share one atomic.
 // Returns true on exactly one lane per index whose count reached zero.  Every round's
 // atomic is issued before any result is read, so they are in flight together.
 __device__ inline bool wave_ref_dec_zero(uint32_t* refs, uint32_t idx) {
@@ -584,37 +567,12 @@ __device__ inline GroupPos group_of(const LevelInfo& L, const BlockGroup& B, uin
     return B.one ? B.G : group_pos(L, slot);
 }
 
-// The fields of a chunk record that the build passes read first.  A wavefront whose
-// lanes all lie in one chunk (every wavefront of a tree of depth >= 3 at the brick
-// level) reads them with scalar loads: vector-memory address processing is what
-// bounds these passes, and a wave-wide load of one address costs as much of it as
-// any other.
-struct ChunkHead {
-    const uint8_t* masks;
-    const void* values;
-    uint64_t root_in;
-    uint64_t init;
-    int32_t status;
-    bool has_fill;
-    bool has_patches;
-};
-
-typedef const __attribute__((address_space(4))) ChunkDev ConstChunk;  // read-only view: scalar loads
-
-// (A record's status may be set negative by another wavefront of the same pass; a
-// reader that misses it is covered by the probe's own status check.)
-__device__ inline ChunkHead chunk_head(const ChunkDev* chunks, uint32_t c) {
-    const uint32_t c0 = __builtin_amdgcn_readfirstlane(c);
-    if (__ballot(c != c0) == 0) {
-        ConstChunk& r = *(ConstChunk*)(chunks + c0);
-        // the four flag bytes (depth, has_fill, has_patches, skip) as one dword
-        const uint32_t flags = *(const __attribute__((address_space(4))) uint32_t*)&r.depth;
-        return ChunkHead{r.masks, r.values, r.root_in, r.init, r.status, ((flags >> 8) & 0xFFu) != 0,
-                         ((flags >> 16) & 0xFFu) != 0};
-    }
-    const ChunkDev& r = chunks[c];
-    return ChunkHead{r.masks, r.values, r.root_in, r.init, r.status, r.has_fill != 0, r.has_patches != 0};
-}
+// A chunk record read by a wavefront whose lanes all lie in one chunk (every wavefront of a
+// tree of depth >= 3 at the brick level): scalar loads, since a wave-wide load of one address
+// costs the vector-memory units as much as any other.  (A record's status may be set negative
+// by another wavefront of the same pass; a reader that misses it is covered by the probe's own
+// status check.)
+typedef const __attribute__((address_space(4))) ChunkDev ConstChunk;
 
 // ------------------------------------------------------------------ launch setup
 
@@ -956,7 +914,8 @@ __device__ inline bool vox8_equal(const V& a, const V& b) {
     return eq;
 }
 
-// Hash of a brick's eight values (products of pairs of words, as in branch_hash).
+// Hash of a brick's eight values: products of pairs of words, as in branch_hash, then the
+// first two thirds of MurmurHash3's 32-bit finalizer (A. Appleby, public domain).
 template <typename V>
 __device__ inline uint32_t vox8_hash(const V& v) {
     const uint32_t* w = (const uint32_t*)&v;
@@ -965,8 +924,8 @@ __device__ inline uint32_t vox8_hash(const V& v) {
     for (int i = 0; i < (int)(sizeof(V) / 4); i += 2)
         s += (uint64_t)(w[i] + 0x4ABEA221u + 0x3A1B5D06u * i) * (w[i + 1] + 0x23148989u + 0x5DCE1B54u * i);
     uint32_t x = (uint32_t)s ^ (uint32_t)(s >> 32);
-    x ^= x >> 15;
-    x *= 0x2C1B3C6Du;
+    x ^= x >> 16;
+    x *= 0x85EBCA6Bu;
     return x ^ (x >> 13);
 }
 
@@ -2455,12 +2414,12 @@ __device__ inline void leaf_cleanup_body(const Pool<T>& P) {
 // in the same launch, while they fit one pass (kGcLocal); more go to the next launch.
 // Only the block whose decrement took a count to zero holds that node, so no other
 // block has to see it, and a chain of small rounds (a few thousand replaced paths) costs
-// one launch instead of one per height.  A launch frees nodes of any depth at or below
-// its round's, so the D + 1 launches of a tree of depth D still reach every node.
+// one launch instead of one per height.
 //
 // The final round takes a front of any size that way and hands nothing on: children past a
-// pass wait in the block's own runs of the next queue.  It ends the rounds early
-// (gc_rounds, with the times).
+// pass wait in the block's own runs of the next queue, and the block goes on until its share
+// and its runs are empty.  So every node that reaches zero is freed, whatever the depth of
+// the trees and the number of rounds before it (gc_rounds, with the times).
 constexpr uint32_t kGcStage = 2048;      // children staged per pass (8 per lane of a 256-lane block)
 constexpr uint32_t kGcLocal = 256;       // the most nodes of one pass a block follows itself
 constexpr uint32_t kGcLocalShare = 64;   // a front up to this many nodes per block is followed
@@ -2946,7 +2905,7 @@ __global__ void k_set_descend(Pool<T> P, ChunkDev* chunks, uint32_t n, const uin
 
 // One height of the set / remove paths (one slot per tree): the node at depth
 // D - h from the result one height below, as voxtree.rs:476-555 (set) and
-// voxtree.rs:597-705 (remove) build it.  Blocks nbuild.. commit height h-1.
+// voxtree.rs:597-705 (remove) build it.
 template <typename T, int TILE>
 __global__ __launch_bounds__(TILE) void k_set_level(
     Pool<T> P, const ChunkDev* chunks, LevelInfo L, const int32_t* xyz,
@@ -2979,9 +2938,8 @@ __global__ __launch_bounds__(TILE) void k_set_level(
             uint64_t cur;
             if (L.h == 1) {
                 if (v != 0) {
-                    // creation failed: the apply aborts; a dry run counts a placeholder
-                    uint32_t li = leaf_index(P, v);
-                    cur = li ? make_leaf(li, tmg_gen(P.tmg[li])) : (P.dry ? make_leaf(P.capacity + v, 0) : kInvalid);
+                    const uint32_t li = leaf_index(P, v);  // 0: its creation failed, the call aborts
+                    cur = li ? make_leaf(li, tmg_gen(P.tmg[li])) : kInvalid;
                 } else {
                     cur = kEmpty;
                 }

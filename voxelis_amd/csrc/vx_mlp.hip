@@ -44,11 +44,13 @@ struct MlpLds {  // odd row lengths: a column walk meets every bank
 // parameter's gradient, accumulated in registers over its tiles and written to
 // part[block][kMlpPart] (or, by a single block, to grad and loss).
 //
-// The tile is 64 samples because one tile's 14 k MFMA cycles per SIMD are about what its
-// loads and barriers take, and a batch of 8192 then gives 128 blocks.  The form it replaces
-// wrote 1 KB per sample to memory and reduced it with one lane per parameter, a chain of n
-// dependent loads: a training step of 8192 rows (gradient and Adam) took 2067 us and takes
-// 24 us now, which is the host's time to call it.
+// The tile is 64 samples: a row block of the products for each wavefront, 224 products of it
+// per tile (about 7.2 k cycles of its SIMD's matrix unit), and 128 blocks for a batch of 8192.
+// The form it replaces wrote 1 KB per sample to memory and reduced it with one lane per
+// parameter, a chain of n dependent loads: a training step of 8192 rows (gradient and Adam)
+// took 2067 us and takes 24 us now, which is the host's time to call it.  The sums are shorter
+// so: the gradient's error against 64 bits (2-norm, mean of 12 seeds) is 6e-8 for 64 rows,
+// 4e-8 for 1000 and 7e-7 for 8192, where the one chain had 1.1e-7, 4e-7 and 1.7e-6.
 template <bool BACK>
 __global__ __launch_bounds__(256) void k_mlp(const float* P, const float* x, uint32_t n, float* y,
                                              const float* target, float* part, float* grad, float* loss) {
