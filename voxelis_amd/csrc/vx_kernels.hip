@@ -485,13 +485,18 @@ __device__ inline void leaf_remove(const Pool<T>& P, uint32_t v) {
     }
 }
 
+// Every allocation past the limit comes here: one of them, not each, updates the word.
+__device__ inline void set_abort(Ctl* ctl, uint32_t bit) {
+    if (!(load_agent(&ctl->abort_) & bit)) atomicOr(&ctl->abort_, bit);
+}
+
 // The index of the launch sequence's k-th allocation: the free stack first, then
 // fresh indices.  ft0 / next0: the allocation window's snapshot (free_top0, next0), which
 // no kernel of the sequence changes before the window is closed.
 template <typename T>
 __device__ inline uint32_t alloc_at(const Pool<T>& P, uint32_t k, bool* ok, uint32_t ft0, uint32_t next0) {
     if (k >= P.alloc_limit) {
-        atomicOr(&P.ctl->abort_, 2u);  // beyond the caller's reservation
+        set_abort(P.ctl, 2u);  // beyond the caller's reservation
         *ok = false;
         return 0;
     }
@@ -501,7 +506,7 @@ __device__ inline uint32_t alloc_at(const Pool<T>& P, uint32_t k, bool* ok, uint
     }
     uint64_t b = (uint64_t)next0 + (uint64_t)(k - ft0);
     if (b >= P.capacity) {
-        atomicOr(&P.ctl->abort_, 1u);  // interner capacity (interner/macros.rs:37-38)
+        set_abort(P.ctl, 1u);  // interner capacity (interner/macros.rs:37-38)
         *ok = false;
         return 0;
     }
