@@ -168,8 +168,10 @@ struct vx_interner {
     // workspace
     Grow records, gc_front[2], stage, scratch, drift, undo, owners;
     Grow set_rec, set_meta;  // single-voxel set: the recorded path of every tree
-    // edit lists: the winners of every voxel and the dirty cells (kept zero), Batch buffers
+    // edit lists: the winners of a window's voxels (kept zero); Batch buffers of edit_voxels
+    // voxels, the masks zero but for the cells that the last calls left as built
     Grow edit_win, edit_dirty, edit_masks, edit_values;
+    uint64_t edit_voxels = 0;
     LevelBufs lv[kLevels + 1];
     // pinned staging ring: a slot is reused only after its copies completed
     static constexpr int kRing = 8;
@@ -605,16 +607,19 @@ int apply_tiled(vx_interner* h, size_t n, uint64_t* roots, const vx_batch_view* 
         uint32_t nall = (uint32_t)opt.nall;  // (the first launch resets every tree's status)
         for (const EditWindow& w : *opt.edit_windows) {
             // runs of up to 2048 edits per block, while there are eight blocks for each CU
-            const uint64_t ne = w.e1 - w.e0, nbr = (w.v1 - w.v0) / 8;
+            // a wavefront per cell, several cells where there are many (k_edit_build)
+            const uint64_t ne = w.e1 - w.e0, cells = (w.v1 - w.v0) / 512;
+            const uint32_t cper = (uint32_t)std::min<uint64_t>(64, std::max<uint64_t>(1, cells / 65536));
             const uint32_t per = (uint32_t)std::min<uint64_t>(8, std::max<uint64_t>(1, ne / (2048 * 256)));
             VX_LAUNCH(h, KID_EDIT_MARK, k_edit_mark, grid_for(std::max<uint64_t>(ne / per, nall)), 256, w.e0, w.e1, per,
                       dedits + w.t0, w.t1 - w.t0, opt.edit_xyz, w.v0, (uint32_t*)h->edit_win.ptr,
                       (uint8_t*)h->edit_dirty.ptr, nall, status, P.per_tree);
             nall = 0;
-            if (nbr)
-                VX_LAUNCH(h, KID_EDIT_BUILD, k_edit_build<T>, grid_for(nbr), 256, nbr, (const T*)opt.edit_values + w.e0,
-                          (uint32_t*)h->edit_win.ptr, (uint8_t*)h->edit_dirty.ptr,
-                          (uint16_t*)h->edit_masks.ptr + w.v0 / 8, (T*)h->edit_values.ptr + w.v0);
+            if (cells)
+                VX_LAUNCH(h, KID_EDIT_BUILD, k_edit_build<T>, grid_for((cells + cper - 1) / cper * 64), 256, cells, cper,
+                          (const T*)opt.edit_values + w.e0, (uint32_t*)h->edit_win.ptr,
+                          (uint8_t*)h->edit_dirty.ptr + w.v0 / 512, (uint16_t*)h->edit_masks.ptr + w.v0 / 8,
+                          (T*)h->edit_values.ptr + w.v0);
         }
     }
     // chunk set-up, plus the old-tree descent over the level-3 slots in extra blocks
@@ -790,9 +795,15 @@ int apply_edits_impl(vx_interner* h, size_t n, uint64_t* roots, const uint8_t* d
         most = std::max(most, w.v1 - w.v0);
     }
     int rc = ensure_zero(h, h->edit_win, most * 4);
-    if (!rc) rc = ensure_zero(h, h->edit_dirty, most / 512);
     if (rc) return rc;
-    if (!h->edit_masks.ensure(nvox / 4) || !h->edit_values.ensure(nvox * sizeof(T))) return VX_E_HIP;
+    if (nvox > h->edit_voxels) {  // the masks and the cells' states go together
+        h->edit_voxels = 0;
+        if (!h->edit_dirty.ensure(nvox / 512) || !h->edit_masks.ensure(nvox / 4)) return VX_E_HIP;
+        HIPCHK(hipMemsetAsync(h->edit_dirty.ptr, 0, h->edit_dirty.cap, h->stream));
+        HIPCHK(hipMemsetAsync(h->edit_masks.ptr, 0, h->edit_masks.cap, h->stream));
+        h->edit_voxels = nvox;
+    }
+    if (!h->edit_values.ensure(nvox * sizeof(T))) return VX_E_HIP;
     std::vector<vx_batch_view> views(trees.size());
     for (size_t i = 0; i < trees.size(); i++) {
         const uint64_t v0 = trees[i].vbase == ~0ull ? 0 : trees[i].vbase;
