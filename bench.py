@@ -135,7 +135,7 @@ def algorithmic_bytes(U):
     probe_miss = 2 + s + 8 + 8 * s  # generation, LOD value, owner entry, the children's values
     return {
         # per tree record and descent: the recorded height-2 nodes (64 B per level-3 slot)
-        # and the nodes above them; u16: the leaf id of every value (map + generation + id)
+        # and the nodes above them
         "k_prepare": U["level3_slots"] * 72 + U["trees"] * 48,
         # per brick slot: the mask pair (2), its share of the recorded height-2 node (1), the
         # result (8); a touched brick: its 8 values; a mixed brick: the old brick-level node
